@@ -279,10 +279,13 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(PlanParams P)
     // every range's start weight, computed once (a thread each: three 64-bit divisions) for the
     // searches below, when it fits in LDS
     const bool tab = R <= kStartsLds;
-    if (tab) {
+    // (every range starts out empty at the list's end: with more than half the ranges carrying
+    // items that outweigh their share, the last ones are carriers whose target is the whole
+    // weight, which no sequence's search below covers)
+    for (int w = tid; w < R; w += kPlanThreads) starts[w] = ns;
+    if (tab)
       for (int w = tid; w <= R; w += kPlanThreads) s_tgt[w] = T.tgt(w);
-      __syncthreads();
-    }
+    __syncthreads();
     auto tgt_at = [&](int w) -> int64_t { return tab ? s_tgt[w] : T.tgt(w); };
     for (int b = tid; b < B; b += kPlanThreads) {
       const int len = P.sl[b];

@@ -107,3 +107,19 @@ def test_cascade_hint_of_unshared_or_short_runs_changes_nothing():
     ref = kv_ref.decode(host["q"].float().numpy().astype(np.float64), host["cache"].float().numpy(),
                         host["indptr"], host["indices"], host["last"], PS)
     np.testing.assert_allclose(got, ref, atol=2e-3, rtol=1e-2)
+
+
+@pytest.mark.parametrize("hq,hkv,d,dtype,runs", [
+    (32, 8, 128, torch.bfloat16, [(96, 78, 78)]),  # 192 items on 256 ranges
+    (32, 8, 64, torch.float16, [(70, 20, 20), (33, 140, 140)]),
+])
+@torch.no_grad()
+def test_cascade_items_on_most_ranges(hq, hkv, d, dtype, runs):
+    """More than half of the ranges carry a prefix item and the items outweigh the suffixes: the
+    last ranges are carriers past the end of the suffix pages, which hold no page."""
+    dv, host = _batch(runs, hq, hkv, d, dtype, seed=hkv * 100 + d)
+    got, R, items = _decode(dv, hq, hkv, d, dtype, hint=True, cascade=True)
+    assert 2 * items > R
+    ref = kv_ref.decode(host["q"].float().numpy().astype(np.float64), host["cache"].float().numpy(),
+                        host["indptr"], host["indices"], host["last"], PS)
+    np.testing.assert_allclose(got, ref, atol=2e-3, rtol=1e-2)
