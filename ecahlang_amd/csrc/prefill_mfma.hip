@@ -1,5 +1,5 @@
 // Paged chunked prefill on the matrix cores (fp16 / bf16 caches, page_size 16, head_dim 64 or
-// 128, GQA group g in {1, 2, 4, 8, 16}).  Same contract as the vector kernel
+// 128, GQA groups g of 1 to 16).  Same contract as the vector kernel
 // (BatchPrefillWithPagedKVCacheWrapper.run, ecahlang/main.py:432-443, :68): query row i of
 // request b (qo_len_b rows) attends keys j <= i + kv_len_b - qo_len_b when causal (bottom-right
 // aligned), else all kv_len_b keys.
@@ -26,6 +26,15 @@
 // would wait behind the other waves' operand reads).
 // An item that is one chunk of a longer key range writes a partial (normalised rows plus
 // running max and sum); the merge kernel folds the partials of each split group.
+//
+// Groups that do not divide 256 (3, 5, 6, 7, 9 .. 15) take the same kernel with the group as a run
+// time value (G = 0): an item holds (256 / g) * g rows, and the few left over are masked like the
+// rows of a short tile.  These groups ran on the vector kernel before, which keeps the softmax
+// weights in fp32; here each weight is the sum of two 16-bit values, P = hi + lo, and P.V takes
+// both (half as many products again as the power-of-two groups), so that the result stays as
+// close to the 64-bit one as it was: the output's own rounding is what is left of the error.
+// Measured at 28 / 4 heads of 128 dims, bf16, 11 prompts of 20 to 1500 tokens (26 GFLOP of valid
+// pairs): 1418 us on the vector kernel, 63.4 us here (413 TFLOP/s), both 1.6e-3 off 64 bits.
 #include <type_traits>
 #include "attn_common.h"
 #include "mfma_common.h"
@@ -47,6 +56,20 @@ constexpr float kLazyMax = 8.f;
 // Source of the value rows that must read as zero (past the chunk, absent pages): P is 0 there,
 // and 0 * NaN would poison P.V.
 __device__ uint4 g_zero_rows[64];
+
+// The two values of a packed pair (Mma<T>::pack) as floats.
+template <typename T>
+__device__ __forceinline__ void unpack2(uint32_t u, float& x, float& y) {
+  if constexpr (std::is_same<T, _Float16>::value) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    const h2 h = bitcast_<h2>(u);
+    x = (float)h[0];
+    y = (float)h[1];
+  } else {
+    x = __uint_as_float(u << 16);
+    y = __uint_as_float(u & 0xFFFF0000u);
+  }
+}
 
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
@@ -89,18 +112,25 @@ struct PrefillMfmaParams {
   void* out;
   int64_t o_sn, o_sh;
   const int32_t* items;
-  float2* part_ml;  // [slot][kRows]
-  float* part_o;    // [slot][kRows][D] (fp16 elements for fp16 caches, else fp32)
+  float2* part_ml;  // [slot][rows of an item]
+  float* part_o;    // [slot][rows of an item][D] (kHalfPartials: fp16 elements, else fp32)
   int32_t o_vec;
 };
 
 // Split groups' partial outputs are kept in fp16 when the cache is fp16 (averages of fp16 V
 // rows, so they fit; half the bytes written by the items and read by the merge), else fp32.
-template <typename T>
-constexpr bool kHalfPartials = std::is_same<T, _Float16>::value;
+// (the run-time groups, G = 0, keep fp32 partials, as they keep fp32-exact weights).
+template <typename T, int G>
+constexpr bool kHalfPartials = std::is_same<T, _Float16>::value && G != 0;
+
+// Query rows per item: 256, or the largest multiple of the group below it.
+template <int G>
+__device__ __forceinline__ int item_rows(int g) { return G ? kRows : kRows / g * g; }
 
 template <typename T, int D, int G>
 __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillMfmaParams P) {
+  constexpr bool SPLIT = G == 0;      // softmax weights as a sum of two 16-bit values
+  const int g = G ? G : P.hq / P.hkv;
   constexpr int KSTEPS = D / 32;      // Q.K^T reduction steps
   constexpr int MT = D / 16;          // output tiles of 16 dims
   constexpr int CPR = D / 8;          // 16-byte chunks per row
@@ -112,7 +142,6 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillMfmaParams P) 
   constexpr int LPP = 16 / RPI;       // loads per page and K or V
   constexpr int KL = NP * LPP / 8;    // K (and V) loads per wave per step
   static_assert(NP * LPP % 8 == 0, "loads per wave");
-  constexpr int TQ = kRows / G;       // query tokens per item
 
   // rings of three stages for K and for V
   __shared__ __align__(16) char s_k[3 * STEPB];
@@ -138,11 +167,11 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillMfmaParams P) 
 #pragma unroll
   for (int rt = 0; rt < 2; ++rt) {
     const int r = 32 * wave + 16 * rt + lr;
-    const int tt = r / G, hh = r % G;
+    const int tt = r / g, hh = r % g;
     rtok[rt] = tt;
     const bool ok = tt < tq;
     const T* src = reinterpret_cast<const T*>(P.q) + (int64_t)(qo_start + t0 + (ok ? tt : 0)) * P.q_sn +
-                   (int64_t)(h * G + hh) * P.q_sh + 8 * lg;
+                   (int64_t)(h * g + hh) * P.q_sh + 8 * lg;
 #pragma unroll
     for (int s = 0; s < KSTEPS; ++s) {
       const uint4 v = *reinterpret_cast<const uint4*>(src + 32 * s);
@@ -157,9 +186,8 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillMfmaParams P) 
   const int npc = nsteps * NP;
   for (int i = threadIdx.x; i < npc; i += blockDim.x) {
     const int64_t pi = k0 / 16 + i;
-    int64_t e = kp0 + (pi < npages_req ? pi : npages_req - 1);
-    e = e < P.num_indices ? e : P.num_indices - 1;
-    const int64_t pg = e >= 0 ? P.indices[e] : -1;
+    const int64_t e = kp0 + (pi < npages_req ? pi : npages_req - 1);
+    const int64_t pg = (uint64_t)e < (uint64_t)P.num_indices ? P.indices[e] : -1;
     s_page[i] = (pg >= 0 && pg < P.num_pages) ? (int)pg : -1;
   }
   // V stage 2 starts zero-filled: the first M phase multiplies it by a zero P (uninitialised LDS
@@ -262,10 +290,14 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillMfmaParams P) 
   // 2j + 3 (the leading waves' S(j + 1), the trailing waves' M(j + 1)).
   f4 sacc[NP][2];    // S^T tiles of the step in flight: [key tile kt][row tile rt]
   uint2 pb[NP][2];   // P of the previous step, packed as the B operand of P.V (zero before step 0)
+  uint2 pl[SPLIT ? NP : 1][2];  // SPLIT: P less the values in pb
 #pragma unroll
   for (int kt = 0; kt < NP; ++kt)
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt) pb[kt][rt] = make_uint2(0, 0);
+    for (int rt = 0; rt < 2; ++rt) {
+      pb[kt][rt] = make_uint2(0, 0);
+      if constexpr (SPLIT) pl[kt][rt] = make_uint2(0, 0);
+    }
   const int tr_row = 4 * lg + (lr >> 2);
   // M(j): the page loads of later steps, then the products as a software pipeline of units of
   // eight 16x16x32 products: units 0-3 are P.V of step j - 1 (pages 2u, 2u + 1 with u = unit / 2,
@@ -310,6 +342,16 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillMfmaParams P) 
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt)
           o[rt][MTU * (i & 1) + m] = Mma<T>::qk(opnd[buf][m], pp[rt], o[rt][MTU * (i & 1) + m]);
+      if constexpr (SPLIT) {
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt)
+          pp[rt] = make_uint4(pl[2 * u][rt].x, pl[2 * u][rt].y, pl[2 * u + 1][rt].x, pl[2 * u + 1][rt].y);
+#pragma unroll
+        for (int m = 0; m < MTU; ++m)
+#pragma unroll
+          for (int rt = 0; rt < 2; ++rt)
+            o[rt][MTU * (i & 1) + m] = Mma<T>::qk(opnd[buf][m], pp[rt], o[rt][MTU * (i & 1) + m]);
+      }
     } else {
       const int kt = i - 4;
 #pragma unroll
@@ -421,6 +463,12 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillMfmaParams P) 
           psum[i] = kt == 0 ? pr[i] : psum[i] + pr[i];
         }
         pb[kt][rt] = make_uint2(Mma<T>::pack(pr[0], pr[1]), Mma<T>::pack(pr[2], pr[3]));
+        if constexpr (SPLIT) {
+          float hi[4];
+          unpack2<T>(pb[kt][rt].x, hi[0], hi[1]);
+          unpack2<T>(pb[kt][rt].y, hi[2], hi[3]);
+          pl[kt][rt] = make_uint2(Mma<T>::pack(pr[0] - hi[0], pr[1] - hi[1]), Mma<T>::pack(pr[2] - hi[2], pr[3] - hi[3]));
+        }
       }
       lsum[rt] += (psum[0] + psum[1]) + (psum[2] + psum[3]);
     }
@@ -475,11 +523,11 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillMfmaParams P) 
     float ltot = lsum[rt] + __shfl_xor(lsum[rt], 16, 64);
     ltot += __shfl_xor(ltot, 32, 64);
     const int r = 32 * wave + 16 * rt + lr;
-    const int tt = rtok[rt], hh = r % G;
+    const int tt = rtok[rt], hh = r % g;
     if (tt >= tq) continue;
     const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
     if (slot < 0) {
-      T* orow = reinterpret_cast<T*>(P.out) + (int64_t)(qo_start + t0 + tt) * P.o_sn + (int64_t)(h * G + hh) * P.o_sh + 4 * lg;
+      T* orow = reinterpret_cast<T*>(P.out) + (int64_t)(qo_start + t0 + tt) * P.o_sn + (int64_t)(h * g + hh) * P.o_sh + 4 * lg;
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
         if (P.o_vec) {
@@ -491,8 +539,8 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillMfmaParams P) 
         }
       }
     } else {
-      const int64_t pr = (int64_t)slot * kRows + r;
-      if constexpr (kHalfPartials<T>) {
+      const int64_t pr = (int64_t)slot * item_rows<G>(g) + r;
+      if constexpr (kHalfPartials<T, G>) {
         _Float16* prow = reinterpret_cast<_Float16*>(P.part_o) + pr * D + 4 * lg;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
@@ -526,10 +574,11 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillMfmaParams P,
   const int32_t* gr = groups + (int64_t)kGroup * (blockIdx.x / (kRows / RB));
   const int s0 = gr[0], ns = gr[1], qo_start = gr[2], t0 = gr[3], tq = gr[4], h = gr[5];
   const int r = (blockIdx.x % (kRows / RB)) * RB + threadIdx.x / TPR, d = (threadIdx.x % TPR) * 8;
-  const int tt = r / G, hh = r % G;
+  const int g = G ? G : P.hq / P.hkv, rows = item_rows<G>(g);
+  const int tt = r / g, hh = r % g;
   if (tt >= tq || ns <= 0) return;
-  const float2* ml = P.part_ml + (int64_t)s0 * kRows + r;
-  const int64_t po = ((int64_t)s0 * kRows + r) * D + d;  // element offset of slot s0's dims
+  const float2* ml = P.part_ml + (int64_t)s0 * rows + r;
+  const int64_t po = ((int64_t)s0 * rows + r) * D + d;  // element offset of slot s0's dims
   float M = -INFINITY;
   float den = 0.f;
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -539,15 +588,15 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillMfmaParams P,
 #pragma unroll
     for (int u = 0; u < kMergeUnroll; ++u) {
       const int64_t sl = min(s + u, ns - 1);
-      w[u] = ml[sl * kRows];
-      if constexpr (kHalfPartials<T>) {
-        const uint4 raw = *reinterpret_cast<const uint4*>(reinterpret_cast<const _Float16*>(P.part_o) + po + sl * kRows * D);
+      w[u] = ml[sl * rows];
+      if constexpr (kHalfPartials<T, G>) {
+        const uint4 raw = *reinterpret_cast<const uint4*>(reinterpret_cast<const _Float16*>(P.part_o) + po + sl * rows * D);
         _Float16 hv[8];
         __builtin_memcpy(hv, &raw, 16);
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[u][e] = (float)hv[e];
       } else {
-        const float4* src = reinterpret_cast<const float4*>(P.part_o + po + sl * kRows * D);
+        const float4* src = reinterpret_cast<const float4*>(P.part_o + po + sl * rows * D);
         const float4 a = src[0], b = src[1];
         v[u][0] = a.x; v[u][1] = a.y; v[u][2] = a.z; v[u][3] = a.w;
         v[u][4] = b.x; v[u][5] = b.y; v[u][6] = b.z; v[u][7] = b.w;
@@ -578,7 +627,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillMfmaParams P,
     }
   }
   const float inv = den > 0.f ? 1.f / den : 0.f;
-  T* orow = reinterpret_cast<T*>(P.out) + (int64_t)(qo_start + t0 + tt) * P.o_sn + (int64_t)(h * G + hh) * P.o_sh + d;
+  T* orow = reinterpret_cast<T*>(P.out) + (int64_t)(qo_start + t0 + tt) * P.o_sn + (int64_t)(h * g + hh) * P.o_sh + d;
   if (P.o_vec) {
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
@@ -611,7 +660,7 @@ int launch_g(const PrefillMfmaParams& P, int g, int n_items, const int32_t* grou
     case 8: return launch<T, D, 8>(P, n_items, groups, n_groups, s);
     case 16: return launch<T, D, 16>(P, n_items, groups, n_groups, s);
   }
-  return kBadGroup;
+  return g >= 1 && g < 16 ? launch<T, D, 0>(P, n_items, groups, n_groups, s) : (int)kBadGroup;
 }
 
 }  // namespace
@@ -621,7 +670,7 @@ extern "C" int pkv_prefill_mfma_supported(int32_t dtype, int32_t head_dim, int32
   if (num_kv_heads <= 0 || num_qo_heads % num_kv_heads) return 0;
   const int g = num_qo_heads / num_kv_heads;
   return (dtype == kF16 || dtype == kBF16) && (head_dim == 64 || head_dim == 128) && page_size == 16 &&
-         (g == 1 || g == 2 || g == 4 || g == 8 || g == 16);
+         g >= 1 && g <= 16;
 }
 
 extern "C" int pkv_batch_prefill_mfma(const void* q, int64_t q_stride_n, int64_t q_stride_h,

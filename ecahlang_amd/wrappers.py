@@ -343,12 +343,25 @@ class BatchPrefillWithPagedKVCacheWrapper:
         self._sm_scale = float(sm_scale) if sm_scale is not None else 1.0 / math.sqrt(self._d)
         self._mfma = bool(lib().pkv_prefill_mfma_supported(dtype_code(self._q_dtype), self._d, self._hq,
                                                           self._hkv, self._ps))
+        g = self._hq // self._hkv
+        # Shapes that can also run without a work list, on the vector kernel, which reads the table
+        # at run time, needs no workspace and can be planned and captured: they do where the work
+        # list cannot be built or kept (plan() while capturing, a workspace too small for it) and
+        # in run() for a captured call or a q of another length than the plan's.
+        self._valu_ok = g not in (1, 2, 4, 8, 16)
+        if self._mfma and self._valu_ok:
+            self._mfma = self._batch > 0 and self._workspace_usable(qo_indptr.device) and \
+                not torch.cuda.is_current_stream_capturing()
         if self._mfma:
             self._schedule(qo_indptr.device)
         self._planned = True
 
     # rows per matrix-core work item (8 waves x 32 rows): 256 / g query tokens of one KV head
     _ROWS = 256
+
+    def _workspace_usable(self, dev: torch.device) -> bool:
+        ws = self._workspace
+        return isinstance(ws, torch.Tensor) and ws.device == dev and ws.is_contiguous() and ws.data_ptr() % 256 == 0
 
     def _schedule(self, dev: torch.device) -> None:
         """The matrix-core kernel's work list (``prefill_work_list``) copied into the
@@ -359,10 +372,17 @@ class BatchPrefillWithPagedKVCacheWrapper:
         last = self._last.cpu().tolist()
         self._nnz_q = qo[-1]
         ws_bytes = self._workspace.numel() * self._workspace.element_size()
-        # (the kernel keeps an fp16 cache's split partials in fp16)
-        wl = prefill_work_list(qo, kp, last, self._hq // self._hkv, self._hkv, self._ps, self._causal, self._d,
-                               _num_cus(dev), ws_bytes, self._ROWS,
-                               partial_bytes=2 if self._q_dtype == torch.float16 else 4)
+        g = self._hq // self._hkv
+        # (the kernel keeps the split partials of an fp16 cache's power-of-two groups in fp16)
+        half = self._q_dtype == torch.float16 and not self._valu_ok
+        try:
+            wl = prefill_work_list(qo, kp, last, g, self._hkv, self._ps, self._causal, self._d, _num_cus(dev),
+                                   ws_bytes, self._ROWS // g * g, partial_bytes=2 if half else 4)
+        except RuntimeError:
+            if not self._valu_ok:
+                raise
+            self._mfma = False
+            return
         items, merges = wl["items_np"], wl["groups_np"]
         off_g, off_ml, off_o = wl["off_groups"], wl["off_ml"], wl["off_o"]
         if len(items):
@@ -398,7 +418,11 @@ class BatchPrefillWithPagedKVCacheWrapper:
             raise ValueError("out must match q's shape and dtype")
         aligned = q.data_ptr() % 16 == 0 and (q.stride(0) * q.element_size()) % 16 == 0 and \
             (q.stride(1) * q.element_size()) % 16 == 0
-        if self._mfma and aligned and not force_valu:
+        mfma = self._mfma and aligned and not force_valu
+        if mfma and self._valu_ok:
+            mfma = nnz == self._nnz_q and (cv.k_ptr | cv.v_ptr) % 16 == 0 and \
+                not torch.cuda.is_current_stream_capturing()
+        if mfma:
             if nnz < self._nnz_q:
                 raise ValueError(f"q has {nnz} rows, qo_indptr needs {self._nnz_q}")
             check(lib().pkv_batch_prefill_mfma(

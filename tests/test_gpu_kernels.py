@@ -507,3 +507,47 @@ def test_read_probe_reads_in_bounds_and_checks_arguments():
     assert lib().pkv_probe_stream_read(x.data_ptr() + 4, 32, 4, sink.data_ptr(), s) < 0  # misaligned
     assert lib().pkv_probe_stream_read(x.data_ptr(), 64, 0, sink.data_ptr(), s) < 0      # no workgroups
     assert lib().pkv_probe_stream_read(x.data_ptr(), 64, 4, 0, s) < 0                    # no sink
+
+
+# Groups that do not divide an item's 256 query rows: tile edges (a request of exactly one item's
+# tokens, one more, one less), one token, an empty request, split key ranges.
+ODD_GROUPS = {
+    "g7_bf16_d128": lambda: workloads.build_batch([36, 37, 35, 1, 73, 900, 50], [36, 37, 35, 1, 73, 40, 0], 14, 2, 128,
+                                                  torch.bfloat16, 61),
+    "g3_fp16_d64": lambda: workloads.build_batch([85, 86, 700, 17], [85, 86, 300, 3], 24, 8, 64, torch.float16, 62),
+    "g5_fp16_d128": lambda: workloads.build_batch([51, 52, 3000], [51, 52, 10], 10, 2, 128, torch.float16, 63),
+    "g6_bf16_d64": lambda: workloads.build_batch([42, 43, 16, 130], [42, 43, 16, 130], 12, 2, 64, torch.bfloat16, 64),
+    "g15_fp16_d128": lambda: workloads.build_batch([17, 18, 300], [17, 18, 33], 15, 1, 128, torch.float16, 65),
+}
+
+
+@pytest.mark.parametrize("name", list(ODD_GROUPS))
+@pytest.mark.parametrize("causal", [True, False])
+def test_prefill_odd_groups_on_the_matrix_cores(name, causal):
+    """Against the float64 oracle, and no further from it than the vector kernel, whose softmax
+    weights are fp32 (both are left with the output's rounding; 5 % for the order of the sums).
+    A captured run and a workspace too small for the work list take the vector kernel."""
+    wb = ODD_GROUPS[name]()
+    dv = wb.to(DEV)
+    _append_dev(dv)
+    _, vals = _oracle_appended(wb)
+    ref = kv_ref.prefill(wb.q.float().numpy(), wb.append_indptr.numpy(), vals, wb.indptr.numpy(),
+                         wb.indices.numpy(), wb.last.numpy(), wb.ps, causal=causal)
+    args = (dv.append_indptr, dv.indptr, dv.indices, dv.last, dv.hq, dv.hkv, dv.d, dv.ps)
+    w = BatchPrefillWithPagedKVCacheWrapper(torch.empty(64 << 20, dtype=torch.uint8, device=DEV), "NHD")
+    w.plan(*args, causal=causal, q_data_type=dv.dtype)
+    assert w._mfma
+    o, ov = w.run(dv.q, dv.cache), w.run(dv.q, dv.cache, force_valu=True)
+    torch.cuda.synchronize()
+    got = o.double().cpu().numpy()
+    np.testing.assert_allclose(got, ref, **TOL[wb.dtype])
+    err, err_v = (np.linalg.norm(x - ref) for x in (got, ov.double().cpu().numpy()))
+    assert err <= 1.05 * err_v, (err, err_v)
+    small = BatchPrefillWithPagedKVCacheWrapper(torch.empty(16, dtype=torch.uint8, device=DEV), "NHD")
+    small.plan(*args, causal=causal, q_data_type=dv.dtype)
+    out, graph, side = torch.zeros_like(dv.q), torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
+        w.run(dv.q, dv.cache, out=out)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(small.run(dv.q, dv.cache), ov) and torch.equal(out, ov)
