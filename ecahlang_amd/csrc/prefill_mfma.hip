@@ -38,24 +38,17 @@
 #include <type_traits>
 #include "attn_common.h"
 #include "mfma_common.h"
+#include "prefill_common.h"
 #include "../../include/pagedkv.h"
 
 using namespace pkv;
 using namespace pkv::mfma;
+using namespace pkv::pre;
 
 namespace {
 
 constexpr int kRows = 256;   // query rows per item (8 waves x 32)
 constexpr int kStepPages = 4;  // pages (16 keys each) staged per step; chunks start at multiples of 64 keys
-constexpr int kMaxChunk = 8192;  // keys per item (its page ids are staged in LDS)
-// Lazy running max (log2 units): a row's reference max moves only when its scores exceed it by
-// more than this, so probabilities stay <= 2^kLazyMax (exact enough in fp16 / bf16 P, and far
-// from fp32 overflow in the sums) and the output rows are rescaled only on such jumps.
-constexpr float kLazyMax = 8.f;
-
-// Source of the value rows that must read as zero (past the chunk, absent pages): P is 0 there,
-// and 0 * NaN would poison P.V.
-__device__ uint4 g_zero_rows[64];
 
 // The two values of a packed pair (Mma<T>::pack) as floats.
 template <typename T>
@@ -71,10 +64,6 @@ __device__ __forceinline__ void unpack2(uint32_t u, float& x, float& y) {
   }
 }
 
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 // A workgroup barrier that also ends the compiler's scheduling region, so that no instruction
 // moves between the phases it separates.
 __device__ __forceinline__ void phase_barrier() {
@@ -82,50 +71,6 @@ __device__ __forceinline__ void phase_barrier() {
   lds_barrier();
   __builtin_amdgcn_sched_barrier(0);
 }
-// One wave-wide 16-byte-per-lane copy global -> LDS: lane l's 16 bytes at sbase + voff (a
-// wave-uniform base in an SGPR pair plus a 32-bit per-lane byte offset) land at LDS byte
-// m0 + 16 * l (m0 uniform).  Written as inline assembly so that the compiler does not track it:
-// the caller orders it with explicit vmcnt waits and barriers (the compiler cannot tell which LDS
-// array a later transposed read touches and would otherwise wait for every copy in flight,
-// draining the prefetch pipeline).
-__device__ __forceinline__ void lds_copy16(const void* sbase, unsigned voff, unsigned m0) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(m0) : "memory", "m0");
-}
-// LDS byte address of a pointer into a __shared__ array.
-__device__ __forceinline__ unsigned lds_addr(const char* p) {
-  return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) char*)(p);
-}
-constexpr int kItem = 12;    // int32 fields per work item
-constexpr int kGroup = 8;    // int32 fields per split group
-
-struct PrefillMfmaParams {
-  const void* q;
-  int64_t q_sn, q_sh;
-  const void* k_cache;
-  const void* v_cache;
-  int64_t page_stride, num_pages;
-  const int32_t* indices;
-  int64_t num_indices;
-  int32_t hq, hkv;
-  int32_t causal;
-  float scale_log2;
-  void* out;
-  int64_t o_sn, o_sh;
-  const int32_t* items;
-  float2* part_ml;  // [slot][rows of an item]
-  float* part_o;    // [slot][rows of an item][D] (kHalfPartials: fp16 elements, else fp32)
-  int32_t o_vec;
-};
-
-// Split groups' partial outputs are kept in fp16 when the cache is fp16 (averages of fp16 V
-// rows, so they fit; half the bytes written by the items and read by the merge), else fp32.
-// (the run-time groups, G = 0, keep fp32 partials, as they keep fp32-exact weights).
-template <typename T, int G>
-constexpr bool kHalfPartials = std::is_same<T, _Float16>::value && G != 0;
-
-// Query rows per item: 256, or the largest multiple of the group below it.
-template <int G>
-__device__ __forceinline__ int item_rows(int g) { return G ? kRows : kRows / g * g; }
 
 template <typename T, int D, int G>
 __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillMfmaParams P) {
@@ -446,7 +391,8 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillMfmaParams P) 
       const bool grow = cms > m[rt] + kLazyMax;  // (false while every score so far is masked)
       if (__ballot(grow)) {
         const float mnew = grow ? cms : m[rt];
-        const float alpha = __builtin_amdgcn_exp2f(m[rt] - mnew);  // 0 from -inf, 1 if unchanged
+        // 0 from -inf; 1 if unchanged (also where no key has been seen: -inf less -inf is NaN)
+        const float alpha = grow ? __builtin_amdgcn_exp2f(m[rt] - mnew) : 1.f;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) o[rt][mt] *= alpha;
         lsum[rt] *= alpha;
@@ -518,8 +464,18 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillMfmaParams P) 
   }
 
   // ---- rows out: normalised output rows, or the partial of a split group
+  uint32_t redo[2] = {0, 0};  // SPLIT: rows of each row tile that did not come out finite
 #pragma unroll
   for (int rt = 0; rt < 2; ++rt) {
+    if constexpr (SPLIT) {
+      float z = 0.f;  // (0, or NaN from an infinity or a NaN)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) z = __builtin_fmaf(o[rt][mt][i], 0.f, z);
+      const uint64_t bad = __ballot(z != 0.f && rtok[rt] < tq);
+      redo[rt] = (uint32_t)((bad | bad >> 16 | bad >> 32 | bad >> 48) & 0xFFFF);
+    }
     float ltot = lsum[rt] + __shfl_xor(lsum[rt], 16, 64);
     ltot += __shfl_xor(ltot, 32, 64);
     const int r = 32 * wave + 16 * rt + lr;
@@ -539,7 +495,7 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillMfmaParams P) 
         }
       }
     } else {
-      const int64_t pr = (int64_t)slot * item_rows<G>(g) + r;
+      const int64_t pr = (int64_t)slot * item_rows<G, kRows>(g) + r;
       if constexpr (kHalfPartials<T, G>) {
         _Float16* prow = reinterpret_cast<_Float16*>(P.part_o) + pr * D + 4 * lg;
 #pragma unroll
@@ -556,88 +512,26 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillMfmaParams P) 
       if (lg == 0) P.part_ml[pr] = make_float2(m[rt], ltot);
     }
   }
-}
-
-// Folds the partials of each split group: group = {first_slot, nslots, qo_start, t0, tq, h}.
-// A workgroup takes merge_rows() rows of one group; D/8 lanes per row, 8 dims each (16-byte
-// loads of fp16 partials).  Each round loads kMergeUnroll slots' (max, sum) and rows together,
-// from clamped (always valid) addresses, and folds them under a running max: one memory round
-// trip per round, and for a group of at most kMergeUnroll slots the plain fold under the
-// group's max.
-constexpr int kMergeUnroll = 4;
-template <int D>
-constexpr int merge_rows() { return 256 / (D / 8); }
-
-template <typename T, int D, int G>
-__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillMfmaParams P, const int32_t* groups) {
-  constexpr int RB = merge_rows<D>(), TPR = D / 8;
-  const int32_t* gr = groups + (int64_t)kGroup * (blockIdx.x / (kRows / RB));
-  const int s0 = gr[0], ns = gr[1], qo_start = gr[2], t0 = gr[3], tq = gr[4], h = gr[5];
-  const int r = (blockIdx.x % (kRows / RB)) * RB + threadIdx.x / TPR, d = (threadIdx.x % TPR) * 8;
-  const int g = G ? G : P.hq / P.hkv, rows = item_rows<G>(g);
-  const int tt = r / g, hh = r % g;
-  if (tt >= tq || ns <= 0) return;
-  const float2* ml = P.part_ml + (int64_t)s0 * rows + r;
-  const int64_t po = ((int64_t)s0 * rows + r) * D + d;  // element offset of slot s0's dims
-  float M = -INFINITY;
-  float den = 0.f;
-  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < ns; s += kMergeUnroll) {
-    float2 w[kMergeUnroll];
-    float v[kMergeUnroll][8];
-#pragma unroll
-    for (int u = 0; u < kMergeUnroll; ++u) {
-      const int64_t sl = min(s + u, ns - 1);
-      w[u] = ml[sl * rows];
-      if constexpr (kHalfPartials<T, G>) {
-        const uint4 raw = *reinterpret_cast<const uint4*>(reinterpret_cast<const _Float16*>(P.part_o) + po + sl * rows * D);
-        _Float16 hv[8];
-        __builtin_memcpy(hv, &raw, 16);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[u][e] = (float)hv[e];
-      } else {
-        const float4* src = reinterpret_cast<const float4*>(P.part_o + po + sl * rows * D);
-        const float4 a = src[0], b = src[1];
-        v[u][0] = a.x; v[u][1] = a.y; v[u][2] = a.z; v[u][3] = a.w;
-        v[u][4] = b.x; v[u][5] = b.y; v[u][6] = b.z; v[u][7] = b.w;
+  if constexpr (SPLIT) {
+    if (redo[0] | redo[1]) {  // (wave-uniform)
+      wait_stores();  // the rows below are written again, by other lanes
+#pragma unroll 1
+      for (uint32_t todo = redo[0] | redo[1] << 16; todo; todo &= todo - 1) {
+        const int r = 32 * wave + __builtin_ctz(todo), tt = r / g, hh = r % g;
+        const int64_t row = qo_start + t0 + tt;
+        const T* q = reinterpret_cast<const T*>(P.q) + row * P.q_sn + (int64_t)(h * g + hh) * P.q_sh;
+        const int l = P.causal ? t0 + tt + kv_len - qo_len + 1 : kv_len;
+        exact_row<T, D>(P, s_page, k0, min(l, k1), hoff, q, [&](int d, float x, float mx, float sum) {
+          if (slot < 0) {
+            reinterpret_cast<T*>(P.out)[row * P.o_sn + (int64_t)(h * g + hh) * P.o_sh + d] = from_f32<T>(x);
+          } else {
+            const int64_t pr = (int64_t)slot * item_rows<G, kRows>(g) + r;
+            P.part_o[pr * D + d] = x;
+            if (d == 0) P.part_ml[pr] = make_float2(mx, sum);
+          }
+        });
       }
     }
-    // the running max over the slots loaded so far (repeats of the last slot included, as in a
-    // separate max pass); what earlier rounds folded is rescaled to it
-    float Mn = M;
-#pragma unroll
-    for (int u = 0; u < kMergeUnroll; ++u) Mn = fmaxf(Mn, w[u].x);
-    if (Mn > M) {
-      const float f = den > 0.f ? exp2f(M - Mn) : 0.f;
-      den *= f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] *= f;
-      M = Mn;
-    }
-#pragma unroll
-    for (int u = 0; u < kMergeUnroll; ++u) {
-      // a slot whose rows saw no key (l = 0) carries no weight; repeats past ns count zero
-      // (such a slot's row may hold anything, hence the branch rather than a zero weight)
-      const float c = (s + u < ns && w[u].y > 0.f) ? exp2f(w[u].x - M) * w[u].y : 0.f;
-      if (c != 0.f) {
-        den += c;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e] += c * v[u][e];
-      }
-    }
-  }
-  const float inv = den > 0.f ? 1.f / den : 0.f;
-  T* orow = reinterpret_cast<T*>(P.out) + (int64_t)(qo_start + t0 + tt) * P.o_sn + (int64_t)(h * g + hh) * P.o_sh + d;
-  if (P.o_vec) {
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      T o4[4] = {from_f32<T>(acc[4 * half] * inv), from_f32<T>(acc[4 * half + 1] * inv),
-                 from_f32<T>(acc[4 * half + 2] * inv), from_f32<T>(acc[4 * half + 3] * inv)};
-      *reinterpret_cast<uint2*>(orow + 4 * half) = *reinterpret_cast<const uint2*>(o4);
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) orow[e] = from_f32<T>(acc[e] * inv);
   }
 }
 
@@ -646,7 +540,7 @@ int launch(const PrefillMfmaParams& P, int n_items, const int32_t* groups, int n
   if (n_items > 0)
     hipLaunchKernelGGL((prefill_mfma_kernel<T, D, G>), dim3(n_items), dim3(512), 0, s, P);
   if (n_groups > 0)
-    hipLaunchKernelGGL((prefill_merge_kernel<T, D, G>), dim3(n_groups * (kRows / merge_rows<D>())), dim3(256), 0, s,
+    hipLaunchKernelGGL((prefill_merge_kernel<T, D, G, kRows>), dim3(n_groups * (kRows / merge_rows<D>())), dim3(256), 0, s,
                        P, groups);
   return (int)hipGetLastError();
 }
@@ -665,11 +559,16 @@ int launch_g(const PrefillMfmaParams& P, int g, int n_items, const int32_t* grou
 
 }  // namespace
 
+namespace pkv {
+int prefill_f32_launch(const pre::PrefillMfmaParams& P, int d, int n_items, const int32_t* groups, int n_groups,
+                       hipStream_t s);
+}
+
 extern "C" int pkv_prefill_mfma_supported(int32_t dtype, int32_t head_dim, int32_t num_qo_heads,
                                           int32_t num_kv_heads, int32_t page_size) {
   if (num_kv_heads <= 0 || num_qo_heads % num_kv_heads) return 0;
   const int g = num_qo_heads / num_kv_heads;
-  return (dtype == kF16 || dtype == kBF16) && (head_dim == 64 || head_dim == 128) && page_size == 16 &&
+  return (dtype == kF16 || dtype == kBF16 || dtype == kF32) && (head_dim == 64 || head_dim == 128) && page_size == 16 &&
          g >= 1 && g <= 16;
 }
 
@@ -684,7 +583,7 @@ extern "C" int pkv_batch_prefill_mfma(const void* q, int64_t q_stride_n, int64_t
   if (!pkv_prefill_mfma_supported(dtype, head_dim, num_qo_heads, num_kv_heads, page_size)) return kBadArg;
   if (n_items < 0 || n_groups < 0 || (n_items > 0 && !items) || (n_groups > 0 && (!groups || !part_ml || !part_o)))
     return kBadArg;
-  const int es = 2;
+  const int es = dtype == kF32 ? 4 : 2;
   if ((uintptr_t)q % 16 || (q_stride_n * es) % 16 || (q_stride_h * es) % 16) return kBadAlign;
   PrefillMfmaParams P;
   P.q = q; P.q_sn = q_stride_n; P.q_sh = q_stride_h;
@@ -696,9 +595,11 @@ extern "C" int pkv_batch_prefill_mfma(const void* q, int64_t q_stride_n, int64_t
   P.items = items;
   P.part_ml = reinterpret_cast<float2*>(part_ml);
   P.part_o = reinterpret_cast<float*>(part_o);
-  P.o_vec = ((uintptr_t)out % 8 == 0) && ((o_stride_n * es) % 8 == 0) && ((o_stride_h * es) % 8 == 0);
+  // four elements at a time
+  P.o_vec = ((uintptr_t)out % (4 * es) == 0) && o_stride_n % 4 == 0 && o_stride_h % 4 == 0;
   hipStream_t s = (hipStream_t)stream;
   const int g = num_qo_heads / num_kv_heads;
+  if (dtype == kF32) return prefill_f32_launch(P, head_dim, n_items, groups, n_groups, s);
   if (dtype == kF16)
     return head_dim == 64 ? launch_g<_Float16, 64>(P, g, n_items, groups, n_groups, s)
                           : launch_g<_Float16, 128>(P, g, n_items, groups, n_groups, s);

@@ -25,8 +25,10 @@ constexpr int kItemWords = 12;
 constexpr int kGroupWords = 8;
 constexpr int kStepKeys = 64;
 constexpr int kChunkMin = 256, kChunkMax = 8192;
-// Makespan model, in microseconds.
-constexpr double kStepUs = 1.9, kItemUs = 11.0, kSplitUs = 6.0;
+// Makespan model, in microseconds.  Items of at most 128 rows are the fp32 kernel's, whose step is
+// its products' issue time on the compute unit (128 x 64 keys x head_dim / 64 at 0.61 TFLOP/s).
+constexpr double kStepUs = 1.9, kItemUs = 11.0, kSplitUs = 6.0, kStepF32Us = 3.4;
+constexpr int kRowsF32 = 128;
 // Candidate chunks, as multiples of total keys / CUs (in 1/16).
 constexpr int kCandidates[] = {8, 10, 12, 14, 16, 17, 18, 20, 24};
 
@@ -59,7 +61,7 @@ Layout layout_for(const std::vector<Group>& groups, int chunk, int rows, int hea
 
 // Simulated kernel time of the work list cut at `chunk`: items longest first, each to the
 // least loaded of ncu compute units.
-double makespan(const std::vector<Group>& groups, int chunk, int ncu) {
+double makespan(const std::vector<Group>& groups, int chunk, int ncu, double step_us) {
   struct It {
     int len;
     bool split;
@@ -75,7 +77,7 @@ double makespan(const std::vector<Group>& groups, int chunk, int ncu) {
   double worst = 0.0;
   for (const It& it : its) {
     const double t = load.top() + kItemUs + (it.split ? kSplitUs : 0.0) +
-                     kStepUs * ((it.len + kStepKeys - 1) / kStepKeys);
+                     step_us * ((it.len + kStepKeys - 1) / kStepKeys);
     load.pop();
     load.push(t);
     worst = std::max(worst, t);
@@ -123,6 +125,7 @@ extern "C" int pkv_prefill_work_list(const int32_t* qo_indptr, const int32_t* kv
   // whose partials fit (ties go to the longer chunk: fewer splits); if none fits, doubled from
   // the longest candidate while the partials do not fit
   const int64_t per_cu = (total + num_cus - 1) / num_cus;
+  const double step_us = rows > kRowsF32 ? kStepUs : kStepF32Us * head_dim / 64;
   int best = 0;
   if (chunk != 0) {
     best = chunk;
@@ -133,7 +136,7 @@ extern "C" int pkv_prefill_work_list(const int32_t* qo_indptr, const int32_t* kv
       const int c = round_chunk(per_cu * f / 16);
       widest = std::max(widest, c);
       if (layout_for(grs, c, rows, head_dim, partial_bytes).bytes > workspace_bytes) continue;
-      const double t = makespan(grs, c, num_cus);
+      const double t = makespan(grs, c, num_cus, step_us);
       if (best == 0 || t < best_t || (t == best_t && c > best)) {
         best = c;
         best_t = t;

@@ -348,16 +348,16 @@ class BatchPrefillWithPagedKVCacheWrapper:
         # at run time, needs no workspace and can be planned and captured: they do where the work
         # list cannot be built or kept (plan() while capturing, a workspace too small for it) and
         # in run() for a captured call or a q of another length than the plan's.
-        self._valu_ok = g not in (1, 2, 4, 8, 16)
+        self._valu_ok = g not in (1, 2, 4, 8, 16) or self._q_dtype == torch.float32
         if self._mfma and self._valu_ok:
-            self._mfma = self._batch > 0 and self._workspace_usable(qo_indptr.device) and \
+            self._mfma = self._batch > 0 and self._sm_scale > 0 and self._workspace_usable(qo_indptr.device) and \
                 not torch.cuda.is_current_stream_capturing()
         if self._mfma:
             self._schedule(qo_indptr.device)
         self._planned = True
 
-    # rows per matrix-core work item (8 waves x 32 rows): 256 / g query tokens of one KV head
-    _ROWS = 256
+    # rows per matrix-core work item (8 waves x 32 rows, fp32 8 x 16): rows / g query tokens of one KV head
+    _ROWS, _ROWS_F32 = 256, 128
 
     def _workspace_usable(self, dev: torch.device) -> bool:
         ws = self._workspace
@@ -376,8 +376,9 @@ class BatchPrefillWithPagedKVCacheWrapper:
         # (the kernel keeps the split partials of an fp16 cache's power-of-two groups in fp16)
         half = self._q_dtype == torch.float16 and not self._valu_ok
         try:
+            rows = self._ROWS_F32 if self._q_dtype == torch.float32 else self._ROWS
             wl = prefill_work_list(qo, kp, last, g, self._hkv, self._ps, self._causal, self._d, _num_cus(dev),
-                                   ws_bytes, self._ROWS // g * g, partial_bytes=2 if half else 4)
+                                   ws_bytes, rows // g * g, partial_bytes=2 if half else 4)
         except RuntimeError:
             if not self._valu_ok:
                 raise

@@ -249,12 +249,12 @@ int pkv_batch_prefill_valu(const void* q, int64_t q_stride_n, int64_t q_stride_h
                            void* stream);
 
 /* BatchPrefillWithPagedKVCacheWrapper.run on the matrix cores (same contract as
- * pkv_batch_prefill_valu; ecahlang/main.py:432-443, :68) for fp16/bf16, head_dim 64 or 128,
- * page_size 16 and GQA groups 1 to 16 (pkv_prefill_mfma_supported).  The work list comes
+ * pkv_batch_prefill_valu; ecahlang/main.py:432-443, :68) for head_dim 64 or 128, page_size 16 and
+ * GQA groups 1 to 16 (pkv_prefill_mfma_supported).  The work list comes
  * from the wrapper's plan: n_items records of 12 int32 {request, kv_head, first query token,
  * query tokens, key chunk begin, key chunk end, partial slot or -1, kv_len, qo_len, first q row,
  * first page-list entry, 0}, each covering 256 / g query tokens, i.e. rows = (256 / g) * g query
- * rows; n_groups records of 8 int32
+ * rows (fp32 caches: 128 in place of 256); n_groups records of 8 int32
  * {first slot, slots, first q row, first query token, query tokens, kv_head, 0, 0} name the
  * split items whose partials (part_ml: float2 x rows per slot, part_o: rows x head_dim per slot,
  * fp16 for fp16 caches with a power-of-two group, else fp32) a second kernel merges.  q must be 16-byte aligned with strides that keep rows
