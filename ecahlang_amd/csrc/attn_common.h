@@ -396,5 +396,7 @@ __device__ __forceinline__ int find_seq_wave(const int32_t* indptr, int B, int64
 int decode_valu_dispatch(const DecodeParams& P, int dtype, int d, hipStream_t s);
 int decode_mfma_dispatch(const DecodeParams& P, int dtype, int d, hipStream_t s);
 bool decode_mfma_supported(int dtype, int d, int g, int hkv, int batch);
+int decode_f32_dispatch(const DecodeParams& P, int d, bool head_counters, hipStream_t s);
+bool decode_f32_supported(int dtype, int d, int g, int ps);
 
 }  // namespace pkv

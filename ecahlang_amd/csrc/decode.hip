@@ -302,6 +302,14 @@ int batch_decode(const void* q, int64_t q_stride_n, int64_t q_stride_h, const Ap
                                       num_indices, kv_last_page_len, batch, num_kv_heads, head_dim, page_size, s);
     if (rc) return rc;
   }
+  // fp32 caches on the fp32 matrix instructions (12 to 25 times the vector kernel's speed at every size
+  // tried): no plan needed, rows read 16 bytes at a time.
+  const uintptr_t kv = (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)(page_stride * es);
+  if (!(flags & PKV_DECODE_VALU) && P.q_vec && kv % 16 == 0 && decode_f32_supported(dtype, head_dim, g, page_size)) {
+    const bool head_counters =
+        (flags & PKV_DECODE_HEAD_COUNTERS) && (int64_t)batch * num_kv_heads <= PKV_MAX_HEAD_COUNTERS;
+    return decode_f32_dispatch(P, head_dim, head_counters, s);
+  }
   return decode_valu_dispatch(P, dtype, head_dim, s);
 }
 
@@ -401,8 +409,9 @@ extern "C" int pkv_batch_decode_noalloc(const void* q, int64_t q_stride_n, int64
   const int64_t ws_bytes = (int64_t)kNoAllocScratchBytes;
   // The array keeps the previous call's contents: the split counters start every call at zero
   // (a fill kernel, not a memset node, so the call can also be captured).
-  if ((rc = pkv_decode_workspace_init(ws, batch, stream))) return rc;
-  int flags = 0;
+  const bool heads = dtype == kF32 && (int64_t)batch * num_kv_heads <= PKV_MAX_HEAD_COUNTERS;
+  if ((rc = pkv_decode_workspace_init(ws, heads ? batch * num_kv_heads : batch, stream))) return rc;
+  int flags = heads ? PKV_DECODE_HEAD_COUNTERS : 0;
   if (page_size == 16 && num_qo_heads % num_kv_heads == 0 &&
       decode_mfma_supported(dtype, head_dim, num_qo_heads / num_kv_heads, num_kv_heads, batch)) {
     if ((rc = pkv_decode_plan(kv_indptr, kv_indices, num_indices, kv_last_page_len, nullptr, batch, num_qo_heads,

@@ -53,8 +53,9 @@ def _unsupported(pos_encoding_mode, window_left, logits_soft_cap, rope_scale, ro
         raise NotImplementedError("in-kernel RoPE is not implemented")
 
 
-_DECODE_VALU, _DECODE_DYNAMIC, _DECODE_PLANNED = 1, 2, 4  # pkv_batch_decode flags (include/pagedkv.h)
+_DECODE_VALU, _DECODE_DYNAMIC, _DECODE_PLANNED, _DECODE_HEAD_COUNTERS = 1, 2, 4, 8  # pkv_batch_decode flags (include/pagedkv.h)
 _PLAN_CASCADE = 1  # pkv_decode_plan flag
+_MAX_HEAD_COUNTERS = 2048  # PKV_MAX_HEAD_COUNTERS
 _INIT_COUNTERS = 8192  # decode split counters zeroed when a workspace is given
 
 class BatchDecodeWithPagedKVCacheWrapper:
@@ -160,11 +161,17 @@ class BatchDecodeWithPagedKVCacheWrapper:
             check(int(need), "decode plan")
         if need > self._workspace.numel() * self._workspace.element_size():
             raise RuntimeError(f"decode workspace too small: need {need} bytes")
-        if self._batch > self._counters_ready:
-            check(lib().pkv_decode_workspace_init(self._workspace.data_ptr(), self._batch,
-                                                  stream_ptr(dev)), "decode plan")
-        self._counters_ready = self._batch  # (the schedule is written after these)
+        # Split counters: one a sequence, the schedule after them; without a schedule, one a sequence
+        # and KV head (up to a number that no workspace's partials reach down to).
         self._flags = 0 if deterministic else _DECODE_DYNAMIC
+        counters = self._batch
+        if not self._mfma and self._batch * self._hkv <= _MAX_HEAD_COUNTERS:
+            counters *= self._hkv
+            self._flags |= _DECODE_HEAD_COUNTERS
+        if counters > self._counters_ready:
+            check(lib().pkv_decode_workspace_init(self._workspace.data_ptr(), counters, stream_ptr(dev)),
+                  "decode plan")
+        self._counters_ready = counters  # (the words after these are overwritten)
         shared = 0
         if kv_shared_pages is not None:
             self._shared = _i32(kv_shared_pages, "kv_shared_pages")

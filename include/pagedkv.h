@@ -121,9 +121,9 @@ int pkv_decode_schedule_layout(int32_t batch, int32_t num_qo_heads, int32_t head
                                int32_t num_ctas, int64_t num_indices, int64_t workspace_bytes,
                                int64_t* out);
 
-/* Zeroes the split-merge counters at the head of the workspace (the device half of plan).
- * pkv_batch_decode leaves them zero again when it finishes, so this is needed only when the
- * buffer is fresh or the batch grows. */
+/* Zeroes the first `batch` split-merge counters (int32) at the head of the workspace (the device
+ * half of plan).  pkv_batch_decode leaves them zero again when it finishes, so this is needed only
+ * when the buffer is fresh or the batch grows. */
 int pkv_decode_workspace_init(void* workspace, int32_t batch, void* stream);
 
 /* The device half of BatchDecodeWithPagedKVCacheWrapper.plan (ecahlang/main.py:341-347,
@@ -171,15 +171,21 @@ int pkv_decode_uses_mfma(int32_t dtype, int32_t head_dim, int32_t num_qo_heads,
  * sequence with no tokens yields zeros.  num_ctas workgroups each stream an equal share of
  * the batch's pages.  flags: PKV_DECODE_PLANNED says pkv_decode_plan has written this page
  * table's schedule into the workspace (same batch, num_indices and num_ctas), which the
- * matrix-core kernel needs; without it the vector-ALU kernel runs.  PKV_DECODE_VALU selects the
+ * matrix-core kernel needs; without it, and for fp32 caches, the kernels that need no plan run.  PKV_DECODE_VALU selects the
  * vector-ALU kernel (cross-checks); PKV_DECODE_DYNAMIC lets that kernel's waves take pages on
  * demand (the summation order, and so the last bits of the result, then vary from call to
- * call).  Otherwise the result is bitwise reproducible for a given num_ctas.  Page ids outside
- * [0, num_pages) and page-list entries past num_indices are never read (their tokens are
+ * call).  PKV_DECODE_HEAD_COUNTERS (fp32 caches) says that the first batch * num_kv_heads words of
+ * the workspace are zeroed counters (pkv_decode_workspace_init of that many; a plan of the matrix-core
+ * schedule overwrites those past batch), so that the merge of a split sequence is shared by its KV
+ * heads' workgroups; it is ignored above PKV_MAX_HEAD_COUNTERS of them.  Without PKV_DECODE_DYNAMIC
+ * the result is bitwise reproducible for a given num_ctas and flags.  Page ids outside [0, num_pages)
+ * and page-list entries past num_indices are never read (their tokens are
  * treated as absent); pages before kv_indptr[0] belong to no sequence. */
 #define PKV_DECODE_VALU 1
 #define PKV_DECODE_DYNAMIC 2
 #define PKV_DECODE_PLANNED 4
+#define PKV_DECODE_HEAD_COUNTERS 8
+#define PKV_MAX_HEAD_COUNTERS 2048
 int pkv_batch_decode(const void* q, int64_t q_stride_n, int64_t q_stride_h, const void* k_cache,
                      const void* v_cache, int64_t page_stride, int64_t num_pages,
                      const int32_t* kv_indptr, const int32_t* kv_indices, int64_t num_indices,

@@ -299,6 +299,47 @@ def test_decode_dynamic_pages_match_oracle(name):
         np.testing.assert_allclose(o.float().cpu().numpy(), ref, **TOL[wb.dtype])
 
 
+# fp32 decode: page and part edges, groups and head counts, over 64 sequences (more than one round of the part
+# search), more head counters than the flag allows, a lone long sequence, one part of over 64 pages a wave.
+F32_DECODE = {
+    "g4_d64": (lambda: workloads.build_batch([1, 15, 16, 17, 127, 128, 129, 640, 2049], [1] * 9, 32, 8, 64, torch.float32, 81), None),
+    "g7_d128": (lambda: workloads.build_batch([1, 16, 300, 1030], [1] * 4, 14, 2, 128, torch.float32, 82), None),
+    "g16_d128": (lambda: workloads.build_batch([33, 500], [1] * 2, 16, 1, 128, torch.float32, 83), None),
+    "g1_hkv3_d64": (lambda: workloads.build_batch([5, 700, 48], [1] * 3, 3, 3, 64, torch.float32, 84), None),
+    "b70_d64": (lambda: workloads.build_batch([(7 * i) % 190 + 1 for i in range(70)], [1] * 70, 4, 2, 64, torch.float32, 85), None),
+    "b300_hkv8_d64": (lambda: workloads.build_batch([(5 * i) % 150 + 1 for i in range(300)], [1] * 300, 8, 8, 64,
+                                                    torch.float32, 86), None),
+    "b1_long_d64": (lambda: workloads.build_batch([9000], [1], 8, 2, 64, torch.float32, 87), None),
+    "b1_one_part_d128": (lambda: workloads.build_batch([4200, 40], [1] * 2, 8, 2, 128, torch.float32, 88), 1),
+}
+
+
+@pytest.mark.parametrize("name", list(F32_DECODE))
+def test_decode_fp32_on_the_matrix_cores(name):
+    """Against the float64 oracle, and no further from it than twice the vector kernel (the order of the
+    sums is all that differs; 1e-7 of the result's norm is below either's rounding).  Slots no sequence
+    owns hold NaN: they reach nothing.  A second run finds the counters at zero."""
+    make, ctas = F32_DECODE[name]
+    wb = make()
+    dv = wb.to(DEV)
+    _append_dev(dv)
+    _, vals = _oracle_appended(wb)
+    ref = kv_ref.decode(wb.q.float().numpy(), vals, wb.indptr.numpy(), wb.indices.numpy(), wb.last.numpy(), wb.ps)
+    for b in range(wb.batch):
+        page, last = int(wb.indices[int(wb.indptr[b + 1]) - 1]), int(wb.last[b])
+        dv.cache[page, :, last:] = float("nan")
+    w = BatchDecodeWithPagedKVCacheWrapper(torch.empty(64 << 20, dtype=torch.uint8, device=DEV), "NHD")
+    w.plan(dv.indptr, dv.indices, dv.last, dv.hq, dv.hkv, dv.d, dv.ps, q_data_type=dv.dtype, num_ctas=ctas)
+    out = torch.full((wb.batch, dv.hq, dv.d + 1), 7.0, device=DEV)[:, :, :dv.d]  # rows that are not 16-byte aligned
+    o = w.run(dv.q, dv.cache)
+    again, ov = w.run(dv.q, dv.cache, out=out), w.run(dv.q, dv.cache, force_valu=True)
+    torch.cuda.synchronize()
+    assert torch.equal(o, again)
+    err, err_v = (np.linalg.norm(x.double().cpu().numpy() - ref) for x in (o, ov))
+    assert err <= max(2 * err_v, 1e-7 * np.linalg.norm(ref)) and err <= 1e-6 * np.linalg.norm(ref), (err, err_v)
+    np.testing.assert_allclose(o.cpu().numpy(), ref, **TOL[torch.float32])
+
+
 @pytest.mark.parametrize("force_valu", [False, True])
 def test_decode_pages_before_first_sequence(force_valu):
     # kv_indptr[0] > 0: the leading page-list entries belong to no sequence
