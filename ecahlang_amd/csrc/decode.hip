@@ -226,6 +226,17 @@ int launch_append_last(const AppendRows& a, int es, void* k_cache, void* v_cache
   return (int)hipGetLastError();
 }
 
+// The new rows as the decode kernels' fused append takes them, if they are 16-byte aligned.
+bool append_rows_16(const AppendRows& a, int es, DecodeParams* P) {
+  const uintptr_t m = (uintptr_t)a.k | (uintptr_t)a.v;
+  const int64_t st = (a.k_sn | a.k_sh | a.v_sn | a.v_sh) * es;
+  if (m % 16 || st % 16) return false;
+  P->ak = (const char*)a.k;
+  P->av = (const char*)a.v;
+  P->ak_sn = a.k_sn * es, P->ak_sh = a.k_sh * es, P->av_sn = a.v_sn * es, P->av_sh = a.v_sh * es;
+  return true;
+}
+
 int batch_decode(const void* q, int64_t q_stride_n, int64_t q_stride_h, const AppendRows* app, void* k_cache,
                  void* v_cache, int64_t page_stride, int64_t num_pages, const int32_t* kv_indptr,
                  const int32_t* kv_indices, int64_t num_indices, const int32_t* kv_last_page_len, int32_t batch,
@@ -283,13 +294,7 @@ int batch_decode(const void* q, int64_t q_stride_n, int64_t q_stride_h, const Ap
       // writes the token there) for the fixed page order of the plan's ranges and 16-byte rows
       // (the page that receives the token is never part of a shared prefix: the plan keeps it
       // in the sequence's own pages); otherwise it is a launch of its own before the decode.
-      const uintptr_t m = (uintptr_t)app->k | (uintptr_t)app->v;
-      const int64_t st = (app->k_sn | app->k_sh | app->v_sn | app->v_sh) * es;
-      if (!P.dynamic && m % 16 == 0 && st % 16 == 0) {
-        P.ak = (const char*)app->k;
-        P.av = (const char*)app->v;
-        P.ak_sn = app->k_sn * es, P.ak_sh = app->k_sh * es, P.av_sn = app->v_sn * es, P.av_sh = app->v_sh * es;
-      } else {
+      if (P.dynamic || !append_rows_16(*app, es, &P)) {
         const int rc = launch_append_last(*app, es, k_cache, v_cache, page_stride, num_pages, kv_indptr, kv_indices,
                                           num_indices, kv_last_page_len, batch, num_kv_heads, head_dim, page_size, s);
         if (rc) return rc;
@@ -297,15 +302,17 @@ int batch_decode(const void* q, int64_t q_stride_n, int64_t q_stride_h, const Ap
     }
     return decode_mfma_dispatch(P, dtype, head_dim, s);
   }
-  if (app) {
+  // fp32 caches on the fp32 matrix instructions (12 to 25 times the vector kernel's speed at every size
+  // tried): no plan needed, rows read 16 bytes at a time.
+  const uintptr_t kv = (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)(page_stride * es);
+  const bool f32 = !(flags & PKV_DECODE_VALU) && P.q_vec && kv % 16 == 0 &&
+                   decode_f32_supported(dtype, head_dim, g, page_size);
+  if (app && !(f32 && append_rows_16(*app, es, &P))) {
     const int rc = launch_append_last(*app, es, k_cache, v_cache, page_stride, num_pages, kv_indptr, kv_indices,
                                       num_indices, kv_last_page_len, batch, num_kv_heads, head_dim, page_size, s);
     if (rc) return rc;
   }
-  // fp32 caches on the fp32 matrix instructions (12 to 25 times the vector kernel's speed at every size
-  // tried): no plan needed, rows read 16 bytes at a time.
-  const uintptr_t kv = (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)(page_stride * es);
-  if (!(flags & PKV_DECODE_VALU) && P.q_vec && kv % 16 == 0 && decode_f32_supported(dtype, head_dim, g, page_size)) {
+  if (f32) {
     const bool head_counters =
         (flags & PKV_DECODE_HEAD_COUNTERS) && (int64_t)batch * num_kv_heads <= PKV_MAX_HEAD_COUNTERS;
     return decode_f32_dispatch(P, head_dim, head_counters, s);

@@ -44,7 +44,7 @@ __device__ __forceinline__ int parts_of(int np, int aim, int max_parts) {
   return max(min((np + aim - 1) / aim, max_parts), 1);
 }
 
-template <int D>
+template <int D, bool APP>
 __global__ __launch_bounds__(W * 64, D == 64 ? 4 : 2) void decode_f32_kernel(DecodeParams P, int nr, int max_parts, int head_counters) {
   constexpr int QS = D / 16;  // 16-dim pieces of a row
   constexpr int NC = D / 64;  // 64-dim pieces of the output
@@ -113,6 +113,15 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 4 : 2) void decode_f32_kernel(Dec
   gfloat* out = (gfloat*)P.out;
   const bool o16 = (((uintptr_t)P.out | (uintptr_t)(P.o_sn * 4) | (uintptr_t)(P.o_sh * 4)) & 15) == 0;
 
+  // The step's new token (pkv_batch_decode_append) goes to the sequence's last position: page app_pi of
+  // the page list, row app_row.  Its rows are loaded in place of that row of the page, and stored there
+  // once they are in (one wave of one workgroup loads the page for this KV head).  A launch of its own
+  // for it costs 3 us more a call (18.9 and 21.8).  APP keeps its selects out of calls without one (0.6 us).
+  const bool app = APP && s0 >= 0 && np > 0 && avail == np && lastp >= 0 && lastp <= 16 && len > 0;
+  const int app_pi = app ? s0 + (len - 1) / 16 : -1, app_row = (len - 1) & 15;
+  const float* akp = app ? reinterpret_cast<const float*>(P.ak + b * P.ak_sn + h * P.ak_sh) + 4 * lg : nullptr;
+  const float* avp = app ? reinterpret_cast<const float*>(P.av + b * P.av_sn + h * P.av_sh) + 4 * lr : nullptr;
+
   // Rows of page k of this wave.  The loads are unconditional, so that every path has the same ones
   // in flight and the waits stay exact: past the wave's last page, and for an id outside the pool,
   // they read a query row instead.
@@ -122,22 +131,26 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 4 : 2) void decode_f32_kernel(Dec
     return k < n && pid >= 0 && (int64_t)pid < P.num_pages ? pid : -1;
   };
   const float* const dummy = qc - 4 * lg;
-  auto load_k = [&](int pid) __attribute__((always_inline)) {
+  auto load_k = [&](int pid, int pi) __attribute__((always_inline)) {
     const float* kp = pid >= 0 ? kc + pid * P.page_stride : dummy;
+    if (APP) kp = pid >= 0 && pi == app_pi && lr == app_row ? akp : kp;
 #pragma unroll
     for (int s = 0; s < QS; ++s) kr[s] = *reinterpret_cast<const f4*>(kp + 16 * s);
   };
-  auto load_v = [&](int pid) __attribute__((always_inline)) {
+  auto load_v = [&](int pid, int pi) __attribute__((always_inline)) {
     const float* vp = pid >= 0 ? vc + pid * P.page_stride : dummy;
     const int64_t rs = pid >= 0 ? rowstride : 0;
+    const int ar = APP && pid >= 0 && pi == app_pi ? app_row - 4 * lg : -1;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 4; ++i) {
+      const float* rp = APP && i == ar ? avp : vp + i * rs;
 #pragma unroll
-      for (int c = 0; c < NC; ++c) vr[i][c] = *reinterpret_cast<const f4*>(vp + i * rs + 64 * c);
+      for (int c = 0; c < NC; ++c) vr[i][c] = *reinterpret_cast<const f4*>(rp + 64 * c);
+    }
   };
   int k = 0, pid = page_of(0);
-  load_k(pid);
-  load_v(pid);
+  load_k(pid, p0 + wave);
+  load_v(pid, p0 + wave);
 
   f4 qr[QS];  // in base-2 units
 #pragma unroll
@@ -161,13 +174,26 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 4 : 2) void decode_f32_kernel(Dec
       }
     const int left = len - 16 * (pi - s0);
     const int nv = pid < 0 || left < 0 ? 0 : left;  // tokens of the page that exist (16 and above: all)
+    if (APP && pi == app_pi && pid >= 0) {
+      typedef __attribute__((address_space(1))) f4 gf4;
+      if (lr == app_row) {
+#pragma unroll
+        for (int s = 0; s < QS; ++s) *(gf4*)(kc + pid * P.page_stride + 16 * s) = kr[s];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (4 * lg + i == app_row) {
+#pragma unroll
+          for (int c = 0; c < NC; ++c) *(gf4*)(vc + pid * P.page_stride + i * rowstride + 64 * c) = vr[i][c];
+        }
+    }
     ++k;
     if ((k & 63) == 0) {
       pidv = P.indices[min(pi + W * (1 + lane), end - 1)];
       __builtin_amdgcn_s_waitcnt(0x0F70);  // (compiler-visible vmcnt(0): the usual path waits for nothing)
     }
     pid = page_of(k);
-    load_k(pid);
+    load_k(pid, pi + W);
     sa += sb;
     if (nv < 16) {
       // tokens past the sequence's end: no score, and rows read as zeros (0 * NaN would poison P.V)
@@ -203,7 +229,7 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 4 : 2) void decode_f32_kernel(Dec
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           o[c][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[i][c][e], sa[i], o[c][e], 0, 0, 0);
-    load_v(pid);
+    load_v(pid, pi + W);
   }
 
   // ---- the waves' states in wave order (a wave without a page: no mass)
@@ -336,10 +362,16 @@ int decode_f32_dispatch(const DecodeParams& P, int d, bool head_counters, hipStr
   const int64_t wgs = ((int64_t)nr + P.batch) * P.hkv;
   if (wgs > INT32_MAX) return kBadArg;
   const dim3 grid((unsigned)wgs);
-  if (d == 64)
-    hipLaunchKernelGGL((decode_f32_kernel<64>), grid, dim3(W * 64), 0, s, P, nr, max_parts, head_counters ? 1 : 0);
-  else
-    hipLaunchKernelGGL((decode_f32_kernel<128>), grid, dim3(W * 64), 0, s, P, nr, max_parts, head_counters ? 1 : 0);
+#define PKV_DECODE_F32(D, APP)                                                                               \
+  hipLaunchKernelGGL((decode_f32_kernel<D, APP>), grid, dim3(W * 64), 0, s, P, nr, max_parts, head_counters ? 1 : 0)
+  if (d == 64) {
+    if (P.ak) PKV_DECODE_F32(64, true);
+    else PKV_DECODE_F32(64, false);
+  } else {
+    if (P.ak) PKV_DECODE_F32(128, true);
+    else PKV_DECODE_F32(128, false);
+  }
+#undef PKV_DECODE_F32
   return (int)hipGetLastError();
 }
 

@@ -206,9 +206,10 @@ int pkv_batch_decode(const void* q, int64_t q_stride_n, int64_t q_stride_h, cons
  * bitwise those of pkv_append_paged_kv_cache at those positions + pkv_batch_decode.  A sequence
  * whose page list is empty or cut at num_indices, whose kv_last_page_len is outside
  * [0, page_size], whose position is negative or whose page id is outside the pool gets no
- * append.  On the matrix-core kernel (PKV_DECODE_PLANNED, no
- * PKV_DECODE_DYNAMIC, a plan without PKV_PLAN_CASCADE, 16-byte aligned rows) the append rides
- * in the decode launch; otherwise it is a launch of its own before the decode. */
+ * append.  With 16-byte aligned rows
+ * the append rides in the decode launch of the matrix-core kernels (PKV_DECODE_PLANNED without
+ * PKV_DECODE_DYNAMIC, and fp32 caches), where a slot that receives a token is read by its own
+ * sequence only; otherwise it is a launch of its own before the decode. */
 int pkv_batch_decode_append(const void* q, int64_t q_stride_n, int64_t q_stride_h,
                             const void* append_key, int64_t k_stride_n, int64_t k_stride_h,
                             const void* append_value, int64_t v_stride_n, int64_t v_stride_h,

@@ -318,16 +318,18 @@ F32_DECODE = {
 def test_decode_fp32_on_the_matrix_cores(name):
     """Against the float64 oracle, and no further from it than twice the vector kernel (the order of the
     sums is all that differs; 1e-7 of the result's norm is below either's rounding).  Slots no sequence
-    owns hold NaN: they reach nothing.  A second run finds the counters at zero."""
+    owns hold NaN: they reach nothing.  A second run finds the counters at zero.  The append inside the
+    launch leaves the same bits as the append before it."""
     make, ctas = F32_DECODE[name]
     wb = make()
     dv = wb.to(DEV)
+    bare = dv.cache.clone()
     _append_dev(dv)
     _, vals = _oracle_appended(wb)
     ref = kv_ref.decode(wb.q.float().numpy(), vals, wb.indptr.numpy(), wb.indices.numpy(), wb.last.numpy(), wb.ps)
     for b in range(wb.batch):
         page, last = int(wb.indices[int(wb.indptr[b + 1]) - 1]), int(wb.last[b])
-        dv.cache[page, :, last:] = float("nan")
+        dv.cache[page, :, last:] = bare[page, :, last:] = float("nan")
     w = BatchDecodeWithPagedKVCacheWrapper(torch.empty(64 << 20, dtype=torch.uint8, device=DEV), "NHD")
     w.plan(dv.indptr, dv.indices, dv.last, dv.hq, dv.hkv, dv.d, dv.ps, q_data_type=dv.dtype, num_ctas=ctas)
     out = torch.full((wb.batch, dv.hq, dv.d + 1), 7.0, device=DEV)[:, :, :dv.d]  # rows that are not 16-byte aligned
@@ -335,6 +337,8 @@ def test_decode_fp32_on_the_matrix_cores(name):
     again, ov = w.run(dv.q, dv.cache, out=out), w.run(dv.q, dv.cache, force_valu=True)
     torch.cuda.synchronize()
     assert torch.equal(o, again)
+    fused = w.run(dv.q, bare, append_kv=(dv.k_new, dv.v_new))
+    assert torch.equal(fused, o) and np.array_equal(_bits(bare), _bits(dv.cache))
     err, err_v = (np.linalg.norm(x.double().cpu().numpy() - ref) for x in (o, ov))
     assert err <= max(2 * err_v, 1e-7 * np.linalg.norm(ref)) and err <= 1e-6 * np.linalg.norm(ref), (err, err_v)
     np.testing.assert_allclose(o.cpu().numpy(), ref, **TOL[torch.float32])
