@@ -33,6 +33,10 @@ __device__ __forceinline__ uint32_t fkey(float f) {
   if (f != f) return 0u;
   return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
+// The float whose fkey is k (k != 0).
+__device__ __forceinline__ float key_float(uint32_t k) {
+  return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
+}
 // Mass of a logit in 32-bit fixed point: floor(exp(x - max) * 2^32), capped at 4294967040 (the
 // largest float below 2^32), so it converts with one 32-bit instruction (a float -> 64-bit
 // integer conversion is a sequence of ten; this runs for every logit on several passes).
@@ -285,12 +289,12 @@ __device__ __forceinline__ void sample_row(const RowT& row, SampleLds& L, int b,
   }
 }
 
-// Which kernel samples a row: its whole distribution (no top-k, no top-p filter), a top-k filter
-// with k <= kTopKMax (then any top-p), or anything else (the one-workgroup kernel).
-enum RowKind : int { kWholeRow = 0, kTopKRow = 1, kOtherRow = 2 };
+// Which kernels sample a row: its whole distribution (no top-k, no top-p filter), a top-k filter with
+// k <= kTopKMax (then any top-p), a top-p filter alone, or anything else (the one-workgroup kernel).
+enum RowKind : int { kWholeRow = 0, kTopKRow = 1, kTopPRow = 2, kOtherRow = 3 };
 constexpr int kTopKMax = 256;
 __host__ __device__ __forceinline__ int row_kind_of(int k, float pp, int vocab) {
-  if (k <= 0 || k >= vocab) return pp < 1.f ? kOtherRow : kWholeRow;
+  if (k <= 0 || k >= vocab) return pp < 1.f ? kTopPRow : kWholeRow;
   return k <= kTopKMax ? kTopKRow : kOtherRow;
 }
 __device__ __forceinline__ int row_kind(int b, int vocab, const int32_t* top_k, int32_t top_k_all,
@@ -306,63 +310,110 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const T* logits, int64
                                                           const int32_t* fallback) {
   __shared__ SampleLds L;
   const int b = blockIdx.x;
-  // with the split kernels in use, whole-distribution and small-top-k rows are theirs, except
-  // the rows they handed back (fallback[b])
+  // with the split kernels in use, all kinds but kOtherRow are theirs, except the rows they handed
+  // back (fallback[b])
   if (split && row_kind(b, vocab, top_k, top_k_all, top_p, top_p_all) != kOtherRow && !fallback[b]) return;
   const T* p = logits + (int64_t)b * row_stride;
   const Row<T> row{p, vocab, ((uintptr_t)p % 16) == 0};
   sample_row<T>(row, L, b, vocab, top_k, top_k_all, top_p, top_p_all, uniform, out);
 }
 
-// ---- Whole-distribution rows (the serving loop's default request: top_k 0, top_p 1) over many
-// workgroups per row.  One workgroup per row leaves half the chip idle and is bound by the
-// vector ALU of the CUs it has, so these rows are cut into slices of kSliceTiles tiles of
-// kSplitTile logits, one workgroup per (slice, row), in two launches:
-//   split_max_kernel     each slice's largest logit
-//   split_sample_kernel  the row's largest logit from the slices', each tile's mass (the same
-//                        integer masses as sample_row), then the workgroup that finishes its
-//                        slice last (a per-row counter) finds the tile and the token holding the
-//                        row's uniform, walking in vocabulary order.
-// The masses and the target are the integers sample_row computes, so the token is identical.
+// ---- Rows over many workgroups.  One workgroup per row leaves half the chip idle and is bound by the
+// vector ALU of the CUs it has (eight passes over a top-p row: 165 us for 32 rows of 151,936), so rows
+// are cut into slices of kSliceTiles tiles of kSplitTile logits, one workgroup per (slice, row), in
+// launches that every kind of row shares:
+//   split_scan_kernel    the logits scaled, if asked for; each slice's largest and smallest logit, and
+//                        the largest of each group of logits (256 of them at a vocabulary of 151,936)
+//   split_pass_kernel    whole rows: each tile's mass, then the workgroup that finishes the row's last
+//                        slice finds the tile and the token; top-k rows: the token; top-p rows: the
+//                        mass by distance from the row's largest logit
+//   split_finish_kernel  top-p rows: the threshold and the token
+//   sample_kernel        other rows, and rows handed back
+// All masses and targets are the integers sample_row computes, so the token is identical.
+// What bounds them: the scan moves the logits, the penalties and the scaled logits (156 MB in 33 us at
+// 128 x 151,936 fp16); the later launches are chains of latencies (arrivals, LDS rounds) beside 3 to 4
+// TB/s of reading.  128 rows of 151,936 fp16 logits, penalty and temperature, two requests in eight
+// top-p alone and five top-k: 260 us when every filtered row but small top-k ran on one workgroup and
+// the scaling was a launch of its own, 96 us; without the scaling 223 and 75; all top_k 50 / top_p 0.9:
+// 54.8 and 32.5; one row: 34.7 and 22.4.
 constexpr int kSplitThreads = 256;
 constexpr int kSplitTile = kSplitThreads * 8;  // 8 logits per thread
 constexpr int kSliceTiles = 8;
 constexpr int kMaxSplitTiles = 2048;           // vocabularies up to 4 M
 
-constexpr int kCandCap = 512;    // candidates a slice hands over for a top-k row
-constexpr int kMergeRegs = 16;   // candidates per lane of the merging wave (64 * 16 per row)
+constexpr int kCandCap = 512;    // candidates a slice hands over for a top-p row
 
-struct SplitWs {
-  uint64_t* tmass;    // [rows][ntiles] tile masses (whole rows)
-  uint64_t* cand;     // [rows][slices][kCandCap] candidates, index << 32 | key (top-k rows)
-  float* smax;        // [rows][slices] slice maxima (whole rows)
-  int32_t* ncand;     // [rows][slices] candidates per slice, -1: more than kCandCap
-  int32_t* counter;   // [rows] slices finished
-  int32_t* fallback;  // [rows] 1: handed back to the one-workgroup kernel
-};
+constexpr int kGroups = 1024;    // group maxima per row at most
+constexpr int kPBins = 512;      // bins of a top-p row's mass
+constexpr int kPCandMax = 1024;  // candidates of a top-p row
+
 __host__ __device__ inline int split_tiles(int vocab) { return (vocab + kSplitTile - 1) / kSplitTile; }
 __host__ __device__ inline int split_slices(int vocab) { return (split_tiles(vocab) + kSliceTiles - 1) / kSliceTiles; }
+// Where a top-p row's threshold lies: its bin (-1: no mass), the mass of the bins above it, the mass to
+// reach.
+struct ToppBin {
+  uint64_t above, need;
+  float mx, scale;  // (PBins)
+  int64_t bin;
+};
+// The groups whose maxima a row keeps, at most kGroups of them and as small as that allows: a thread's
+// logits of 2^tg tiles of a slice, over 2^gl neighbouring threads.
+struct GroupShape {
+  int tg, gl, per_slice, ps, n;  // (per_slice = 2^ps)
+};
+inline GroupShape group_shape(int vocab) {
+  const int S = split_slices(vocab);
+  GroupShape g{0, 0, 0, 0, 0};
+  auto count = [&]() { return S * ((kSliceTiles * kSplitThreads) >> (g.tg + g.gl)); };
+  while (count() > kGroups && (1 << g.tg) < kSliceTiles) ++g.tg;
+  while (count() > kGroups && g.gl < 6) ++g.gl;
+  g.per_slice = (kSliceTiles * kSplitThreads) >> (g.tg + g.gl);
+  while ((1 << g.ps) < g.per_slice) ++g.ps;
+  g.n = S * g.per_slice;
+  return g;
+}
+
+constexpr int kCountStride = 32;
+struct SplitWs {
+  uint64_t* tmass;    // [rows][ntiles] tile masses (whole and top-p rows)
+  uint64_t* hist;     // [rows][slices][kPBins] masses by bin (top-p rows)
+  uint64_t* cand;     // [rows][slices][kCandCap] candidates, index << 32 | key (top-p rows)
+  ToppBin* bin;       // [rows] where the threshold lies (top-p rows)
+  uint16_t* gmax;     // [rows][kGroups] group maxima: the keys' upper halves
+  float* smax;        // [rows][slices] slice maxima
+  float* smin;        // [rows][slices] slice minima
+  int32_t* ncand;     // [rows][slices] candidates per slice, -1: more than kCandCap
+  int32_t* counter;   // [rows][kCountStride] slices finished: a cache line each
+  int32_t* fallback;  // [rows] 1: handed back to the one-workgroup kernel
+  GroupShape g;
+};
 __host__ __device__ inline int64_t split_ws_bytes(int rows, int vocab) {
   const int64_t S = split_slices(vocab);
-  return (int64_t)rows * (split_tiles(vocab) * 8 + S * kCandCap * 8 + S * 4 + S * 4 + 4 + 4);
+  return (int64_t)rows * (split_tiles(vocab) * 8 + S * (kPBins + kCandCap) * 8 + (int64_t)sizeof(ToppBin) + kGroups * 2 + S * 12 + kCountStride * 4 + 4);
 }
-__host__ __device__ inline SplitWs split_ws(void* ws, int rows, int vocab) {
+inline SplitWs split_ws(void* ws, int rows, int vocab) {
   const int64_t S = split_slices(vocab);
   char* c = reinterpret_cast<char*>(ws);
+  auto take = [&](int64_t bytes) {
+    char* p = c;
+    c += (int64_t)rows * bytes;
+    return p;
+  };
   SplitWs w;
-  w.tmass = reinterpret_cast<uint64_t*>(c);
-  c += (int64_t)rows * split_tiles(vocab) * 8;
-  w.cand = reinterpret_cast<uint64_t*>(c);
-  c += (int64_t)rows * S * kCandCap * 8;
-  w.smax = reinterpret_cast<float*>(c);
-  c += (int64_t)rows * S * 4;
-  w.ncand = reinterpret_cast<int32_t*>(c);
-  c += (int64_t)rows * S * 4;
-  w.counter = reinterpret_cast<int32_t*>(c);
-  c += (int64_t)rows * 4;
-  w.fallback = reinterpret_cast<int32_t*>(c);
+  w.tmass = reinterpret_cast<uint64_t*>(take(split_tiles(vocab) * 8));
+  w.hist = reinterpret_cast<uint64_t*>(take(S * kPBins * 8));
+  w.cand = reinterpret_cast<uint64_t*>(take(S * kCandCap * 8));
+  w.bin = reinterpret_cast<ToppBin*>(take(sizeof(ToppBin)));
+  w.gmax = reinterpret_cast<uint16_t*>(take(kGroups * 2));
+  w.smax = reinterpret_cast<float*>(take(S * 4));
+  w.smin = reinterpret_cast<float*>(take(S * 4));
+  w.ncand = reinterpret_cast<int32_t*>(take(S * 4));
+  w.counter = reinterpret_cast<int32_t*>(take(kCountStride * 4));
+  w.fallback = reinterpret_cast<int32_t*>(take(4));
+  w.g = group_shape(vocab);
   return w;
 }
+static_assert(kMaxSplitTiles / kSliceTiles * (kSplitThreads >> 6) <= kGroups, "the largest rows' groups");
 
 // Thread t's 8 logits of tile j: indices j * kSplitTile + 8 t .. + 7 (ok: inside the row).
 template <typename T>
@@ -408,142 +459,296 @@ struct SliceLoad {
       for (int v = 0; v < R; ++v) raw[jj][v] = *reinterpret_cast<const uint4*>(p + base + v * (16 / sizeof(T)));
     }
   }
-  __device__ __forceinline__ void get(const T* p, int vocab, bool vec, int j, int jj, float (&x)[8],
-                                      bool (&ok)[8]) const {
+  __device__ __forceinline__ void get_raw(const T* p, int vocab, bool vec, int j, int jj, T (&e)[8],
+                                          bool (&ok)[8]) const {
     const int base = j * kSplitTile + 8 * (int)threadIdx.x;
     if (vec && vocab >= 8 && base + 8 <= vocab) {
-      T e[8];
       __builtin_memcpy(e, raw[jj], 8 * sizeof(T));
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        x[k] = to_f32(e[k]);
-        ok[k] = true;
-      }
+      for (int k = 0; k < 8; ++k) ok[k] = true;
     } else {
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         ok[k] = base + k < vocab;
-        x[k] = ok[k] ? to_f32(p[base + k]) : 0.f;
+        if (ok[k]) e[k] = p[base + k];
       }
     }
   }
+  __device__ __forceinline__ void get(const T* p, int vocab, bool vec, int j, int jj, float (&x)[8],
+                                      bool (&ok)[8]) const {
+    T e[8];
+    get_raw(p, vocab, vec, j, jj, e, ok);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) x[k] = ok[k] ? to_f32(e[k]) : 0.f;
+  }
 };
 
-__device__ __forceinline__ float block_max256(float v, float* red) {
-  v = wave_max_f32(v);
+// The tiles' sums of a slice, each over the workgroup: add() per tile, then store() by all threads.
+struct TileSums {
+  uint64_t (*red)[4];  // [kSliceTiles][4] in LDS
+  __device__ __forceinline__ void add(int jj, uint64_t m) const {
+    m = wave_sum_u64(m);
+    if ((threadIdx.x & 63) == 0) red[jj][threadIdx.x >> 6] = m;
+  }
+  // (written through to device scope)
+  __device__ __forceinline__ void store(uint64_t* tm, int n) const {
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t < n)
+      __hip_atomic_store(tm + t, red[t][0] + red[t][1] + red[t][2] + red[t][3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+};
+// Largest of mx (x) and smallest of mn (y) over the workgroup; red: 8 floats.
+__device__ __forceinline__ float2 block_range256(float mx, float mn, float* red) {
+  mx = wave_max_f32(mx);
+  mn = wave_max_f32(-mn);
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  if ((threadIdx.x & 63) == 0) {
+    red[threadIdx.x >> 6] = mx;
+    red[4 + (threadIdx.x >> 6)] = mn;
+  }
   __syncthreads();
-  return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  return make_float2(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])),
+                     -fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7])));
 }
-__device__ __forceinline__ uint64_t block_sum256(uint64_t v, uint64_t* red) {
-  v = wave_sum_u64(v);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return red[0] + red[1] + red[2] + red[3];
+// One scaled logit: x / penalty rounded to T, then / temperature in fp32, both IEEE divisions (a divisor
+// of 1 leaves the value unchanged).
+template <typename T>
+__device__ __forceinline__ float scale_logit(T xv, T pv, bool pen, float t) {
+  float y = to_f32(xv);
+  if (pen) {
+    const float d = to_f32(pv);
+    if (d != 1.f) y = to_f32(from_f32<T>(y / d));
+  }
+  if (t != 1.f) y = y / t;
+  return y;
 }
 
+// What split_scan_kernel<T, true> scales by, and where the fp32 results go (rows of out_stride floats,
+// a multiple of 4).
 template <typename T>
-__global__ __launch_bounds__(kSplitThreads) void split_max_kernel(const T* logits, int64_t row_stride, int vocab,
-                                                                  const int32_t* top_k, int32_t top_k_all,
-                                                                  const float* top_p, float top_p_all,
-                                                                  SplitWs ws) {
-  __shared__ float red[4];
+struct ScaleArgs {
+  const T* penalty;
+  int64_t penalty_stride;
+  int32_t slots;
+  const int32_t* rows;
+  const float* temperature;
+  float* out;
+  int64_t out_stride;
+};
+
+template <typename T, bool SCALE>
+__global__ __launch_bounds__(kSplitThreads) void split_scan_kernel(const T* logits, int64_t row_stride, int vocab,
+                                                                   const int32_t* top_k, int32_t top_k_all,
+                                                                   const float* top_p, float top_p_all,
+                                                                   ScaleArgs<T> sc, SplitWs ws) {
+  __shared__ float red[8];
   const int s = blockIdx.x, b = blockIdx.y, S = gridDim.x, ntiles = split_tiles(vocab);
   if (s == 0 && threadIdx.x == 0) {  // (read by the later launches on this stream)
-    ws.counter[b] = 0;
+    ws.counter[b * kCountStride] = 0;
     ws.fallback[b] = 0;
   }
-  if (row_kind(b, vocab, top_k, top_k_all, top_p, top_p_all) != kWholeRow) return;
+  const int kind = row_kind(b, vocab, top_k, top_k_all, top_p, top_p_all);
+  if (!SCALE && kind == kOtherRow) return;
   const T* p = logits + (int64_t)b * row_stride;
   const bool vec = ((uintptr_t)p % 16) == 0;
-  float mx = -INFINITY;
   const int j0 = s * kSliceTiles, j1 = min(j0 + kSliceTiles, ntiles);
-  SliceLoad<T> sl;
-  sl.issue(p, vocab, vec, j0, j1);
+  const GroupShape& g = ws.g;
+  uint16_t* gm = ws.gmax + (int64_t)b * kGroups + s * g.per_slice;
+  float mn = INFINITY, mx = -INFINITY, gx = -INFINITY;  // the slice's smallest and largest, the group's largest so far
+  auto see = [&](const float (&x)[8], const bool (&ok)[8]) __attribute__((always_inline)) {
 #pragma unroll
-  for (int jj = 0; jj < kSliceTiles; ++jj) {
-    if (j0 + jj >= j1) break;  // (uniform)
-    float x[8];
-    bool ok[8];
-    sl.get(p, vocab, vec, j0 + jj, jj, x, ok);
+    for (int k = 0; k < 8; ++k) {
+      gx = ok[k] ? fmaxf(gx, x[k]) : gx;
+      mn = ok[k] ? fminf(mn, x[k]) : mn;
+    }
+  };
+  auto group_end = [&](int jj) __attribute__((always_inline)) {
+    if ((kind == kTopKRow || kind == kTopPRow) && ((jj + 1) & ((1 << g.tg) - 1)) == 0) {  // (uniform)
+      mx = fmaxf(mx, gx);
+      for (int o = 1; o < (1 << g.gl); o <<= 1) gx = fmaxf(gx, __shfl_xor(gx, o, kWave));
+      const int at = ((jj >> g.tg) * kSplitThreads + (int)threadIdx.x) >> g.gl;
+      if ((threadIdx.x & ((1 << g.gl) - 1)) == 0) gm[at] = (uint16_t)(fkey(gx) >> 16);  // (no number in it: as -inf)
+      gx = -INFINITY;
+    }
+  };
+  if constexpr (!SCALE) {
+    SliceLoad<T> sl;
+    sl.issue(p, vocab, vec, j0, j1);
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (ok[k]) mx = fmaxf(mx, x[k]);
+    for (int jj = 0; jj < kSliceTiles; ++jj) {
+      if (j0 + jj < j1) {
+        float x[8];
+        bool ok[8];
+        sl.get(p, vocab, vec, j0 + jj, jj, x, ok);
+        see(x, ok);
+      }
+      group_end(jj);
+    }
+  } else {
+    // a tile at a time, the next one's vectors on their way: the divisions are long, and eight tiles
+    // unrolled with their logits and penalties in registers spilled (128 x 151,936 fp16: 50 us; four at
+    // once 38, two ahead 36, one ahead 32)
+    constexpr int R = 8 * sizeof(T) / 16;
+    float* o = sc.out + (int64_t)b * sc.out_stride;
+    const float temp = sc.temperature ? sc.temperature[b] : 1.f;
+    const int pr = sc.penalty ? sc.rows[b] : 0;
+    const bool bad = sc.penalty && (pr < 0 || pr >= sc.slots);  // no such penalty row: the row reads as NaN
+    const T* pen = sc.penalty ? sc.penalty + (int64_t)(bad ? 0 : pr) * sc.penalty_stride : p;
+    const bool has_pen = sc.penalty != nullptr, whole = vec && ((uintptr_t)pen % 16) == 0 && vocab >= 8;
+    const int last = (vocab - 8) / 8 * 8;
+    uint4 nx[R], np[R];
+    auto issue = [&](int j) __attribute__((always_inline)) {  // (clamped: whole vectors inside the row)
+      const int base = min(j * kSplitTile + 8 * (int)threadIdx.x, last);
+#pragma unroll
+      for (int v = 0; v < R; ++v) {
+        nx[v] = *reinterpret_cast<const uint4*>(p + base + v * (16 / sizeof(T)));
+        np[v] = *reinterpret_cast<const uint4*>(pen + base + v * (16 / sizeof(T)));
+      }
+    };
+    if (whole) issue(j0);
+#pragma unroll 1
+    for (int jj = 0; jj < kSliceTiles; ++jj) {
+      if (j0 + jj < j1) {
+        const int base = (j0 + jj) * kSplitTile + 8 * (int)threadIdx.x;
+        T xs[8], ps[8];
+        bool ok[8];
+        if (whole) {
+          __builtin_memcpy(xs, nx, 8 * sizeof(T));
+          __builtin_memcpy(ps, np, 8 * sizeof(T));
+          issue(min(j0 + jj + 1, j1 - 1));
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          ok[k] = base + k < vocab;
+          if (ok[k] && !(whole && base + 8 <= vocab)) {
+            xs[k] = p[base + k];
+            ps[k] = pen[base + k];
+          }
+        }
+        float x[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) x[k] = bad ? __builtin_nanf("") : scale_logit<T>(xs[k], ps[k], has_pen, temp);
+        if (base + 8 <= vocab) {
+          *reinterpret_cast<float4*>(o + base) = make_float4(x[0], x[1], x[2], x[3]);
+          *reinterpret_cast<float4*>(o + base + 4) = make_float4(x[4], x[5], x[6], x[7]);
+        } else {
+#pragma unroll
+          for (int k = 0; k < 8; ++k)
+            if (ok[k]) o[base + k] = x[k];
+        }
+        see(x, ok);
+      }
+      group_end(jj);
+    }
   }
-  mx = block_max256(mx, red);
-  if (threadIdx.x == 0) ws.smax[(int64_t)b * S + s] = mx;
+  if (kind == kWholeRow || kind == kTopPRow) {
+    const float2 r = block_range256(fmaxf(mx, gx), mn, red);
+    if (threadIdx.x == 0) {
+      ws.smax[(int64_t)b * S + s] = r.x;
+      ws.smin[(int64_t)b * S + s] = r.y;
+    }
+  }
 }
 
+// Inclusive sum over the threads below and at this one (and, in `all`, over all of them).
+__device__ __forceinline__ uint64_t block_scan256(uint64_t v, uint64_t* red, uint64_t& all) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint64_t y = __shfl_up(v, o, kWave);
+    if (lane >= o) v += y;
+  }
+  __syncthreads();
+  if (lane == 63) red[wv] = v;
+  __syncthreads();
+  for (int i = 0; i < wv; ++i) v += red[i];
+  all = red[0] + red[1] + red[2] + red[3];
+  return v;
+}
+
+// Each of n <= 256 entries against every one, by the workgroup: 256 / n (a power of two) neighbouring
+// threads share an entry and call f(i) for their part of i = 0 .. n - 1; entry() is the thread's.
+struct Pairs {
+  int n, shift;
+  __device__ __forceinline__ Pairs(int n_) : n(n_), shift(n_ <= 32 ? 3 : n_ <= 64 ? 2 : n_ <= 128 ? 1 : 0) {}
+  __device__ __forceinline__ int entry() const { return (int)threadIdx.x >> shift; }
+  __device__ __forceinline__ bool first() const { return (threadIdx.x & ((1 << shift) - 1)) == 0; }
+  // The mass of the entries with key >= lo and index < lim.  The entries are read four at a time before
+  // any is used: one by one, each LDS read's latency is waited out.
+  __device__ __forceinline__ uint64_t mass(const uint64_t* cand, const uint64_t* mass, uint32_t lo, uint32_t lim) const {
+    const int parts = 1 << shift, sub = threadIdx.x & (parts - 1);
+    uint64_t f = 0;
+#pragma unroll 1
+    for (int i0 = sub; i0 < n; i0 += 4 * parts) {
+      uint64_t c[4], m[4];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const int i = min(i0 + x * parts, n - 1);
+        c[x] = cand[i];
+        m[x] = mass[i];
+      }
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+        f += i0 + x * parts < n && (uint32_t)c[x] >= lo && (uint32_t)(c[x] >> 32) < lim ? m[x] : 0;
+    }
+#pragma unroll 1
+    for (int o = 1; o < parts; o <<= 1) f += __shfl_xor(f, o, kWave);
+    return f;
+  }
+};
+// A wave's largest (sum) into LDS.  Reduced in registers first: from an atomic whose lanes hold different
+// values for one address the compiler makes a loop over the lanes, about 1 us.
+__device__ __forceinline__ void wave_to_lds_max(uint32_t* p, uint32_t v) {
+  v = wave_max_u32(v);
+  if ((threadIdx.x & 63) == 0) atomicMax(p, v);
+}
+__device__ __forceinline__ void wave_to_lds_sum(uint64_t* p, uint64_t v) {
+  v = wave_sum_u64(v);
+  if ((threadIdx.x & 63) == 0) atomicAdd((unsigned long long*)p, (unsigned long long)v);
+}
+struct TokenAt {
+  uint64_t before;  // the kept mass of the tiles before the token's
+  int tile;
+};
+// The token of a whole or top-p row from its tiles' kept masses (in s_tile, for every thread): the
+// tile holding the target, then each thread's kept mass in it, an exclusive scan in thread (=
+// vocabulary) order, and the owner walks its 8 logits.  Kept: key >= thr.
 template <typename T>
-__global__ __launch_bounds__(kSplitThreads) void split_sample_kernel(const T* logits, int64_t row_stride, int vocab,
-                                                                     const int32_t* top_k, int32_t top_k_all,
-                                                                     const float* top_p, float top_p_all,
-                                                                     const float* uniform, int32_t* out, SplitWs ws) {
-  __shared__ float redf[4];
-  __shared__ uint64_t redu[4];
-  __shared__ uint64_t s_tile[kMaxSplitTiles];
-  __shared__ int s_last;
-  const int s = blockIdx.x, b = blockIdx.y, S = gridDim.x, ntiles = split_tiles(vocab);
-  if (row_kind(b, vocab, top_k, top_k_all, top_p, top_p_all) != kWholeRow) return;
-  const T* p = logits + (int64_t)b * row_stride;
-  const bool vec = ((uintptr_t)p % 16) == 0;
-  // this slice's logits (requested first), and the row's largest logit from the slices'
-  // (written by the previous launch)
-  const int j0 = s * kSliceTiles, j1 = min(j0 + kSliceTiles, ntiles);
-  SliceLoad<T> sl;
-  sl.issue(p, vocab, vec, j0, j1);
-  float mx = -INFINITY;
-  for (int i = threadIdx.x; i < S; i += kSplitThreads) mx = fmaxf(mx, ws.smax[(int64_t)b * S + i]);
-  mx = block_max256(mx, redf);
-  // this slice's tile masses, written through to device scope
-  uint64_t* tm = ws.tmass + (int64_t)b * ntiles;
-#pragma unroll
-  for (int jj = 0; jj < kSliceTiles; ++jj) {
-    if (j0 + jj >= j1) break;  // (uniform)
-    float x[8];
-    bool ok[8];
-    sl.get(p, vocab, vec, j0 + jj, jj, x, ok);
-    uint64_t m = 0;
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (ok[k]) m += fmass(x[k], mx);
-    m = block_sum256(m, redu);
-    if (threadIdx.x == 0) __hip_atomic_store(tm + j0 + jj, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  // arrival: the last slice of the row to finish samples it
-  if (threadIdx.x == 0) {
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // this slice's tile masses are complete (device-visible)
-    const int old = atomicAdd(&ws.counter[b], 1);
-    s_last = old == S - 1;
-  }
-  __syncthreads();
-  if (!s_last) return;
-  for (int j = threadIdx.x; j < ntiles; j += kSplitThreads)
-    s_tile[j] = __hip_atomic_load(tm + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __syncthreads();
-  uint64_t ms = 0;
-  for (int j = 0; j < ntiles; ++j) ms += s_tile[j];  // (every thread: uniform)
-  if (ms == 0) {
-    if (threadIdx.x == 0) out[b] = -1;  // (no token carries mass: an all-NaN row)
+__device__ __forceinline__ void pick_token(const T* p, int vocab, bool vec, float mx, uint32_t thr, const uint64_t* s_tile,
+                                           int ntiles, float u, int32_t* out, uint64_t* redu, TokenAt* at) {
+  // thread t: the tiles [per t, per (t + 1))
+  const int per = (ntiles + kSplitThreads - 1) / kSplitThreads, q0 = per * (int)threadIdx.x;
+  uint64_t own = 0, ms;
+  for (int j = q0; j < min(q0 + per, ntiles); ++j) own += s_tile[j];
+  const uint64_t upto = block_scan256(own, redu, ms);
+  if (ms == 0) {  // (uniform)
+    if (threadIdx.x == 0) *out = -1;  // (no token carries mass: an all-NaN row)
     return;
   }
-  const double uu = fminf(fmaxf(uniform[b], 0.f), 1.f);
+  const double uu = fminf(fmaxf(u, 0.f), 1.f);
   uint64_t target = (uint64_t)(uu * (double)ms);
   if (target >= ms) target = ms - 1;
-  int tt = 0;
-  uint64_t before = 0;
-  while (tt < ntiles - 1 && before + s_tile[tt] <= target) before += s_tile[tt++];
-  // inside tile tt: each thread's mass, exclusive scan in thread (= vocabulary) order, then the
-  // owner walks its 8 logits
+  if (upto > target && upto - own <= target) {
+    uint64_t before = upto - own;
+    int tt = q0;
+    while (before + s_tile[tt] <= target) before += s_tile[tt++];
+    at->before = before;
+    at->tile = tt;
+  }
+  __syncthreads();
+  const int tt = at->tile;
+  const uint64_t before = at->before;
   float x[8];
   bool ok[8];
   load8(p, vocab, vec, tt, x, ok);
   uint64_t mine = 0;
 #pragma unroll
-  for (int k = 0; k < 8; ++k)
+  for (int k = 0; k < 8; ++k) {
+    ok[k] = ok[k] && fkey(x[k]) >= thr;
     if (ok[k]) mine += fmass(x[k], mx);
+  }
   uint64_t inc = mine;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
 #pragma unroll
@@ -567,488 +772,751 @@ __global__ __launch_bounds__(kSplitThreads) void split_sample_kernel(const T* lo
         if (run > target) found = tt * kSplitTile + 8 * (int)threadIdx.x + k;
       }
     }
-    out[b] = found;
+    *out = found;
   }
 }
-
-__device__ __forceinline__ int block_sum_i256(int v, int* red) {
-  v = wave_sum_i32(v);
+// Arrival of a slice whose results are written through to device scope: true in the workgroup that
+// finishes the row's last slice.
+__device__ __forceinline__ bool slice_arrive(int32_t* counter, int S, int* s_last) {
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // this thread's results are complete (device-visible)
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  if (threadIdx.x == 0) *s_last = atomicAdd(counter, 1) == S - 1;
   __syncthreads();
-  return red[0] + red[1] + red[2] + red[3];
+  return *s_last;
 }
-__device__ __forceinline__ uint32_t block_max_u256(uint32_t v, uint32_t* red) {
-  v = wave_max_u32(v);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return max(max(red[0], red[1]), max(red[2], red[3]));
+__device__ __forceinline__ void st_dev_u64(uint64_t* p, uint64_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// The float whose fkey is k (k != 0).
-__device__ __forceinline__ float key_float(uint32_t k) {
-  return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
+template <typename V>
+__device__ __forceinline__ V ld_dev(const V* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// ---- Top-k rows (0 < k <= kTopKMax, any top-p) over many workgroups per row, one launch.
-// Each (slice, row) workgroup holds its slice's keys in registers and bisects for a key t_s
-// with k <= #{key >= t_s} <= kCandCap (or takes every non-NaN logit when there are at most
-// kCandCap of them), and hands those logits over as candidates.  No slice can hold k logits
-// above the row's k-th largest key T*, so t_s <= T* and every logit with key >= T* is a
-// candidate: over the candidates, the largest T with #{key >= T} >= k is T* itself.  The last
-// slice of the row to finish then runs sample_row's rule on the candidates alone: T*, the top-p
-// threshold (the largest T with mass{key >= T} >= need, as its mass-weighted selection finds),
-// and the inverse CDF in vocabulary order, with the same integer masses, so the token is the
-// same.  One wave does that merge with shuffle reductions (a search takes up to 32 steps, and
-// workgroup barriers at every step made it the kernel's critical path); slices hand over between
-// k and 2k logits to keep the candidates within its registers.  Rows it cannot finish this way
-// (a slice's ties beyond kCandCap, more candidates than the wave holds, fewer than k finite
-// logits, a kept set beyond kKeptCap) are handed back to sample_kernel through `fallback`.
-constexpr int kKeptCap = 1024;
-constexpr int kRadixBins = 2048;  // the largest digit (11 bits) of the merge's radix selection
+// A row's largest and smallest logit from its slices' (written by the scan's launch).
+__device__ __forceinline__ float2 row_range(const SplitWs& ws, int b, int S, float* red) {
+  float mx = -INFINITY, mn = INFINITY;
+  for (int i = threadIdx.x; i < S; i += kSplitThreads) {
+    mx = fmaxf(mx, ws.smax[(int64_t)b * S + i]);
+    mn = fminf(mn, ws.smin[(int64_t)b * S + i]);
+  }
+  return block_range256(mx, mn, red);
+}
 
 template <typename T>
-__global__ __launch_bounds__(kSplitThreads) __attribute__((amdgpu_waves_per_eu(5))) void split_topk_kernel(
-    const T* logits, int64_t row_stride, int vocab,
-                                                                   const int32_t* top_k, int32_t top_k_all,
-                                                                   const float* top_p, float top_p_all,
-                                                                   const float* uniform, int32_t* out, SplitWs ws) {
-  __shared__ __align__(16) int s_h[kRadixBins];
-  __shared__ int s_wsum[kSplitThreads / kWave];
-  __shared__ int s_n, s_dig, s_above, s_cnt, s_total;
-  const int s = blockIdx.x, b = blockIdx.y, S = gridDim.x, ntiles = split_tiles(vocab);
-  if (row_kind(b, vocab, top_k, top_k_all, top_p, top_p_all) != kTopKRow) return;
-  const int k = top_k ? top_k[b] : top_k_all;
-  const T* p = logits + (int64_t)b * row_stride;
-  const bool vec = ((uintptr_t)p % 16) == 0;
-  const int t = threadIdx.x, lane = t & (kWave - 1), wv = t / kWave;
-  // the slice's keys (0: past the row's end, or NaN)
-  const int j0 = s * kSliceTiles, j1 = min(j0 + kSliceTiles, ntiles);
-  SliceLoad<T> sl;
-  sl.issue(p, vocab, vec, j0, j1);
-  // The slice's keys, cut to their 16 most significant bits (still in the logits' order, ties
-  // merged) and packed two to a register: key i in the half i & 1 of kp[i / 2] (0: past the
-  // row's end, or NaN).  Held as 16 bits, every slice's workgroup of the batch is resident at
-  // once; a candidate's full key is recomputed from its logit when it is handed over.
-  uint32_t kp[kSliceTiles * 4];
+__device__ __forceinline__ void whole_slice(const T* p, int vocab, bool vec, const SliceLoad<T>& sl, int s, int b, int S,
+                                            const float* uniform, int32_t* out, const SplitWs& ws, uint64_t* s_tile,
+                                            float* redf, uint64_t (*redu)[4], int* s_last, TokenAt* at) {
+  const TileSums sums{redu};
+  const int ntiles = split_tiles(vocab), j0 = s * kSliceTiles, j1 = min(j0 + kSliceTiles, ntiles);
+  const float mx = row_range(ws, b, S, redf).x;
+  // this slice's tile masses, written through to device scope
+  uint64_t* tm = ws.tmass + (int64_t)b * ntiles;
 #pragma unroll
   for (int jj = 0; jj < kSliceTiles; ++jj) {
+    if (j0 + jj >= j1) break;  // (uniform)
     float x[8];
     bool ok[8];
-    if (j0 + jj < j1) {
-      sl.get(p, vocab, vec, j0 + jj, jj, x, ok);
-    } else {
+    sl.get(p, vocab, vec, j0 + jj, jj, x, ok);
+    uint64_t m = 0;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) ok[e] = false;
-    }
-#pragma unroll
-    for (int e = 0; e < 8; e += 2)
-      kp[jj * 4 + e / 2] = (ok[e] ? fkey(x[e]) >> 16 : 0u) | (ok[e + 1] ? fkey(x[e + 1]) & 0xFFFF0000u : 0u);
+    for (int k = 0; k < 8; ++k)
+      if (ok[k]) m += fmass(x[k], mx);
+    sums.add(jj, m);
   }
-  auto key16 = [&](int i) __attribute__((always_inline)) -> uint32_t {
-    return (i & 1) ? kp[i >> 1] >> 16 : kp[i >> 1] & 0xFFFFu;
-  };
-  // The threshold t_s: the start of the range of 16-bit keys (a digit of 11 bits, then one of 5)
-  // that holds the slice's k-th largest, refined until at most 2k keys lie at or above it: each
-  // level histograms, in LDS, the keys inside the range chosen so far, and one scan of the
-  // histogram finds the digit (where a bisection counted every key once per halving, with a
-  // workgroup reduction each time).  Keys at or above t_s include every logit at or above the
-  // slice's k-th largest, so every logit at or above the row's k-th largest is a candidate.
-  uint32_t ts = 1u, prefix = 0u, himask = 0u;
-  int above = 0, cnt = 0;
-#pragma unroll 1
-  for (int level = 0; level < 2; ++level) {
-    const int shift = level == 0 ? 5 : 0;
-    const uint32_t nb = level == 0 ? 2048u : 32u;
-#pragma unroll
-    for (int i = 0; i < kRadixBins / kSplitThreads / 4; ++i)
-      reinterpret_cast<int4*>(s_h)[t * (kRadixBins / kSplitThreads / 4) + i] = make_int4(0, 0, 0, 0);
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kSliceTiles * 8; ++i) {
-      const uint32_t kk = key16(i);
-      if (kk != 0u && (kk & himask) == prefix) atomicAdd(&s_h[(kk >> shift) & (nb - 1u)], 1);
-    }
-    __syncthreads();
-    // thread t owns bins [8t, 8t + 8); the count in its bins and in every bin above them
-    int bins[8];
-    {
-      const int4 a = reinterpret_cast<const int4*>(s_h)[2 * t], c = reinterpret_cast<const int4*>(s_h)[2 * t + 1];
-      bins[0] = a.x; bins[1] = a.y; bins[2] = a.z; bins[3] = a.w;
-      bins[4] = c.x; bins[5] = c.y; bins[6] = c.z; bins[7] = c.w;
-    }
-    int own = 0;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) own += bins[e];
-    int incl = own;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const int v = __shfl_down(incl, o, kWave);
-      incl += lane + o < kWave ? v : 0;
-    }
-    if (lane == 0) s_wsum[wv] = incl;
-    __syncthreads();
-    for (int w2 = wv + 1; w2 < kSplitThreads / kWave; ++w2) incl += s_wsum[w2];
-    if (t == 0) s_total = incl;  // (thread 0's: every key in the range)
-    if (above + incl >= k && above + incl - own < k) {  // the thread whose bins hold the k-th largest
-      int acc = above + incl - own;
-#pragma unroll
-      for (int e = 7; e >= 0; --e) {
-        if (acc + bins[e] >= k) {
-          s_dig = 8 * t + e;
-          s_above = acc;
-          s_cnt = acc + bins[e];
-          break;
-        }
-        acc += bins[e];
-      }
-    }
-    __syncthreads();
-    if (level == 0 && s_total < k) {  // (uniform) fewer than k finite keys: all of them
-      ts = 1u;
-      cnt = s_total;
-      break;
-    }
-    cnt = s_cnt;
-    prefix |= (uint32_t)s_dig << shift;
-    himask |= (nb - 1u) << shift;
-    above = s_above;
-    ts = prefix;
-    if (cnt <= 2 * k) break;  // (uniform) at most 2k keys at or above ts
-    __syncthreads();  // (s_dig, s_above, s_cnt read by every thread before the next level writes them)
-  }
-  const bool bad = cnt > kCandCap;  // (ties at the threshold beyond the slice's capacity)
-  if (t == 0) s_n = 0;
+  sums.store(tm + j0, j1 - j0);
+  if (!slice_arrive(&ws.counter[b * kCountStride], S, s_last)) return;
+  for (int j = threadIdx.x; j < ntiles; j += kSplitThreads) s_tile[j] = ld_dev(tm + j);
   __syncthreads();
-  uint64_t* cand = ws.cand + ((int64_t)b * S + s) * kCandCap;
-  if (!bad) {
-#pragma unroll
-    for (int i = 0; i < kSliceTiles * 8; ++i) {
-      if (key16(i) >= ts) {
-        const int pos = atomicAdd(&s_n, 1);
-        const int idx = (j0 + i / 8) * kSplitTile + 8 * t + (i % 8);
-        cand[pos] = ((uint64_t)(uint32_t)idx << 32) | fkey(to_f32(p[idx]));
-      }
-    }
-  }
-  __syncthreads();
-  if (t == 0) ws.ncand[(int64_t)b * S + s] = bad ? -1 : s_n;
+  pick_token(p, vocab, vec, mx, 0u, s_tile, ntiles, uniform[b], out + b, redu[0], at);
 }
 
-// The merge of a top-k row's candidates (the launch after split_topk_kernel), one wave per row:
-// the row's k-th largest key T* over its slices' candidates, the top-p threshold over the top-k
-// set, and the inverse CDF in vocabulary order, with sample_row's integer masses, so the token is
-// the same.  A launch of its own rather than the last slice to finish: the slice kernel then
-// holds only its slice's keys and a chip's worth of its workgroups are resident at once.
-__global__ __launch_bounds__(kWave) void split_topk_merge_kernel(int vocab, const int32_t* top_k, int32_t top_k_all,
-                                                                 const float* top_p, float top_p_all,
-                                                                 const float* uniform, int32_t* out, SplitWs ws) {
-  __shared__ int s_off[kMaxSplitTiles / kSliceTiles + 1];
-  __shared__ int s_sidx[kKeptCap];
-  __shared__ uint64_t s_smass[kKeptCap];
-  __shared__ uint32_t s_skey[kKeptCap];
-  __shared__ __align__(16) int s_hist[kRadixBins];  // (16-byte vector accesses)
-  const int b = blockIdx.x, S = split_slices(vocab);
-  if (row_kind(b, vocab, top_k, top_k_all, top_p, top_p_all) != kTopKRow) return;
-  const int k = top_k ? top_k[b] : top_k_all;
-  const int lane = threadIdx.x;
-  if (lane == 0) ws.fallback[b] = 0;
-  // the slices' candidate counts, 64 at a time, and their running offsets
-  int off = 0, anybad = 0;
-  for (int i0 = 0; i0 < S; i0 += kWave) {
-    const int i = i0 + lane;
-    const int c = i < S ? ws.ncand[(int64_t)b * S + i] : 0;
-    anybad |= c < 0 ? 1 : 0;
-    const int cc = c < 0 ? 0 : c;
-    int incl = cc;  // inclusive prefix over the lanes below
+// ---- Top-p rows.  The row's masses are binned by distance from its largest logit (kPBins bins over
+// the range that carries mass: a monotone function of the logit, so the bins are in the logits'
+// order); the bin where the mass from the top reaches the target holds the threshold, and the workgroup
+// that finishes the row's last slice finds it.  In the next launch logits in the bins above are kept,
+// those in it are candidates (a few hundred of 151,936), and the last slice's workgroup selects the
+// exact threshold among them.  That launch reads only the groups whose largest logit reaches the bin.
+struct PBins {
+  float mx, scale;
+  __device__ __forceinline__ PBins(float mx_, float scale_) : mx(mx_), scale(scale_) {}
+  __device__ __forceinline__ PBins(float2 range)
+      : mx(range.x), scale((float)kPBins / fmaxf(fminf(range.x - range.y, 23.f), 1e-20f)) {}
+  __device__ __forceinline__ int of(float x) const { return min((int)((mx - x) * scale), kPBins - 1); }
+};
+
+template <typename T>
+__device__ __forceinline__ void topp_hist(const T* p, int vocab, bool vec, const SliceLoad<T>& sl, int s, int b, int S,
+                                          float pp, int32_t* out, const SplitWs& ws, uint64_t* s_hist, float* redf,
+                                          uint64_t* redu, int* s_last) {
+  const int ntiles = split_tiles(vocab), j0 = s * kSliceTiles, j1 = min(j0 + kSliceTiles, ntiles), t = threadIdx.x;
+  for (int i = t; i < kPBins; i += kSplitThreads) s_hist[i] = 0;
+  const PBins bins(row_range(ws, b, S, redf));  // (synchronises)
 #pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const int v = __shfl_up(incl, o, kWave);
-      incl += lane >= o ? v : 0;
+  for (int jj = 0; jj < kSliceTiles; ++jj) {
+    if (j0 + jj >= j1) break;  // (uniform)
+    float x[8];
+    bool ok[8];
+    sl.get(p, vocab, vec, j0 + jj, jj, x, ok);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const uint64_t m = ok[k] ? fmass(x[k], bins.mx) : 0;
+      if (m) atomicAdd((unsigned long long*)&s_hist[bins.of(x[k])], (unsigned long long)m);
     }
-    if (i < S) s_off[i] = off + incl - cc;
-    off += __shfl(incl, kWave - 1, kWave);
   }
-  if (lane == 0) s_off[S] = off;
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the offsets are in LDS for every lane
-  __builtin_amdgcn_wave_barrier();
-  const int n = off;
-  if (wave_max_u32((uint32_t)anybad) || n == 0 || n > kWave * kMergeRegs) {
-    if (lane == 0) ws.fallback[b] = 1;
-    return;
+  __syncthreads();
+  uint64_t* h = ws.hist + (int64_t)b * S * kPBins;
+  for (int i = t; i < kPBins; i += kSplitThreads) st_dev_u64(h + (int64_t)s * kPBins + i, s_hist[i]);
+  if (!slice_arrive(&ws.counter[b * kCountStride], S, s_last)) return;
+  // ---- the bin that holds the threshold; thread t: bins 2t, 2t + 1
+  static_assert(kPBins == 2 * kSplitThreads, "two bins a thread");
+  uint64_t h0 = 0, h1 = 0;
+#pragma unroll 8
+  for (int i = 0; i < S; ++i) {
+    h0 += ld_dev(h + (int64_t)i * kPBins + 2 * t);
+    h1 += ld_dev(h + (int64_t)i * kPBins + 2 * t + 1);
   }
-  auto wsum_i = [](int v) __attribute__((always_inline)) { return wave_sum_i32(v); };
-  auto wmax_u = [](uint32_t v) __attribute__((always_inline)) { return wave_max_u32(v); };
-  uint32_t ck[kMergeRegs];
-  int cidx[kMergeRegs];
-  // the slice holding candidate lane + 64 r and its first candidate's offset: the slices' offsets
-  // come to every lane through scalar registers (one readlane each), in slice order
-  int csl[kMergeRegs], cso[kMergeRegs];
+  uint64_t mk;
+  const uint64_t incl = block_scan256(h0 + h1, redu, mk), excl = incl - h0 - h1;
+  const double needd = ceil((double)fmaxf(pp, 0.f) * (double)mk);
+  uint64_t need = needd < 1.0 ? 1 : (uint64_t)needd;
+  if (need > mk) need = mk;
+  if (t == 0) ws.counter[b * kCountStride] = 0;  // (for the next launch's arrivals)
+  if (mk == 0) {  // (no token carries mass)
+    if (t == 0) {
+      ws.bin[b].bin = -1;
+      out[b] = -1;
+    }
+  } else if (incl >= need && excl < need) {
+    const bool lo = excl + h0 >= need;
+    ws.bin[b] = ToppBin{lo ? excl : excl + h0, need, bins.mx, bins.scale, lo ? 2 * t : 2 * t + 1};
+  }
+}
+
+struct ToppLds {
+  uint64_t cand[kPCandMax];
+  uint64_t mass[kPCandMax];
+  uint64_t hist[kSplitThreads];
+  uint64_t redu[4], tsum[kSliceTiles][4];
+  uint64_t above;
+  TokenAt at;
+  int off[kMaxSplitTiles / kSliceTiles + 1];
+  uint32_t diff, thr;
+  int bin, n, last;
+};
+
+template <typename T>
+__device__ __forceinline__ void topp_finish(const T* p, int vocab, int s, int b, int S, const float* uniform, int32_t* out,
+                                            const SplitWs& ws, ToppLds& L, uint64_t* s_tile) {
+  const int t = threadIdx.x;
+  const int ntiles = split_tiles(vocab), j0 = s * kSliceTiles, j1 = min(j0 + kSliceTiles, ntiles);
+  const bool vec = ((uintptr_t)p % 16) == 0;
+  const GroupShape& g = ws.g;
+  const uint16_t* gm = ws.gmax + (int64_t)b * kGroups + s * g.per_slice;
+  const ToppBin tb = ws.bin[b];
+  const int cb = (int)tb.bin;
+  const uint64_t above = tb.above, need = tb.need;
+  if (cb < 0) return;  // (uniform; the token is written)
+  if (t == 0) L.n = 0, L.diff = 0;
+  const PBins bins(tb.mx, tb.scale);
+  __syncthreads();
+  // ---- this slice: its tiles' mass above the bin, and its candidates, written through to device scope
+  const TileSums sums{L.tsum};
+  uint64_t* tm = ws.tmass + (int64_t)b * ntiles;
+  uint64_t* pc = ws.cand + ((int64_t)b * S + s) * kCandCap;
+  // a group's largest logit is at most the float of its key's upper half and all lower bits set; threads
+  // of groups that do not reach the bin load the row's first vector instead
+  constexpr int R = 8 * sizeof(T) / 16;
+  const bool vecs = vec && vocab >= 8;
+  bool act[kSliceTiles];
+  uint4 raw[kSliceTiles][R];
+  {
+    uint32_t gk[kSliceTiles];
 #pragma unroll
-  for (int r = 0; r < kMergeRegs; ++r) csl[r] = cso[r] = 0;
-  for (int i0 = 0; i0 < S; i0 += kWave) {
-    const int offv = i0 + lane < S ? s_off[i0 + lane] : 0;
-    const int nin = min(kWave, S - i0);
-    for (int ii = 0; ii < nin; ++ii) {
-      const int oi = __builtin_amdgcn_readlane(offv, ii);
+    for (int jj = 0; jj < kSliceTiles; ++jj) gk[jj] = gm[((jj >> g.tg) * kSplitThreads + t) >> g.gl];
 #pragma unroll
-      for (int r = 0; r < kMergeRegs; ++r) {
-        if (oi <= min(lane + kWave * r, n - 1)) {
-          csl[r] = i0 + ii;
-          cso[r] = oi;
-        }
+    for (int jj = 0; jj < kSliceTiles; ++jj) {
+      const int base = (j0 + jj) * kSplitTile + 8 * t;
+      act[jj] = base < vocab && bins.of(key_float(gk[jj] << 16 | 0xFFFFu)) <= cb;
+#pragma unroll
+      for (int v = 0; v < R; ++v)
+        if (vecs) raw[jj][v] = *reinterpret_cast<const uint4*>(p + (act[jj] && base + 8 <= vocab ? base : 0) + v * (16 / sizeof(T)));
+    }
+  }
+  uint64_t in = 0;  // this thread's logits in the bin
+#pragma unroll
+  for (int jj = 0; jj < kSliceTiles; ++jj) {
+    if (j0 + jj >= j1) break;  // (uniform)
+    uint64_t m = 0;
+    if (act[jj]) {
+      const int base = (j0 + jj) * kSplitTile + 8 * t;
+      T e[8];
+      __builtin_memcpy(e, raw[jj], sizeof(e));
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const bool ok = base + k < vocab;
+        if (ok && !(vecs && base + 8 <= vocab)) e[k] = p[base + k];
+        const float x = ok ? to_f32(e[k]) : -INFINITY;
+        const uint64_t f = fmass(x, bins.mx);
+        const int ib = f ? bins.of(x) : kPBins;
+        m += ib < cb ? f : 0;
+        in |= (uint64_t)(ib == cb) << (8 * jj + k);
       }
     }
+    sums.add(jj, m);
   }
-#pragma unroll
-  for (int r = 0; r < kMergeRegs; ++r) {  // unconditional loads of clamped candidates
-    const int ci = min(lane + kWave * r, n - 1);
-    const uint64_t v = ws.cand[((int64_t)b * S + csl[r]) * kCandCap + (ci - cso[r])];
-    const bool real = lane + kWave * r < n;
-    ck[r] = real ? (uint32_t)v : 0u;
-    cidx[r] = (int)(v >> 32);
+  for (; in; in &= in - 1) {  // (a loop over those it has, not 64 copies of the code)
+    const int pos = atomicAdd(&L.n, 1);
+    const int i = __builtin_ctzll(in), idx = (j0 + (i >> 3)) * kSplitTile + 8 * t + (i & 7);
+    if (pos < kCandCap) st_dev_u64(pc + pos, ((uint64_t)(uint32_t)idx << 32) | fkey(to_f32(p[idx])));
   }
-  uint32_t mxk = 0;
-  int nfin = 0;
-#pragma unroll
-  for (int r = 0; r < kMergeRegs; ++r) {
-    mxk = max(mxk, ck[r]);
-    nfin += ck[r] != 0u ? 1 : 0;
-  }
-  mxk = wmax_u(mxk);
-  if (wsum_i(nfin) < k) {  // K would take NaN logits: not a candidate case
-    if (lane == 0) ws.fallback[b] = 1;
+  sums.store(tm + j0, j1 - j0);
+  if (t == 0) __hip_atomic_store(&ws.ncand[(int64_t)b * S + s], L.n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (!slice_arrive(&ws.counter[b * kCountStride], S, &L.last)) return;
+  // ---- the row's last slice: all candidates
+  static_assert(kMaxSplitTiles / kSliceTiles <= kSplitThreads, "a slice a thread");
+  const int nc = t < S ? ld_dev(&ws.ncand[(int64_t)b * S + t]) : 0;
+  uint64_t n64;
+  const uint64_t upto = block_scan256((uint64_t)nc | ((uint64_t)(nc > kCandCap ? 1 : 0) << 40), L.redu, n64);
+  const int n = (int)(uint32_t)n64;
+  if ((n64 >> 40) || n > kPCandMax) {  // (uniform)
+    if (t == 0) ws.fallback[b] = 1;
     return;
   }
-  // The k-th largest key T* (ties kept): the largest T with #{key >= T} >= k, by radix
-  // selection over the bits in which the candidates' keys differ (the others are those of the
-  // largest key, and so of T*), in digits of up to 11 bits from the most significant: a
-  // histogram of the candidates that agree with the digits chosen so far, then the digit at
-  // which the count from the top reaches k.  One to three histograms replace the up to 32
-  // halvings of a bisection, each of which was a wave-wide reduction in turn.
-  uint32_t diff = 0;  // the bits in which some finite candidate differs from the largest
-#pragma unroll
-  for (int r = 0; r < kMergeRegs; ++r) diff |= ck[r] != 0u ? ck[r] ^ mxk : 0u;
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) diff |= (uint32_t)__shfl_xor((int)diff, o, kWave);
-  diff = (uint32_t)__builtin_amdgcn_readfirstlane((int)diff);
-  uint32_t thr = mxk;
-  if (diff != 0u) {
-    const int top = 32 - __builtin_clz(diff), bot = __builtin_ctz(diff);  // bits [bot, top) vary
-    thr = mxk & ~((top == 32 ? ~0u : ((1u << top) - 1u)) & ~((1u << bot) - 1u));
-    int above = 0;  // candidates above the digits chosen so far
-    for (int hi = top; hi > bot;) {
-      const int width = min(hi - bot, 11), shift = hi - width;
-      const uint32_t nb = 1u << width;
-      const uint32_t himask = hi == 32 ? 0u : ~0u << hi;  // the bits above this digit
+  if (t < S) L.off[t] = (int)(uint32_t)upto - nc;
+  if (t == 0) L.off[S] = n;
+  for (int j = t; j < ntiles; j += kSplitThreads) s_tile[j] = ld_dev(tm + j);
+  __syncthreads();
+  uint32_t diff = 0, key0 = 0;
+  for (int i = t; i < n; i += kSplitThreads) {
+    int lo = 0, hi = S;  // the slice whose candidates include the i-th: off[lo] <= i < off[lo + 1]
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (L.off[mid] <= i) lo = mid; else hi = mid;
+    }
+    const uint64_t c = ld_dev(ws.cand + ((int64_t)b * S + lo) * kCandCap + (i - L.off[lo]));
+    L.cand[i] = c;
+    L.mass[i] = fmass(key_float((uint32_t)c), bins.mx);
+  }
+  if (t == 0) L.thr = 0;
+  __syncthreads();
+  // ---- the threshold: the largest key whose candidates at or above it, with the bins above, carry
+  // `need`; each candidate against all, or over 256 of them (ties) radix selection by mass over the bits
+  // in which they differ, 8 at a time
+  uint32_t thr = 0;
+  if (n <= kSplitThreads) {
+    const Pairs pairs(n);
+    const uint32_t key = (uint32_t)L.cand[min(pairs.entry(), n - 1)];
+    const uint64_t f = above + pairs.mass(L.cand, L.mass, key, ~0u);
+    wave_to_lds_max(&L.thr, pairs.entry() < n && f >= need ? key : 0u);
+    __syncthreads();
+    thr = L.thr;
+  } else {
+    key0 = (uint32_t)L.cand[0];
+    for (int i = t; i < n; i += kSplitThreads) diff |= (uint32_t)L.cand[i] ^ key0;
+    if (diff) atomicOr(&L.diff, diff);
+    __syncthreads();
+    diff = L.diff;
+    thr = key0;
+  }
+  if (diff) {
+    const int top = 32 - __builtin_clz(diff);
+    thr = top == 32 ? 0u : key0 >> top << top;
+    uint64_t acc = above;
+    for (int hi = top; hi > 0;) {
+      const int width = min(hi, 8), shift = hi - width;
+      const uint32_t himask = hi == 32 ? 0u : ~0u << hi, nb = 1u << width;
       hi = shift;
-      int4* hv = reinterpret_cast<int4*>(s_hist + lane * 32);  // this lane's 32 bins, 4 a vector
-#pragma unroll
-      for (int i = 0; i < 8; ++i) hv[i] = make_int4(0, 0, 0, 0);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int r = 0; r < kMergeRegs; ++r)
-        if (ck[r] != 0u && (ck[r] & himask) == (thr & himask))
-          atomicAdd(&s_hist[(ck[r] >> shift) & (nb - 1u)], 1);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_wave_barrier();
-      // this lane's bins [32 lane, 32 lane + 32), in registers; the count in the bins of the
-      // lanes above
-      int bins[32];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int4 v = hv[i];
-        bins[4 * i] = v.x;
-        bins[4 * i + 1] = v.y;
-        bins[4 * i + 2] = v.z;
-        bins[4 * i + 3] = v.w;
+      __syncthreads();
+      L.hist[t] = 0;
+      __syncthreads();
+      for (int i = t; i < n; i += kSplitThreads) {
+        const uint32_t key = (uint32_t)L.cand[i];
+        if ((key & himask) == (thr & himask))
+          atomicAdd((unsigned long long*)&L.hist[(key >> shift) & (nb - 1u)],
+                    (unsigned long long)L.mass[i]);
       }
-      int own = 0;
-#pragma unroll
-      for (int i = 0; i < 32; ++i) own += bins[i];
-      int incl = own;  // bins of this lane and every lane above it
-#pragma unroll
-      for (int o = 1; o < kWave; o <<= 1) {
-        const int v = __shfl_down(incl, o, kWave);
-        incl += lane + o < kWave ? v : 0;
+      __syncthreads();
+      const uint64_t own = L.hist[kSplitThreads - 1 - t];  // (from the largest digit down)
+      uint64_t sum;
+      const uint64_t in = acc + block_scan256(own, L.redu, sum);
+      if (in >= need && in - own < need) {
+        L.bin = kSplitThreads - 1 - t;
+        L.above = in - own;
       }
-      const bool mine = above + incl >= k && above + incl - own < k;
-      int dig = 0, abv = 0;
-      {
-        int acc = above + incl - own;
-        bool found = false;
+      __syncthreads();
+      thr |= (uint32_t)L.bin << shift;
+      acc = L.above;
+    }
+  }
+  for (int i = t; i < n; i += kSplitThreads) {
+    const uint64_t c = L.cand[i];
+    if ((uint32_t)c >= thr)
+      atomicAdd((unsigned long long*)&s_tile[(uint32_t)(c >> 32) / kSplitTile],
+                (unsigned long long)L.mass[i]);
+  }
+  __syncthreads();
+  pick_token(p, vocab, vec, bins.mx, thr, s_tile, ntiles, uniform[b], out + b, L.redu, &L.at);
+}
+
+// ---- Top-k rows (0 < k <= kTopKMax, any top-p), one workgroup a row.  The k-th largest of the row's
+// group maxima is a lower bound T0 of its k-th largest logit T* (k logits lie at or above it), and a
+// close one: with 640 groups of 256 logits, about 57 logits lie above it at k = 50.  Only the groups
+// whose maximum reaches T0 are read again (a tenth of the row), and their logits with key >= T0 are the
+// candidates: over them, the largest T with #{key >= T} >= k is T* itself.  sample_row's rule on the
+// candidates alone (T*, the top-p threshold, the inverse CDF in vocabulary order, with the same integer
+// masses) gives the same token.  Where more than kTopkCands logits lie above T0 (large logits close
+// together in the vocabulary), the bound is raised first.  Rows that cannot be finished this way (ties
+// beyond kTopkCands, fewer than k numbers) are handed back to sample_kernel through `fallback`.
+constexpr int kRadixBins = 2048;  // the largest digit (11 bits) of the radix selection
+
+constexpr int kTopkCands = 1024;  // candidates of a top-k row at most
+struct TopkLds {
+  union {
+    int h[kRadixBins];  // (16-byte vector accesses)
+    uint64_t mass[kTopkCands];
+  };
+  uint64_t cand[kTopkCands];  // index << 32 | key
+  uint64_t sum;
+  uint16_t active[kGroups];
+  int wsum[kSplitThreads / kWave];
+  uint32_t top, thr;  // (thr: complemented)
+  int n, na, dig, above, cnt;
+};
+
+// The digit of the histogram L.h[0 .. 2048) at which the count from the top, `above` included, reaches
+// k: L.dig, the count above it (L.above) and up to it (L.cnt), for every thread.
+__device__ __forceinline__ void digit_select(TopkLds& L, int above, int k) {
+  const int t = threadIdx.x, lane = t & (kWave - 1), wv = t / kWave;
+  // thread t owns bins [8t, 8t + 8); the count in its bins and in every bin above them
+  int bins[8];
+  {
+    const int4 a = reinterpret_cast<const int4*>(L.h)[2 * t], c = reinterpret_cast<const int4*>(L.h)[2 * t + 1];
+    bins[0] = a.x; bins[1] = a.y; bins[2] = a.z; bins[3] = a.w;
+    bins[4] = c.x; bins[5] = c.y; bins[6] = c.z; bins[7] = c.w;
+  }
+  int own = 0;
 #pragma unroll
-        for (int i = 31; i >= 0; --i) {
-          const bool hit = !found && acc + bins[i] >= k;
-          dig = hit ? lane * 32 + i : dig;
-          abv = hit ? acc : abv;
-          found = found || hit;
-          acc += bins[i];
+  for (int e = 0; e < 8; ++e) own += bins[e];
+  int incl = own;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const int v = __shfl_down(incl, o, kWave);
+    incl += lane + o < kWave ? v : 0;
+  }
+  if (lane == 0) L.wsum[wv] = incl;
+  __syncthreads();
+  for (int w2 = wv + 1; w2 < kSplitThreads / kWave; ++w2) incl += L.wsum[w2];
+  if (above + incl >= k && above + incl - own < k) {  // the thread whose bins hold the k-th largest
+    int acc = above + incl - own;
+#pragma unroll
+    for (int e = 7; e >= 0; --e) {
+      if (acc + bins[e] >= k) {
+        L.dig = 8 * t + e;
+        L.above = acc;
+        L.cnt = acc + bins[e];
+        break;
+      }
+      acc += bins[e];
+    }
+  }
+  __syncthreads();
+}
+__device__ __forceinline__ void clear_hist(TopkLds& L) {
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kRadixBins / kSplitThreads / 4; ++i)
+    reinterpret_cast<int4*>(L.h)[threadIdx.x * (kRadixBins / kSplitThreads / 4) + i] = make_int4(0, 0, 0, 0);
+  __syncthreads();
+}
+
+// A bound that k of the row's n group maxima reach, and no more than the upper half of the k-th largest
+// of them (0: fewer than k groups), by bisection on its bits; every wave for itself, the maxima in its
+// registers.
+__device__ __forceinline__ uint32_t group_bound(const uint16_t* gm, int n, int k) {
+  constexpr int R = kGroups / kWave / 4;
+  const int lane = threadIdx.x & (kWave - 1);
+  uint32_t v[kGroups / kWave];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int i = 4 * (r * kWave + lane);
+    const uint2 u = *reinterpret_cast<const uint2*>(gm + i);
+    v[4 * r] = i < n ? u.x & 0xFFFFu : 0u;
+    v[4 * r + 1] = i + 1 < n ? u.x >> 16 : 0u;
+    v[4 * r + 2] = i + 2 < n ? u.y & 0xFFFFu : 0u;
+    v[4 * r + 3] = i + 3 < n ? u.y >> 16 : 0u;
+  }
+  // the bits in which some maximum differs from the largest, from the highest such bit down; a bound
+  // that exactly k maxima reach is as good as the k-th largest
+  uint32_t hi = 0, lo = 0xFFFFu;
+#pragma unroll
+  for (int r = 0; r < kGroups / kWave; ++r) {
+    hi = max(hi, v[r]);
+    lo = min(lo, v[r] ? v[r] : 0xFFFFu);
+  }
+  hi = wave_max_u32(hi);
+  lo = ~wave_max_u32(~lo);
+  if (n < k) return 0;
+  const uint32_t diff = hi ^ min(lo, hi);
+  uint32_t bit = diff ? 0x80000000u >> __builtin_clz(diff) : 0u;
+  uint32_t t = bit ? hi & ~(2 * bit - 1) : hi;
+#pragma unroll 1
+  for (; bit; bit >>= 1) {
+    const uint32_t c = t | bit;
+    int cnt = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (4 * r * kWave >= n) break;  // (uniform)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) cnt += __popcll(__ballot(v[4 * r + e] >= c));
+    }
+    if (cnt >= k) t = c;
+    if (cnt == k) break;
+  }
+  return t;
+}
+
+// The least logit whose key's upper half is at or above ts (ts 1: any number; a zero may be taken for
+// the other one, a candidate too many).
+__device__ __forceinline__ float half_key_float(uint32_t ts) { return ts <= 0x7Fu ? -INFINITY : key_float(ts << 16); }
+
+// The token of a top-k row from its n candidates (in L.cand; at least the row's k largest): the k-th
+// largest key T*, the top-p threshold over the top-k set, and the inverse CDF in vocabulary order, each by
+// comparing every entry with all (Pairs; over 256 candidates, T* by radix selection).  The three stages
+// share one loop: the code runs once a row, and its length is what it costs (instruction fetch).
+__device__ __forceinline__ void topk_merge(int b, int n, int k, float pp, const float* uniform, int32_t* out,
+                                           const SplitWs& ws, TopkLds& L) {
+  const int t = threadIdx.x;
+  constexpr int Q = kTopkCands / kSplitThreads;
+  uint32_t most = 0;
+  if (t == 0) {
+    L.top = 0u;
+    L.thr = 0u;
+    L.sum = 0;
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int i = t; i < n; i += kSplitThreads) {
+    most = max(most, (uint32_t)L.cand[i]);
+    if (n <= kSplitThreads) L.mass[i] = 1;  // (counts)
+  }
+  wave_to_lds_max(&L.top, most);
+  if (n > kSplitThreads) {
+    uint32_t prefix = 0u, himask = 0u;
+    int above = 0;
+#pragma unroll 1
+    for (int level = 0; level < 3; ++level) {  // digits of 11, 11 and 10 bits
+      const int shift = level == 0 ? 21 : (level == 1 ? 10 : 0);
+      const uint32_t nb = level < 2 ? 2048u : 1024u;
+      clear_hist(L);
+#pragma unroll 1
+      for (int i = t; i < n; i += kSplitThreads) {
+        const uint32_t key = (uint32_t)L.cand[i];
+        if ((key & himask) == prefix) atomicAdd(&L.h[(key >> shift) & (nb - 1u)], 1);
+      }
+      __syncthreads();
+      digit_select(L, above, k);
+      prefix |= (uint32_t)L.dig << shift;
+      himask |= (nb - 1u) << shift;
+      above = L.above;
+    }
+    if (t == 0) L.thr = ~prefix;
+  }
+  __syncthreads();
+  const float mx = key_float(L.top);
+  uint32_t thr = 0;
+  uint64_t need = 0, target = 0;
+  int m = n;
+#pragma unroll 1
+  for (int stage = n > kSplitThreads ? 1 : 0; stage < 3; ++stage) {
+    // 0: the entries above each; 1: at or above it; 2: kept and before it in vocabulary order
+    const bool skip = stage == 1 && !(pp < 1.f);
+    if (stage == 1) {
+      // the top-k set, in any order: index and key, mass
+      thr = ~L.thr;
+      uint64_t c[Q];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) c[q] = t + q * kSplitThreads < n ? L.cand[t + q * kSplitThreads] : 0;
+      if (t == 0) L.na = 0;
+      __syncthreads();
+      uint64_t own = 0;
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        if (t + q * kSplitThreads < n && (uint32_t)c[q] >= thr) {
+          const int pos = atomicAdd(&L.na, 1);
+          const uint64_t f = fmass(key_float((uint32_t)c[q]), mx);
+          L.cand[pos] = c[q];
+          L.mass[pos] = f;
+          own += f;
         }
       }
-      const uint64_t who = __ballot(mine);
-      const int src = (int)__builtin_ctzll(who);
-      dig = __shfl(dig, src, kWave);
-      above = __shfl(abv, src, kWave);
-      thr |= (uint32_t)dig << shift;
+      wave_to_lds_sum(&L.sum, own);
+      if (t == 0) L.top = 0u;
+      __syncthreads();
+      m = L.na;
+      const uint64_t kmass = L.sum;
+      const double needd = ceil((double)fmaxf(pp, 0.f) * (double)kmass);
+      need = needd < 1.0 ? 1 : (uint64_t)needd;
+      if (need > kmass) need = kmass;
+    } else if (stage == 2) {
+      // the kept mass, and where in it the uniform falls
+      thr = max(thr, L.top);
+      if (t == 0) L.sum = 0;
+      __syncthreads();
+      uint64_t own = 0;
+#pragma unroll 1
+      for (int e = t; e < m; e += kSplitThreads) own += (uint32_t)L.cand[e] >= thr ? L.mass[e] : 0;
+      wave_to_lds_sum(&L.sum, own);
+      __syncthreads();
+      const uint64_t ms = L.sum;
+      if (ms == 0) {  // (uniform)
+        if (t == 0) out[b] = -1;
+        return;
+      }
+      const double uu = fminf(fmaxf(uniform[b], 0.f), 1.f);
+      target = (uint64_t)(uu * (double)ms);
+      if (target >= ms) target = ms - 1;
     }
+    const Pairs pairs(m);
+    uint32_t pick = 0;
+    if (!skip) {
+#pragma unroll 1
+      for (int e = pairs.entry(); e < (m + kSplitThreads - 1) / kSplitThreads * kSplitThreads; e += kSplitThreads) {
+        const uint64_t ce = L.cand[min(e, m - 1)];
+        const uint32_t key = (uint32_t)ce;
+        const uint64_t f = pairs.mass(L.cand, L.mass, stage == 0 ? key + 1 : stage == 1 ? key : thr,
+                                      stage == 2 ? (uint32_t)(ce >> 32) : ~0u);
+        if (e < m) {
+          if (stage == 0) {
+            if ((int)f < k) pick = max(pick, ~key);  // (the least key with fewer than k above it)
+          } else if (stage == 1) {
+            if (f >= need) pick = max(pick, key);
+          } else {
+            const uint64_t me = key >= thr ? L.mass[e] : 0;
+            if (me > 0 && f <= target && target < f + me && pairs.first()) out[b] = (int32_t)(ce >> 32);
+          }
+        }
+      }
+      if (stage < 2) wave_to_lds_max(stage == 0 ? &L.thr : &L.top, pick);
+    }
+    __syncthreads();
   }
-  const float mx = key_float(mxk);
-  // the top-k set K, compacted into LDS in a fixed order (ballots): index, key, mass
-  uint64_t kmass = 0;
-  int m = 0;
+}
+
+// The row's active groups as vectors of 8 logits: item i is at base(i) in the row.
+struct ActiveVectors {
+  const GroupShape& g;
+  const uint16_t* active;
+  __device__ __forceinline__ int base(int item) const {
+    const int vs = g.tg + g.gl;
+    const int gi = active[item >> vs], v = item & ((1 << vs) - 1);
+    const int sl = gi >> g.ps, q = (gi & (g.per_slice - 1)) << g.gl;  // (a tile group's threads from q % 256 on)
+    const int tile = sl * kSliceTiles + ((q / kSplitThreads) << g.tg) + (v >> g.gl);
+    return tile * kSplitTile + 8 * (q % kSplitThreads + (v & ((1 << g.gl) - 1)));
+  }
+};
+// f(first item, x, ok) for U vectors of this thread at a time (the u-th: item first + u * kSplitThreads).
+template <int U, typename T, typename F>
+__device__ __forceinline__ void each_active(const T* p, int vocab, bool vec, const ActiveVectors& av, int total, F&& f) {
+  constexpr int R = 8 * sizeof(T) / 16;
+  const bool whole = vec && vocab >= 8;
+  const int last = (vocab - 8) / 8 * 8;
+#pragma unroll 1
+  for (int i0 = threadIdx.x; i0 < total; i0 += U * kSplitThreads) {
+    int base[U];
+    uint4 raw[U][R];
 #pragma unroll
-  for (int r = 0; r < kMergeRegs; ++r) {
-    const bool keep = ck[r] >= thr;
-    const uint64_t bal = __ballot(keep);
-    const uint64_t cm = keep ? fmass(key_float(ck[r]), mx) : 0;
-    if (keep) {
-      const int pos = m + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
-                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0));
-      if (pos < kKeptCap) {
-        s_sidx[pos] = cidx[r];
-        s_skey[pos] = ck[r];
-        s_smass[pos] = cm;
+    for (int u = 0; u < U; ++u) {
+      const int item = i0 + u * kSplitThreads;
+      base[u] = item < total ? av.base(item) : vocab;
+      if (whole) {
+#pragma unroll
+        for (int v = 0; v < R; ++v)
+          raw[u][v] = *reinterpret_cast<const uint4*>(p + min(base[u], last) + v * (16 / sizeof(T)));
       }
     }
-    kmass += cm;
-    m += __popcll(bal);
-  }
-  kmass = wave_sum_u64(kmass);
-  if (m > kKeptCap) {
-    if (lane == 0) ws.fallback[b] = 1;
-    return;
-  }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // K is in LDS for every lane
-  __builtin_amdgcn_wave_barrier();
-  // The top-p threshold over K: the largest T with mass{key >= T} >= need, which is the key of
-  // one of K's members; each lane weighs its members' keys over all of K.
-  uint64_t ms = kmass;
-  const float pp = top_p ? top_p[b] : top_p_all;
-  if (pp < 1.f && kmass > 0) {
-    const double needd = ceil((double)fmaxf(pp, 0.f) * (double)kmass);
-    uint64_t need = needd < 1.0 ? 1 : (uint64_t)needd;
-    if (need > kmass) need = kmass;
-    uint32_t tp = 0;
-    for (int e0 = 0; e0 < m; e0 += kWave) {
-      const int e = e0 + lane;
-      const uint32_t ke = e < m ? s_skey[e] : ~0u;
-      uint64_t f = 0;  // mass{key >= ke} over K, its members taken 64 at a time through readlane
-      for (int x0 = 0; x0 < m; x0 += kWave) {
-        const uint32_t kx = x0 + lane < m ? s_skey[x0 + lane] : 0u;
-        const uint64_t mx2 = x0 + lane < m ? s_smass[x0 + lane] : 0;
-        const uint32_t mlo = (uint32_t)mx2, mhi = (uint32_t)(mx2 >> 32);
-        const int nx = min(kWave, m - x0);
-#pragma unroll 8
-        for (int xx = 0; xx < nx; ++xx) {
-          const uint32_t kk = (uint32_t)__builtin_amdgcn_readlane(kx, xx);
-          const uint64_t mm = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(mhi, xx) << 32) |
-                              (uint64_t)(uint32_t)__builtin_amdgcn_readlane(mlo, xx);  // (readlane is signed)
-          f += kk >= ke ? mm : 0;
-        }
+    float x[U][8];
+    bool ok[U][8];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      T e[8];
+      __builtin_memcpy(e, raw[u], sizeof(e));
+      if (!(whole && base[u] + 8 <= vocab)) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          if (base[u] + k < vocab) e[k] = p[base[u] + k];
       }
-      if (e < m && f >= need) tp = max(tp, ke);
-    }
-    tp = wmax_u(tp);
-    if (tp > thr) {  // the kept set shrinks to S = {key >= tp}: recompact it in place, in order
-      thr = tp;
-      int n2 = 0;
-      uint64_t m2 = 0;
-      for (int e0 = 0; e0 < m; e0 += kWave) {
-        const int e = e0 + lane;
-        const bool keep = e < m && s_skey[e] >= thr;
-        const int ie = keep ? s_sidx[e] : 0;
-        const uint32_t kk = keep ? s_skey[e] : 0u;
-        const uint64_t mm = keep ? s_smass[e] : 0;
-        const uint64_t bal = __ballot(keep);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_wave_barrier();  // (every lane has read its entry before any is moved)
-        if (keep) {
-          const int pos = n2 + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
-                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0));
-          s_sidx[pos] = ie;
-          s_skey[pos] = kk;
-          s_smass[pos] = mm;
-        }
-        m2 += mm;
-        n2 += __popcll(bal);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_wave_barrier();
-      }
-      m = n2;
-      ms = wave_sum_u64(m2);
-    }
-  }
-  if (ms == 0) {
-    if (lane == 0) out[b] = -1;
-    return;
-  }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the kept set is in LDS for every lane
-  __builtin_amdgcn_wave_barrier();
-  const double uu = fminf(fmaxf(uniform[b], 0.f), 1.f);
-  uint64_t target = (uint64_t)(uu * (double)ms);
-  if (target >= ms) target = ms - 1;
-  for (int e0 = 0; e0 < m; e0 += kWave) {
-    const int e = e0 + lane;
-    const int ie = e < m ? s_sidx[e] : 0x7fffffff;
-    const uint64_t me = e < m ? s_smass[e] : 0;
-    uint64_t pre = 0;  // mass of the kept logits before this one in vocabulary order, their members
-                       // taken 64 at a time through readlane
-    for (int f0 = 0; f0 < m; f0 += kWave) {
-      const int fi = f0 + lane < m ? s_sidx[f0 + lane] : 0x7fffffff;
-      const uint64_t fm = f0 + lane < m ? s_smass[f0 + lane] : 0;
-      const uint32_t flo = (uint32_t)fm, fhi = (uint32_t)(fm >> 32);
-      const int nf = min(kWave, m - f0);
-#pragma unroll 8
-      for (int ff = 0; ff < nf; ++ff) {
-        const int ii = __builtin_amdgcn_readlane(fi, ff);
-        const uint64_t mm = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(fhi, ff) << 32) |
-                            (uint64_t)(uint32_t)__builtin_amdgcn_readlane(flo, ff);  // (readlane is signed)
-        pre += ii < ie ? mm : 0;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        ok[u][k] = base[u] + k < vocab;
+        x[u][k] = to_f32(e[k]);
       }
     }
-    if (e < m && me > 0 && pre <= target && target < pre + me) out[b] = ie;
+    f(i0, x, ok);
   }
 }
 
 template <typename T>
+__device__ __forceinline__ void topk_row(const T* p, int vocab, bool vec, int b, int k, float pp, const float* uniform,
+                                         int32_t* out, const SplitWs& ws, TopkLds& L) {
+  const int t = threadIdx.x;
+  const GroupShape& g = ws.g;
+  const uint16_t* gm = ws.gmax + (int64_t)b * kGroups;
+  if (t == 0) L.n = L.na = 0;
+  uint32_t ts = max(group_bound(gm, g.n, k), 1u);  // (0 is no number)
+  __syncthreads();
+  for (int i = t; i < g.n; i += kSplitThreads)
+    if (gm[i] >= ts) L.active[atomicAdd(&L.na, 1)] = (uint16_t)i;
+  __syncthreads();
+  const ActiveVectors av{g, L.active};
+  const int total = L.na << (g.tg + g.gl);
+#pragma unroll 1
+  for (bool raised = false;; raised = true) {
+    const float lim = half_key_float(ts);
+    each_active<2>(p, vocab, vec, av, total, [&](int i0, const float (&x)[2][8], const bool (&ok)[2][8]) __attribute__((always_inline)) {
+      uint32_t in = 0;
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) in |= (uint32_t)(ok[u][e] && x[u][e] >= lim) << (8 * u + e);
+      for (; in; in &= in - 1) {  // (few threads have any)
+        const int pos = atomicAdd(&L.n, 1);
+        const int i = __builtin_ctz(in), idx = av.base(i0 + (i >> 3) * kSplitThreads) + (i & 7);
+        if (pos < kTopkCands) L.cand[pos] = ((uint64_t)(uint32_t)idx << 32) | fkey(to_f32(p[idx]));
+      }
+    });
+    __syncthreads();
+    if (raised || L.n <= kTopkCands) break;  // (uniform)
+    // The start of the range of 16-bit keys (a digit of 11 bits, then one of 5) that holds the k-th
+    // largest, refined until the keys at or above it fit: each level histograms, in LDS, the keys inside
+    // the range chosen so far.
+    const uint32_t floor_key = ts;
+    uint32_t prefix = 0u, himask = 0u;
+    int above = 0;
+#pragma unroll 1
+    for (int level = 0; level < 2; ++level) {
+      const int shift = level == 0 ? 5 : 0;
+      const uint32_t nb = level == 0 ? 2048u : 32u;
+      clear_hist(L);
+      each_active<1>(p, vocab, vec, av, total, [&](int, const float (&x)[1][8], const bool (&ok)[1][8]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t kk = ok[0][e] ? fkey(x[0][e]) >> 16 : 0u;
+          if (kk >= floor_key && (kk & himask) == prefix) atomicAdd(&L.h[(kk >> shift) & (nb - 1u)], 1);
+        }
+      });
+      if (t == 0) L.n = 0;
+      __syncthreads();
+      digit_select(L, above, k);
+      prefix |= (uint32_t)L.dig << shift;
+      himask |= (nb - 1u) << shift;
+      above = L.above;
+      ts = max(prefix, floor_key);
+      if (L.cnt <= kTopkCands) break;  // (uniform)
+    }
+  }
+  const int n = L.n;
+  if (n > kTopkCands || n < k) {  // (uniform; fewer than k: the row has fewer numbers)
+    if (t == 0) ws.fallback[b] = 1;
+    return;
+  }
+  topk_merge(b, n, k, pp, uniform, out, ws, L);
+}
+
+template <typename T>
+__global__ __launch_bounds__(kSplitThreads) __attribute__((amdgpu_waves_per_eu(5))) void split_pass_kernel(
+    const T* logits, int64_t row_stride, int vocab, const int32_t* top_k, int32_t top_k_all, const float* top_p,
+    float top_p_all, const float* uniform, int32_t* out, SplitWs ws) {
+  union Lds {
+    uint64_t tile[kMaxSplitTiles];
+    uint64_t hist[kPBins];
+    TopkLds k;
+  };
+  __shared__ __align__(16) Lds L;
+  __shared__ float redf[8];
+  __shared__ uint64_t redu[kSliceTiles][4];
+  __shared__ int s_last;
+  __shared__ TokenAt s_at;
+  const int s = blockIdx.x, b = blockIdx.y, S = gridDim.x;
+  const int kind = row_kind(b, vocab, top_k, top_k_all, top_p, top_p_all);
+  if (kind == kOtherRow) return;
+  const T* p = logits + (int64_t)b * row_stride;
+  const bool vec = ((uintptr_t)p % 16) == 0;
+  const int j0 = s * kSliceTiles, j1 = min(j0 + kSliceTiles, split_tiles(vocab));
+  const float pp = top_p ? top_p[b] : top_p_all;
+  if (kind == kTopKRow) {
+    if (s == 0) topk_row(p, vocab, vec, b, top_k ? top_k[b] : top_k_all, pp, uniform, out, ws, L.k);
+    return;
+  }
+  SliceLoad<T> sl;
+  sl.issue(p, vocab, vec, j0, j1);
+  if (kind == kWholeRow) whole_slice(p, vocab, vec, sl, s, b, S, uniform, out, ws, L.tile, redf, redu, &s_last, &s_at);
+  else topp_hist(p, vocab, vec, sl, s, b, S, pp, out, ws, L.hist, redf, redu[0], &s_last);
+}
+
+template <typename T>
+__global__ __launch_bounds__(kSplitThreads) void split_finish_kernel(const T* logits, int64_t row_stride, int vocab,
+                                                                     const int32_t* top_k, int32_t top_k_all,
+                                                                     const float* top_p, float top_p_all,
+                                                                     const float* uniform, int32_t* out, SplitWs ws) {
+  __shared__ ToppLds L;
+  extern __shared__ uint64_t s_tile[];  // [ntiles]
+  const int s = blockIdx.x, b = blockIdx.y;
+  if (row_kind(b, vocab, top_k, top_k_all, top_p, top_p_all) == kTopPRow)
+    topp_finish(logits + (int64_t)b * row_stride, vocab, s, b, gridDim.x, uniform, out, ws, L, s_tile);
+}
+
+// Which kinds of rows a call can hold (scalars settle it on the host, per-row tensors need all), and
+// whether the workspace takes them over many workgroups.
+struct SamplePlan {
+  bool topk = true, topp = true, whole = true, other = true, split = false;
+  SamplePlan(int rows, int vocab, const int32_t* top_k, int32_t top_k_all, const float* top_p, float top_p_all,
+             const void* ws, int64_t ws_bytes) {
+    if (!top_k && !top_p) {
+      const int kind = row_kind_of(top_k_all, top_p_all, vocab);
+      whole = kind == kWholeRow;
+      topk = kind == kTopKRow;
+      topp = kind == kTopPRow;
+      other = kind == kOtherRow;
+    }
+    split = ws && (whole || topk || topp) && rows <= 65535 && split_tiles(vocab) <= kMaxSplitTiles &&
+            ws_bytes >= split_ws_bytes(rows, vocab);
+  }
+};
+
+// The launches after the scan.
+template <typename T>
 int launch_sample(const T* logits, int64_t row_stride, int rows, int vocab, const int32_t* top_k, int32_t top_k_all,
-                  const float* top_p, float top_p_all, const float* uniform, int32_t* out, void* ws,
-                  int64_t ws_bytes, hipStream_t s) {
-  // which kinds of rows there are: scalars settle it on the host, per-row tensors need all
-  bool any_whole = true, any_topk = true, any_other = true;
-  if (!top_k && !top_p) {
-    const int kind = row_kind_of(top_k_all, top_p_all, vocab);
-    any_whole = kind == kWholeRow;
-    any_topk = kind == kTopKRow;
-    any_other = kind == kOtherRow;
-  }
-  const bool split = ws && (any_whole || any_topk) && rows <= 65535 && split_tiles(vocab) <= kMaxSplitTiles &&
-                     ws_bytes >= split_ws_bytes(rows, vocab);
-  SplitWs w{};
-  if (split) {
-    w = split_ws(ws, rows, vocab);
-    const dim3 grid((unsigned)split_slices(vocab), (unsigned)rows);
-    // (split_max_kernel also resets every row's counter and fallback flag for the kernels below;
-    // the top-k merge sets its rows' flags itself, so a batch of top-k rows alone skips it)
-    if (any_whole) {
-      hipLaunchKernelGGL(split_max_kernel<T>, grid, dim3(kSplitThreads), 0, s, logits, row_stride, vocab, top_k,
-                         top_k_all, top_p, top_p_all, w);
-      hipLaunchKernelGGL(split_sample_kernel<T>, grid, dim3(kSplitThreads), 0, s, logits, row_stride, vocab, top_k,
+                  const float* top_p, float top_p_all, const float* uniform, int32_t* out, const SamplePlan& plan,
+                  const SplitWs& w, hipStream_t s) {
+  const dim3 grid((unsigned)split_slices(vocab), (unsigned)rows);
+  if (plan.split) {
+    // (top-k rows take one workgroup)
+    hipLaunchKernelGGL(split_pass_kernel<T>, plan.whole || plan.topp ? grid : dim3(1, (unsigned)rows),
+                       dim3(kSplitThreads), 0, s, logits, row_stride, vocab, top_k, top_k_all, top_p, top_p_all, uniform,
+                       out, w);
+    if (plan.topp)
+      hipLaunchKernelGGL(split_finish_kernel<T>, grid, dim3(kSplitThreads), split_tiles(vocab) * sizeof(uint64_t), s, logits, row_stride, vocab, top_k,
                          top_k_all, top_p, top_p_all, uniform, out, w);
-    }
-    if (any_topk) {
-      hipLaunchKernelGGL(split_topk_kernel<T>, grid, dim3(kSplitThreads), 0, s, logits, row_stride, vocab, top_k,
-                         top_k_all, top_p, top_p_all, uniform, out, w);
-      hipLaunchKernelGGL(split_topk_merge_kernel, dim3((unsigned)rows), dim3(kWave), 0, s, vocab, top_k, top_k_all,
-                         top_p, top_p_all, uniform, out, w);
-    }
   }
-  if (!split || any_other || any_topk)  // (top-k rows may be handed back)
+  if (!plan.split || plan.other || plan.topk || plan.topp)  // (rows may be handed back)
     hipLaunchKernelGGL(sample_kernel<T>, dim3(rows), dim3(kThreads), 0, s, logits, row_stride, vocab, top_k,
-                       top_k_all, top_p, top_p_all, uniform, out, split ? 1 : 0, w.fallback);
+                       top_k_all, top_p, top_p_all, uniform, out, plan.split ? 1 : 0, w.fallback);
   return (int)hipGetLastError();
+}
+
+template <typename T>
+int scan_and_sample(const T* logits, int64_t row_stride, int rows, int vocab, const int32_t* top_k, int32_t top_k_all,
+                    const float* top_p, float top_p_all, const float* uniform, int32_t* out, void* ws,
+                    int64_t ws_bytes, hipStream_t s) {
+  const SamplePlan plan(rows, vocab, top_k, top_k_all, top_p, top_p_all, ws, ws_bytes);
+  SplitWs w{};
+  if (plan.split) {
+    w = split_ws(ws, rows, vocab);
+    hipLaunchKernelGGL((split_scan_kernel<T, false>), dim3((unsigned)split_slices(vocab), (unsigned)rows),
+                       dim3(kSplitThreads), 0, s, logits, row_stride, vocab, top_k, top_k_all, top_p, top_p_all,
+                       ScaleArgs<T>{}, w);
+  }
+  return launch_sample(logits, row_stride, rows, vocab, top_k, top_k_all, top_p, top_p_all, uniform, out, plan, w, s);
 }
 
 // The serving loop's scaling before sampling (ecahlang/main.py:169-170, 483-487), in one pass:
@@ -1076,13 +1544,7 @@ __global__ void scale_logits_kernel(const T* __restrict__ logits, int64_t row_st
     return;
   }
   auto scale = [&](T xv, T pv) __attribute__((always_inline)) -> float {
-    float y = to_f32(xv);
-    if (pen) {
-      const float d = to_f32(pv);
-      if (d != 1.f) y = to_f32(from_f32<T>(y / d));
-    }
-    if (t != 1.f) y = y / t;
-    return y;
+    return scale_logit<T>(xv, pv, pen != nullptr, t);
   };
   if (VEC && i0 + N <= vocab) {
     T xs[N], ps[N];
@@ -1151,13 +1613,13 @@ static int sample_entry(const void* logits, int64_t row_stride, int32_t rows, in
   if ((int64_t)vocab > (int64_t)kMaxTiles * kThreads * (16 / es)) return kBadArg;
   hipStream_t s = (hipStream_t)stream;
   if (dtype == kF16)
-    return launch_sample((const _Float16*)logits, row_stride, rows, vocab, top_k, top_k_all, top_p, top_p_all,
+    return scan_and_sample((const _Float16*)logits, row_stride, rows, vocab, top_k, top_k_all, top_p, top_p_all,
                          uniform, out, workspace, workspace_bytes, s);
   if (dtype == kBF16)
-    return launch_sample((const __hip_bfloat16*)logits, row_stride, rows, vocab, top_k, top_k_all, top_p,
+    return scan_and_sample((const __hip_bfloat16*)logits, row_stride, rows, vocab, top_k, top_k_all, top_p,
                          top_p_all, uniform, out, workspace, workspace_bytes, s);
   if (dtype == kF32)
-    return launch_sample((const float*)logits, row_stride, rows, vocab, top_k, top_k_all, top_p, top_p_all,
+    return scan_and_sample((const float*)logits, row_stride, rows, vocab, top_k, top_k_all, top_p, top_p_all,
                          uniform, out, workspace, workspace_bytes, s);
   return kBadDType;
 }
@@ -1181,4 +1643,42 @@ extern "C" int pkv_top_k_top_p_sampling_ws(const void* logits, int64_t row_strid
   if (workspace && ((uintptr_t)workspace % 8)) return kBadAlign;
   return sample_entry(logits, row_stride, rows, vocab, dtype, top_k, top_k_all, top_p, top_p_all, uniform, out,
                       workspace, workspace_bytes, stream);
+}
+
+// The two calls above in one: the sampler's first pass over the logits scales them.
+extern "C" int pkv_scaled_top_k_top_p_sampling(const void* logits, int64_t row_stride, int32_t rows, int32_t vocab,
+                                               int32_t dtype, const void* penalty, int64_t penalty_stride,
+                                               int32_t penalty_slots, const int32_t* penalty_rows,
+                                               const float* temperature, float* scaled, int64_t scaled_stride,
+                                               const int32_t* top_k, int32_t top_k_all, const float* top_p,
+                                               float top_p_all, const float* uniform, int32_t* out, void* workspace,
+                                               int64_t workspace_bytes, void* stream) {
+  if (workspace && ((uintptr_t)workspace % 8)) return kBadAlign;
+  if (rows < 0 || vocab <= 0 || row_stride < vocab || !uniform || !out) return kBadArg;
+  if (rows == 0) return kOk;
+  if (scaled_stride < vocab || !scaled) return kBadArg;
+  if (penalty && (!penalty_rows || penalty_stride < vocab || penalty_slots <= 0)) return kBadArg;
+  if (dtype != kF16 && dtype != kBF16 && dtype != kF32) return kBadDType;
+  const SamplePlan plan(rows, vocab, top_k, top_k_all, top_p, top_p_all, workspace, workspace_bytes);
+  if (!plan.split || ((uintptr_t)scaled | (uintptr_t)(scaled_stride * 4)) % 16) {
+    const int rc = pkv_scale_logits(logits, row_stride, rows, vocab, dtype, penalty, penalty_stride, penalty_slots,
+                                    penalty_rows, temperature, scaled, scaled_stride, stream);
+    return rc ? rc : sample_entry(scaled, scaled_stride, rows, vocab, kF32, top_k, top_k_all, top_p, top_p_all, uniform,
+                                  out, workspace, workspace_bytes, stream);
+  }
+  hipStream_t s = (hipStream_t)stream;
+  const SplitWs w = split_ws(workspace, rows, vocab);
+  const dim3 grid((unsigned)split_slices(vocab), (unsigned)rows);
+#define PKV_SCALE_SCAN(T)                                                                                          \
+  hipLaunchKernelGGL((split_scan_kernel<T, true>), grid, dim3(kSplitThreads), 0, s, (const T*)logits, row_stride,  \
+                     vocab, top_k, top_k_all, top_p, top_p_all,                                                    \
+                     (ScaleArgs<T>{(const T*)penalty, penalty_stride, penalty_slots, penalty_rows, temperature, scaled, \
+                                   scaled_stride}),                                                                \
+                     w)
+  if (dtype == kF16) PKV_SCALE_SCAN(_Float16);
+  else if (dtype == kBF16) PKV_SCALE_SCAN(__hip_bfloat16);
+  else PKV_SCALE_SCAN(float);
+#undef PKV_SCALE_SCAN
+  return launch_sample((const float*)scaled, scaled_stride, rows, vocab, top_k, top_k_all, top_p, top_p_all, uniform, out,
+                       plan, w, s);
 }

@@ -45,8 +45,8 @@ def top_k_top_p_sampling_from_logits(logits: torch.Tensor, top_k, top_p, indices
     ``penalty`` / ``penalty_rows`` / ``temperature`` (extensions) fold in the scaling the
     serving loop applies before sampling (ecahlang/main.py:169-170, 483-487):
     ``logits / penalty[penalty_rows]`` in the logits' dtype, then ``/ temperature`` in float32,
-    rounded exactly as those tensor ops round, in one pass (:func:`scale_logits`) before the
-    sampler.
+    rounded exactly as those tensor ops round, in the sampler's first pass (as
+    :func:`scale_logits` does it).
     ``penalty`` is the [slots, vocab] table in the logits' dtype (the manager's
     ``mask_penalty``), ``penalty_rows`` the int32 slot of each row (``batch_to_seq_len``), and
     ``temperature`` a float32 tensor with one entry per row, or a number."""
@@ -71,15 +71,21 @@ def top_k_top_p_sampling_from_logits(logits: torch.Tensor, top_k, top_p, indices
         if uniform.numel() != rows:
             raise ValueError("uniform must have one entry per row")
     out = torch.empty(rows, dtype=torch.int32, device=dev)
-    if penalty is not None or temperature is not None:
-        logits = scale_logits(logits, penalty, penalty_rows, temperature)
     ws_bytes = lib().pkv_sampling_workspace_bytes(rows, vocab)
     ws = torch.empty(max(ws_bytes, 8), dtype=torch.uint8, device=dev)
-    check(lib().pkv_top_k_top_p_sampling_ws(
-        logits.data_ptr(), logits.stride(0), rows, vocab, dtype_code(logits.dtype),
-        k_t.data_ptr() if k_t is not None else None, int(k_all),
-        p_t.data_ptr() if p_t is not None else None, float(p_all),
-        uniform.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(), stream_ptr(dev)), "top-k / top-p sampling")
+    filters = (k_t.data_ptr() if k_t is not None else None, int(k_all),
+               p_t.data_ptr() if p_t is not None else None, float(p_all),
+               uniform.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(), stream_ptr(dev))
+    if penalty is not None or temperature is not None:
+        scale, _keep = _scale_args(logits, penalty, penalty_rows, temperature)
+        # whole 16-byte vectors a row, whatever the vocabulary
+        scaled = torch.empty(rows, (vocab + 3) // 4 * 4, dtype=torch.float32, device=dev)
+        check(lib().pkv_scaled_top_k_top_p_sampling(*scale, scaled.data_ptr(), scaled.stride(0), *filters),
+              "scaled top-k / top-p sampling")
+    else:
+        check(lib().pkv_top_k_top_p_sampling_ws(
+            logits.data_ptr(), logits.stride(0), rows, vocab, dtype_code(logits.dtype), *filters),
+            "top-k / top-p sampling")
     return out
 
 
@@ -91,6 +97,15 @@ def scale_logits(logits: torch.Tensor, penalty: torch.Tensor | None = None,
     materialising ``penalty[penalty_rows]``.  Returns a new float32 [rows, vocab] tensor; a row
     whose ``penalty_rows`` entry is not a row of ``penalty`` comes back as NaN (and samples as
     -1), where the tensor expression would raise an indexing error."""
+    args, _keep = _scale_args(logits, penalty, penalty_rows, temperature)
+    out = torch.empty(logits.shape, dtype=torch.float32, device=logits.device)
+    check(lib().pkv_scale_logits(*args, out.data_ptr(), out.stride(0), stream_ptr(logits.device)), "scale_logits")
+    return out
+
+
+def _scale_args(logits, penalty, penalty_rows, temperature):
+    """The checked arguments of the library's scaling calls up to temperature, and the tensors they
+    point into."""
     if logits.dim() != 2 or logits.stride(1) != 1 or logits.device.type != "cuda":
         raise ValueError("logits must be a [batch, vocab] CUDA tensor with a unit inner stride")
     rows, vocab = logits.shape
@@ -119,8 +134,5 @@ def scale_logits(logits: torch.Tensor, penalty: torch.Tensor | None = None,
             temp = temp.contiguous()
         else:
             temp = torch.full((rows,), float(temperature), dtype=torch.float32, device=dev)
-    out = torch.empty(rows, vocab, dtype=torch.float32, device=dev)
-    check(lib().pkv_scale_logits(logits.data_ptr(), logits.stride(0), rows, vocab, dtype_code(logits.dtype),
-                                 pen_ptr, pen_stride, slots, rows_ptr, temp.data_ptr() if temp is not None else None,
-                                 out.data_ptr(), out.stride(0), stream_ptr(dev)), "scale_logits")
-    return out
+    return ((logits.data_ptr(), logits.stride(0), rows, vocab, dtype_code(logits.dtype), pen_ptr, pen_stride, slots,
+             rows_ptr, temp.data_ptr() if temp is not None else None), (penalty_rows, temp))

@@ -413,6 +413,16 @@ int pkv_scale_logits(const void* logits, int64_t row_stride, int32_t rows, int32
                      const int32_t* penalty_rows, const float* temperature, float* out, int64_t out_stride,
                      void* stream);
 
+/* pkv_scale_logits into scaled (float32, rows of scaled_stride floats: a scratch area), then
+ * pkv_top_k_top_p_sampling_ws on it, with the scaling done in the sampler's first pass (where the
+ * workspace suffices and scaled's rows are 16-byte aligned; else as two calls).  Tokens as by the two. */
+int pkv_scaled_top_k_top_p_sampling(const void* logits, int64_t row_stride, int32_t rows, int32_t vocab, int32_t dtype,
+                                    const void* penalty, int64_t penalty_stride, int32_t penalty_slots,
+                                    const int32_t* penalty_rows, const float* temperature, float* scaled,
+                                    int64_t scaled_stride, const int32_t* top_k, int32_t top_k_all,
+                                    const float* top_p, float top_p_all, const float* uniform, int32_t* out,
+                                    void* workspace, int64_t workspace_bytes, void* stream);
+
 /* A measurement helper with no counterpart in the reference: reads `bytes` of device memory at
  * src (16-byte aligned, a multiple of 16 bytes) with `blocks` workgroups of 1024 threads, each
  * workgroup a contiguous slice, with 16-byte non-temporal loads; *sink (device, 4 bytes) may be

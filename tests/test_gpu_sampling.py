@@ -338,3 +338,50 @@ def test_top_k_split_path_graph_replays():
         for r in range(16):
             assert sr.kept_set(xs[r], 50, 0.9)[int(d[r])]
     assert len(set(seen)) > 1
+
+
+@pytest.mark.parametrize("dtype,vocab", [(torch.float16, 151936), (torch.bfloat16, 32003), (torch.float32, 20000),
+                                         (torch.float16, 2049), (torch.float32, 7), (torch.bfloat16, 600011)])
+def test_top_p_split_path_equals_single_workgroup(dtype, vocab):
+    """Top-p rows run over many workgroups through bins of mass; the token must be the one-workgroup
+    kernel's, bit for bit, whatever the logits' spread: peaked, flat, tied (more candidates than a slice
+    holds: handed back), masked, NaN, infinite, sorted.  Mixed with the other kinds in one call, and
+    through the fused scaling."""
+    from ecahlang_amd.sampling import scale_logits
+
+    rows = 24 if vocab < 500000 else 12
+    g = torch.Generator().manual_seed(vocab + 2)
+    x = (torch.randn(rows, vocab, generator=g) * 3).to(dtype)
+    x[1] = torch.round(x[1])
+    x[2] = 0.5
+    x[3, : vocab - 3] = float("nan")
+    x[4, vocab // 3] = 60.0
+    x[5, : vocab // 2] = float("-inf")
+    x[6] = x[6].sort(descending=True).values
+    x[7] = (torch.randn(vocab, generator=g) * 0.05).to(dtype)
+    x[8] = float("nan")
+    x[9, 2] = float("inf")
+    x[10] = -0.0
+    x[10, ::2] = 0.0
+    x[11] = (torch.randn(vocab, generator=g) * 40).to(dtype)
+    x = x.to(DEV)
+    ps = torch.tensor([0.9, 0.95, 0.5, 0.9, 0.99, 0.9, 0.8, 0.9, 0.5, 0.9, 0.5, 0.999] * 2, dtype=torch.float32)[:rows].to(DEV)
+    for trial in range(2):
+        u = torch.rand(rows, generator=g).to(DEV)
+        for p in (ps, 0.9, 0.0, 1e-6, 0.9999999):
+            got, want = sample(x, 0, p, uniform=u), _single_wg(x, 0, p, u)
+            torch.cuda.synchronize()
+            assert torch.equal(got, want), (trial, p, (got != want).nonzero().flatten().tolist())
+    ks = torch.tensor([0, 50, 256, 300, 0, 1, 100, 0, 5, 0, 200, 0] * 2, dtype=torch.int32)[:rows].to(DEV)
+    mixed = torch.where(torch.arange(rows, device=DEV) % 5 == 4, torch.ones_like(ps), ps)
+    table = torch.ones(rows + 1, vocab, dtype=dtype, device=DEV)
+    table[:, ::7] = 1.25
+    slots = torch.arange(rows, dtype=torch.int32, device=DEV)
+    slots[3] = rows + 1  # no such penalty row
+    temp = torch.linspace(0.5, 1.5, rows, device=DEV)
+    got, want = sample(x, ks, mixed, uniform=u), _single_wg(x, ks, mixed, u)
+    y = scale_logits(x, table, slots, temp)
+    got2, want2 = sample(x, ks, mixed, uniform=u, penalty=table, penalty_rows=slots, temperature=temp), _single_wg(y, ks, mixed, u)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and torch.equal(got2, want2)
+    assert got2[3].item() == -1
