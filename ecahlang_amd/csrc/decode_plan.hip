@@ -6,8 +6,7 @@
 // synchronises and the step's page table can be rebuilt on the device right before it (also
 // inside a captured graph).
 //
-// First phase (decode_plan_kernel, one workgroup of 1024 threads; every loop strides over the
-// batch):
+// First phase (decode_plan_kernel, one workgroup; every loop strides over the batch):
 //  1. total = min(kv_indptr[B], num_indices), first = kv_indptr[0]; sequence b owns pages
 //     [s0, s1) = kv_indptr[b .. b+1] clipped to [first, total).  An exclusive scan of (s1 > s0)
 //     gives each non-empty sequence its rank; sequences with no page are listed.
@@ -79,9 +78,10 @@ struct Targets {
   }
 };
 
-// Block-wide exclusive scan of v (all 1024 threads call it); `carry` holds the sum of the
+// Block-wide exclusive scan of v (all NT threads call it; sync: their barrier); `carry` holds the sum of the
 // earlier rounds and is advanced by this round's total (the same in every thread).
-__device__ __forceinline__ int block_scan(int v, int& carry, int* s_wsum) {
+template <int NT, typename Sync>
+__device__ __forceinline__ int block_scan(int v, int& carry, int* s_wsum, Sync&& sync) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   int x = v;
 #pragma unroll
@@ -90,41 +90,71 @@ __device__ __forceinline__ int block_scan(int v, int& carry, int* s_wsum) {
     x += lane >= off ? y : 0;
   }
   if (lane == 63) s_wsum[wv] = x;
-  __syncthreads();
+  sync();
   int off = 0, blk = 0;
 #pragma unroll
-  for (int k = 0; k < kPlanThreads / 64; ++k) {
+  for (int k = 0; k < NT / 64; ++k) {
     off += k < wv ? s_wsum[k] : 0;
     blk += s_wsum[k];
   }
   const int ex = carry + off + x - v;
   carry += blk;
-  __syncthreads();  // s_wsum is rewritten by the next call
+  sync();  // s_wsum is rewritten by the next call
   return ex;
 }
 
-__global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(PlanParams P) {
-  __shared__ int s_total, s_first, s_nempty, s_bad;
+// SMALL (at most NT sequences and SL ranges): the per-sequence, per-run and per-range scratch stays in
+// LDS until it is written out at the end, and barriers wait for LDS alone.  Through memory, every
+// exchange is a round trip and every barrier waits for the stores before it.  A whole plan, both phases
+// in a graph, at 4 to 256 sequences: 18.2 us with 1024 threads and the scratch in memory, 13.4 us; this
+// kernel 14.2 and 9.2 in a trace.  (256 threads: the line is where the serving loop's batches end.)
+template <int NT, int SL, bool SMALL>
+__global__ __launch_bounds__(NT) void decode_plan_kernel(PlanParams P) {
+  constexpr int kPlanThreads = NT, kStartsLds = SL;
+  __shared__ int s_seq[SMALL ? 9 : 1][SMALL ? NT : 1], s_run[SMALL ? 5 : 1][SMALL ? NT : 1];
+  __shared__ int s_bf[SMALL ? SL : 1], s_nzb[SMALL ? SL + 1 : 1];
+  int* const g_rank = SMALL ? s_seq[0] : P.rank;
+  int* const g_swin = SMALL ? s_seq[SMALL ? 1 : 0] : P.swin;
+  int* const g_ss = SMALL ? s_seq[SMALL ? 2 : 0] : P.ss;
+  int* const g_sp = SMALL ? s_seq[SMALL ? 3 : 0] : P.sp;
+  int* const g_sl = SMALL ? s_seq[SMALL ? 4 : 0] : P.sl;
+  int* const g_npb = SMALL ? s_seq[SMALL ? 5 : 0] : P.npb;
+  int* const g_sbase = SMALL ? s_seq[SMALL ? 6 : 0] : P.sbase;
+  int* const g_runof = SMALL ? s_seq[SMALL ? 7 : 0] : P.runof;
+  int* const g_lcp = SMALL ? s_seq[SMALL ? 8 : 0] : P.lcp;
+  int* const g_run_r0 = SMALL ? s_run[0] : P.run_r0;
+  int* const g_run_p = SMALL ? s_run[SMALL ? 1 : 0] : P.run_p;
+  int* const g_run_c = SMALL ? s_run[SMALL ? 2 : 0] : P.run_c;
+  int* const g_run_np = SMALL ? s_run[SMALL ? 3 : 0] : P.run_np;
+  int* const g_run_i0 = SMALL ? s_run[SMALL ? 4 : 0] : P.run_i0;
+  int* const g_bf = SMALL ? s_bf : P.bf;
+  int* const g_nzb = SMALL ? s_nzb : P.nzb;
+  auto sync = [&]() __attribute__((always_inline)) {
+    if constexpr (SMALL) lds_barrier();
+    else __syncthreads();
+  };
+  __shared__ int s_nempty, s_bad;
   __shared__ int s_wsum[kPlanThreads / 64];
   __shared__ unsigned long long s_xt;
   __shared__ int s_starts[kStartsLds + 1];
   __shared__ int64_t s_tgt[kStartsLds + 1];
   const int tid = threadIdx.x, lane = tid & 63;
   const int B = P.batch;
+  // (each thread's sequence is requested with the totals: one round trip)
+  const int mine = tid < B ? tid : B - 1;
+  const int raw0 = P.indptr[mine], raw1 = P.indptr[mine + 1], rawp = P.indptr[mine > 0 ? mine - 1 : 0];
+  int64_t t64 = P.indptr[B];
+  t64 = t64 < P.num_indices ? t64 : P.num_indices;
+  t64 = t64 > 0 ? t64 : 0;
+  int64_t f64 = P.indptr[0];
+  f64 = f64 < 0 ? 0 : (f64 > t64 ? t64 : f64);
+  const int total = (int)t64, first = (int)f64;
   if (tid == 0) {
-    int64_t t = P.indptr[B];
-    t = t < P.num_indices ? t : P.num_indices;
-    t = t > 0 ? t : 0;
-    int64_t f = P.indptr[0];
-    f = f < 0 ? 0 : (f > t ? t : f);
-    s_total = (int)t;
-    s_first = (int)f;
     s_nempty = 0;
     s_bad = 0;
     s_xt = 0;
   }
-  __syncthreads();
-  const int total = s_total, first = s_first;
+  sync();
   auto clip = [&](int64_t x) -> int { return (int)(x < first ? first : (x > total ? total : x)); };
   const bool hint = P.shared != nullptr;
   const bool group = hint && P.cascade && P.group >= 2;
@@ -135,10 +165,10 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(PlanParams P)
     const int b = base + tid;
     int s0 = 0, s1 = 0, lc = 0;
     if (b < B) {
-      s0 = clip(P.indptr[b]);
-      s1 = clip(P.indptr[b + 1]);
+      s0 = clip(base == 0 ? raw0 : P.indptr[b]);
+      s1 = clip(base == 0 ? raw1 : P.indptr[b + 1]);
       if (hint && b > 0) {
-        const int p0 = clip(P.indptr[b - 1]);
+        const int p0 = clip(base == 0 ? rawp : P.indptr[b - 1]);
         // each keeps its own the pages that can receive the step's token: its last page, and the
         // one before it when the last is empty (kv_last_page_len 0)
         const int cap = min(s1 - s0 - (P.last[b] > 0 ? 1 : 2), s0 - p0 - (P.last[b - 1] > 0 ? 1 : 2));
@@ -149,28 +179,28 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(PlanParams P)
     const bool ne = b < B && s1 > s0;
     const bool link = b < B && lc >= kPrefixMinPages;
     const bool head = b < B && !link;
-    const int rk = block_scan(ne ? 1 : 0, nne, s_wsum);
-    const int rid = block_scan(head ? 1 : 0, nruns, s_wsum) - (head ? 0 : 1);
+    const int rk = block_scan<NT>(ne ? 1 : 0, nne, s_wsum, sync);
+    const int rid = block_scan<NT>(head ? 1 : 0, nruns, s_wsum, sync) - (head ? 0 : 1);
     if (b < B) {
-      P.rank[b] = rk;
-      P.runof[b] = rid;
-      P.lcp[b] = link ? lc : 0;
+      g_rank[b] = rk;
+      g_runof[b] = rid;
+      g_lcp[b] = link ? lc : 0;
       if (head) {
-        P.run_r0[rid] = b;
-        P.run_p[rid] = kNone;
+        g_run_r0[rid] = b;
+        g_run_p[rid] = kNone;
       }
       if (!ne) P.ghdr[kGlobHdr + atomicAdd(&s_nempty, 1)] = b;
     }
   }
-  __syncthreads();
+  sync();
 
   // ---- 2b: each run's shared pages, the minimum hint over its linked members (a segmented
   // minimum inside each wave, then one atomic per piece of a run)
   if (hint) {
     for (int base = 0; base < B; base += kPlanThreads) {
       const int b = base + tid;
-      int v = b < B && P.lcp[b] > 0 ? P.lcp[b] : kNone;
-      const int rid = b < B ? P.runof[b] : -1;
+      int v = b < B && g_lcp[b] > 0 ? g_lcp[b] : kNone;
+      const int rid = b < B ? g_runof[b] : -1;
 #pragma unroll
       for (int off = 1; off < 64; off <<= 1) {
         const int y = __shfl_up(v, off, 64);
@@ -179,9 +209,9 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(PlanParams P)
       }
       const int rn = __shfl_down(rid, 1, 64);
       const bool tail = lane == 63 || rn != rid;
-      if (b < B && tail && v != kNone) atomicMin(&P.run_p[rid], v);
+      if (b < B && tail && v != kNone) atomicMin(&g_run_p[rid], v);
     }
-    __syncthreads();
+    sync();
   }
 
   // ---- 2c: chunks and items of each run
@@ -194,9 +224,9 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(PlanParams P)
     if (r < nruns) {
       int pp = 0, np = 0, c = 0;
       if (hint) {
-        const int r0 = P.run_r0[r];
-        const int size = (r + 1 < nruns ? P.run_r0[r + 1] : B) - r0;
-        pp = size >= 2 ? P.run_p[r] : 0;
+        const int r0 = g_run_r0[r];
+        const int size = (r + 1 < nruns ? g_run_r0[r + 1] : B) - r0;
+        pp = size >= 2 ? g_run_p[r] : 0;
         pp = pp == kNone ? 0 : pp;  // (kept as the run's shared pages even when not grouping)
         if (pp > 0 && group) {
           np = (pp + kPrefixChunkMin - 1) / kPrefixChunkMin;
@@ -213,16 +243,16 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(PlanParams P)
             ((unsigned long long)c * kPrefixCostNum + kPrefixCostDen - 1) / kPrefixCostDen + kPrefixItemFixed;
         xt = (unsigned long long)items * x;
       }
-      P.run_p[r] = pp;
-      P.run_np[r] = np;
-      P.run_c[r] = c;
+      g_run_p[r] = pp;
+      g_run_np[r] = np;
+      g_run_c[r] = c;
     }
-    const int i0 = block_scan(items, nitems, s_wsum);
-    if (r < nruns) P.run_i0[r] = i0;
-    block_scan(parts, nparts, s_wsum);
+    const int i0 = block_scan<NT>(items, nitems, s_wsum, sync);
+    if (r < nruns) g_run_i0[r] = i0;
+    block_scan<NT>(parts, nparts, s_wsum, sync);
     if (xt) atomicAdd(&s_xt, xt);
   }
-  __syncthreads();
+  sync();
   // The cascade must fit: one carrier range per item, and a partial slot for every chunk of
   // every grouped sequence beside the suffix ranges' R + B.
   const bool casc = group && nitems > 0 && nitems <= P.r_cap &&
@@ -236,25 +266,25 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(PlanParams P)
     const int b = base + tid;
     int s0 = 0, s1 = 0, pp = 0, np = 0, shp = 0;
     if (b < B) {
-      s0 = clip(P.indptr[b]);
-      s1 = clip(P.indptr[b + 1]);
+      s0 = clip(base == 0 ? raw0 : P.indptr[b]);
+      s1 = clip(base == 0 ? raw1 : P.indptr[b + 1]);
       if (hint) {
-        const int r = P.runof[b];
-        shp = P.run_p[r];
+        const int r = g_runof[b];
+        shp = g_run_p[r];
         if (casc) {
-          np = P.run_np[r];
+          np = g_run_np[r];
           pp = np > 0 ? shp : 0;
         }
       }
     }
     const int len = s1 > s0 ? s1 - s0 - pp : 0;
-    const int pos = block_scan(len, ns, s_wsum);
+    const int pos = block_scan<NT>(len, ns, s_wsum, sync);
     if (b < B) {
-      P.ss[b] = s0 + pp;
-      P.sl[b] = len;
-      P.sp[b] = pos;
-      P.npb[b] = np;
-      P.lcp[b] = s0 + shp;  // end of the pages b shares with its run (kv_indices position)
+      g_ss[b] = s0 + pp;
+      g_sl[b] = len;
+      g_sp[b] = pos;
+      g_npb[b] = np;
+      g_lcp[b] = s0 + shp;  // end of the pages b shares with its run (kv_indices position)
     }
   }
 
@@ -267,9 +297,9 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(PlanParams P)
   }
   R = R > Rp ? R : Rp;
   R = R < P.r_cap ? R : P.r_cap;  // (the host sized r_cap for num_indices >= ns, and Rp <= r_cap)
-  int* starts = R <= kStartsLds ? s_starts : P.starts;
-  for (int w = tid; w < P.r_cap; w += kPlanThreads) P.bf[w] = -1;
-  __syncthreads();
+  int* starts = SMALL || R <= kStartsLds ? s_starts : P.starts;
+  for (int w = tid; w < P.r_cap; w += kPlanThreads) g_bf[w] = -1;
+  sync();
   // Sequence k (in rank order) covers weights [W0 - c, W0 + len) with W0 = pos + c * k (the
   // first part is the gap before its start); range w starts where weight tgt(w) falls.  If a
   // range comes out over kRangePages pages, the plain equal split is used.
@@ -278,19 +308,19 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(PlanParams P)
     const Targets T((int64_t)ns + (int64_t)c * (nne > 0 ? nne - 1 : 0), pass == 0 ? XT : 0, R, Rp);
     // every range's start weight, computed once (a thread each: three 64-bit divisions) for the
     // searches below, when it fits in LDS
-    const bool tab = R <= kStartsLds;
+    const bool tab = SMALL || R <= kStartsLds;
     // (every range starts out empty at the list's end: with more than half the ranges carrying
     // items that outweigh their share, the last ones are carriers whose target is the whole
     // weight, which no sequence's search below covers)
     for (int w = tid; w < R; w += kPlanThreads) starts[w] = ns;
     if (tab)
       for (int w = tid; w <= R; w += kPlanThreads) s_tgt[w] = T.tgt(w);
-    __syncthreads();
+    sync();
     auto tgt_at = [&](int w) -> int64_t { return tab ? s_tgt[w] : T.tgt(w); };
     for (int b = tid; b < B; b += kPlanThreads) {
-      const int len = P.sl[b];
+      const int len = g_sl[b];
       if (len <= 0) continue;
-      const int k = P.rank[b], pos = P.sp[b];
+      const int k = g_rank[b], pos = g_sp[b];
       const int64_t w0 = (int64_t)pos + (int64_t)c * k;
       const int64_t lo = k == 0 ? 0 : w0 - c, hi = w0 + len;
       int wl = 0, wh = R;  // smallest w in [0, R] with tgt(w) >= lo
@@ -302,18 +332,18 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(PlanParams P)
         const int64_t tw = tgt_at(w);
         if (tw >= hi) break;
         starts[w] = tw < w0 ? pos : (int)(pos + (tw - w0));
-        P.bf[w] = b;
+        g_bf[w] = b;
       }
     }
     if (tid == 0) starts[R] = ns;
-    __syncthreads();
+    sync();
     for (int w = tid; w < R; w += kPlanThreads) {
       const int len = starts[w + 1] - starts[w];
       if (len < 0 || len > kRangePages) s_bad = 1;
     }
-    __syncthreads();
+    sync();
     if (!s_bad) break;
-    __syncthreads();  // every thread has read s_bad before it is cleared
+    sync();  // every thread has read s_bad before it is cleared
     if (tid == 0) s_bad = 0;
   }
   // range holding suffix position p (largest w with starts[w] <= p: empty ranges are skipped)
@@ -330,29 +360,50 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(PlanParams P)
   int nnz = 0;
   for (int base = 0; base <= R; base += kPlanThreads) {
     const int w = base + tid;
-    const int ex = block_scan(w < R && starts[w + 1] > starts[w] ? 1 : 0, nnz, s_wsum);
-    if (w <= R) P.nzb[w] = ex;
+    const int ex = block_scan<NT>(w < R && starts[w + 1] > starts[w] ? 1 : 0, nnz, s_wsum, sync);
+    if (w <= R) g_nzb[w] = ex;
   }
-  __syncthreads();
+  sync();
   int nslots = 0;
   for (int base = 0; base < B; base += kPlanThreads) {
     const int b = base + tid;
     int parts = 0;
     if (b < B) {
-      const int len = P.sl[b];
+      const int len = g_sl[b];
       if (len > 0) {
-        const int pos = P.sp[b];
+        const int pos = g_sp[b];
         const int wlo = owner(pos), whi = owner(pos + len - 1);
-        P.swin[b] = wlo | (whi << 16);
-        parts = P.npb[b] + P.nzb[whi] - P.nzb[wlo] + 1;
+        g_swin[b] = wlo | (whi << 16);
+        parts = g_npb[b] + g_nzb[whi] - g_nzb[wlo] + 1;
       } else {
-        P.swin[b] = -1;
+        g_swin[b] = -1;
       }
     }
-    const int sb = block_scan(parts, nslots, s_wsum);
-    if (b < B) P.sbase[b] = sb;
+    const int sb = block_scan<NT>(parts, nslots, s_wsum, sync);
+    if (b < B) g_sbase[b] = sb;
   }
-  if (starts != P.starts)
+  if constexpr (SMALL) {
+    if (tid < B) {  // (its own entries; a run's come from its thread)
+      P.rank[tid] = g_rank[tid];
+      P.swin[tid] = g_swin[tid];
+      P.ss[tid] = g_ss[tid];
+      P.sp[tid] = g_sp[tid];
+      P.sl[tid] = g_sl[tid];
+      P.npb[tid] = g_npb[tid];
+      P.sbase[tid] = g_sbase[tid];
+      P.lcp[tid] = g_lcp[tid];
+    }
+    if (tid < nruns) {
+      P.run_r0[tid] = g_run_r0[tid];
+      P.run_p[tid] = g_run_p[tid];
+      P.run_c[tid] = g_run_c[tid];
+      P.run_np[tid] = g_run_np[tid];
+      P.run_i0[tid] = g_run_i0[tid];
+    }
+    for (int w = tid; w < P.r_cap; w += NT) P.bf[w] = g_bf[w];
+    for (int w = tid; w <= R; w += NT) P.nzb[w] = g_nzb[w];
+  }
+  if (SMALL || starts != P.starts)
     for (int w = tid; w <= R; w += kPlanThreads) P.starts[w] = starts[w];
   if (tid == 0) {
     P.ghdr[kGhRanges] = R;
@@ -548,7 +599,10 @@ int decode_plan_launch(const int32_t* indptr, const int32_t* indices, int64_t nu
   P.rank = a[0]; P.swin = a[1]; P.ss = a[2]; P.sp = a[3]; P.sl = a[4]; P.npb = a[5];
   P.sbase = a[6]; P.runof = a[7]; P.lcp = a[8];
   P.run_r0 = a[9]; P.run_p = a[10]; P.run_c = a[11]; P.run_np = a[12]; P.run_i0 = a[13];
-  hipLaunchKernelGGL(decode_plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, P);
+  if (batch <= 256 && r_cap <= 1024)
+    hipLaunchKernelGGL((decode_plan_kernel<256, 1024, true>), dim3(1), dim3(256), 0, s, P);
+  else
+    hipLaunchKernelGGL((decode_plan_kernel<kPlanThreads, kStartsLds, false>), dim3(1), dim3(kPlanThreads), 0, s, P);
   hipLaunchKernelGGL(decode_plan_records_kernel, dim3(r_cap), dim3(kRecThreads), 0, s, P);
   return (int)hipGetLastError();
 }

@@ -99,3 +99,18 @@ def test_schedule_of_edge_tables(k, geom):
     n_idx = int(indptr[-1]) - c.get("cut", 0)
     hq, hkv, d, dt = geom
     _plan_check(indptr, indices, last, hq, hkv, d, dt, ctas=c["R"], num_indices=n_idx)
+
+
+@pytest.mark.parametrize("B,ctas", [(1, 256), (255, 256), (256, 256), (257, 256), (256, 1024), (200, 1025), (256, 1)])
+@pytest.mark.parametrize("hinted", [True, False])
+def test_schedule_at_the_small_plan_kernel_limits(B, ctas, hinted):
+    """Up to 256 sequences and 1024 ranges the plan's scratch stays in LDS: one below, at and above the
+    limits, empty sequences among the rest, with and without shared prefixes."""
+    rng = np.random.default_rng(7 * B + ctas)
+    if hinted:
+        ip, idx, lt, hint = _shared_prefix_table(rng, B=B, prefix_pages=20, lo=16, hi=400)
+        _plan_check(ip, idx, lt, 16, 2, 128, torch.float16, ctas=ctas, hint=hint)
+    else:
+        lens = [0 if b % 7 == 3 else int(L) for b, L in enumerate(rng.integers(1, 500, size=B))]
+        indptr, indices, last = _table(rng, lens, None, 0, bad_ids=0)
+        _plan_check(indptr, indices, last, 32, 8, 128, torch.bfloat16, ctas=ctas, num_indices=int(indptr[-1]))
