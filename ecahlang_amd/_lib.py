@@ -135,4 +135,7 @@ def dtype_code(dt: torch.dtype) -> int:
 
 
 def stream_ptr(device: torch.device | None = None) -> int:
+    # (the raw handle, without a Stream object around it: 0.2 us instead of 1.5)
+    if isinstance(device, torch.device) and device.index is not None and device.type == "cuda":
+        return torch._C._cuda_getCurrentRawStream(device.index)
     return torch.cuda.current_stream(device).cuda_stream

@@ -56,7 +56,7 @@ class CacheView:
                 raise ValueError("paged_kv_cache must be contiguous")
             self.num_pages, _, self.page_size, self.num_kv_heads, self.head_dim = c.shape
             self.k_ptr = c.data_ptr()
-            self.v_ptr = c[:, 1].data_ptr()
+            self.v_ptr = self.k_ptr + c.stride(1) * c.element_size() if self.k_ptr else 0
             self.page_stride = c.stride(0)
             self.dtype, self.device = c.dtype, c.device
         if not (self.device.type == "cuda"):

@@ -15,6 +15,7 @@ keep that call shape:
 from __future__ import annotations
 
 
+import functools
 import math
 import os
 
@@ -38,6 +39,7 @@ def _as_dtype(d) -> torch.dtype:
         raise ValueError(f"unsupported data type {d!r}") from None
 
 
+@functools.lru_cache(maxsize=64)
 def _num_cus(device: torch.device) -> int:
     return torch.cuda.get_device_properties(device).multi_processor_count
 
