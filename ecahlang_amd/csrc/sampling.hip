@@ -344,8 +344,9 @@ constexpr int kMaxSplitTiles = 2048;           // vocabularies up to 4 M
 constexpr int kCandCap = 512;    // candidates a slice hands over for a top-p row
 
 constexpr int kGroups = 1024;    // group maxima per row at most
-constexpr int kPBins = 512;      // bins of a top-p row's mass
-constexpr int kPCandMax = 1024;  // candidates of a top-p row
+constexpr int kPBins = 1024;     // bins of a top-p row's mass
+constexpr int kPCandMax = 2048;  // candidates of a top-p row (at 512 bins and 1024 of them, a wide body at a high
+                                 // temperature went over, and the one row handed back took 45 us)
 
 __host__ __device__ inline int split_tiles(int vocab) { return (vocab + kSplitTile - 1) / kSplitTile; }
 __host__ __device__ inline int split_slices(int vocab) { return (split_tiles(vocab) + kSliceTiles - 1) / kSliceTiles; }
@@ -867,16 +868,16 @@ __device__ __forceinline__ void topp_hist(const T* p, int vocab, bool vec, const
   uint64_t* h = ws.hist + (int64_t)b * S * kPBins;
   for (int i = t; i < kPBins; i += kSplitThreads) st_dev_u64(h + (int64_t)s * kPBins + i, s_hist[i]);
   if (!slice_arrive(&ws.counter[b * kCountStride], S, s_last)) return;
-  // ---- the bin that holds the threshold; thread t: bins 2t, 2t + 1
-  static_assert(kPBins == 2 * kSplitThreads, "two bins a thread");
-  uint64_t h0 = 0, h1 = 0;
-#pragma unroll 8
-  for (int i = 0; i < S; ++i) {
-    h0 += ld_dev(h + (int64_t)i * kPBins + 2 * t);
-    h1 += ld_dev(h + (int64_t)i * kPBins + 2 * t + 1);
-  }
+  // ---- the bin that holds the threshold; thread t: bins 4t .. 4t + 3
+  static_assert(kPBins == 4 * kSplitThreads, "four bins a thread");
+  uint64_t hb[4] = {0, 0, 0, 0};
+#pragma unroll 4
+  for (int i = 0; i < S; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) hb[e] += ld_dev(h + (int64_t)i * kPBins + 4 * t + e);
+  const uint64_t own = hb[0] + hb[1] + hb[2] + hb[3];
   uint64_t mk;
-  const uint64_t incl = block_scan256(h0 + h1, redu, mk), excl = incl - h0 - h1;
+  const uint64_t incl = block_scan256(own, redu, mk), excl = incl - own;
   const double needd = ceil((double)fmaxf(pp, 0.f) * (double)mk);
   uint64_t need = needd < 1.0 ? 1 : (uint64_t)needd;
   if (need > mk) need = mk;
@@ -887,14 +888,21 @@ __device__ __forceinline__ void topp_hist(const T* p, int vocab, bool vec, const
       out[b] = -1;
     }
   } else if (incl >= need && excl < need) {
-    const bool lo = excl + h0 >= need;
-    ws.bin[b] = ToppBin{lo ? excl : excl + h0, need, bins.mx, bins.scale, lo ? 2 * t : 2 * t + 1};
+    uint64_t above = excl;
+    int e = 0;
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+      const bool on = e == x && above + hb[x] < need;
+      above += on ? hb[x] : 0;
+      e += on ? 1 : 0;
+    }
+    ws.bin[b] = ToppBin{above, need, bins.mx, bins.scale, 4 * t + e};
   }
 }
 
 struct ToppLds {
   uint64_t cand[kPCandMax];
-  uint64_t mass[kPCandMax];
+  uint64_t mass[kSplitThreads];  // (of up to 256 candidates)
   uint64_t hist[kSplitThreads];
   uint64_t redu[4], tsum[kSliceTiles][4];
   uint64_t above;
@@ -995,7 +1003,7 @@ __device__ __forceinline__ void topp_finish(const T* p, int vocab, int s, int b,
     }
     const uint64_t c = ld_dev(ws.cand + ((int64_t)b * S + lo) * kCandCap + (i - L.off[lo]));
     L.cand[i] = c;
-    L.mass[i] = fmass(key_float((uint32_t)c), bins.mx);
+    if (n <= kSplitThreads) L.mass[i] = fmass(key_float((uint32_t)c), bins.mx);
   }
   if (t == 0) L.thr = 0;
   __syncthreads();
@@ -1033,7 +1041,7 @@ __device__ __forceinline__ void topp_finish(const T* p, int vocab, int s, int b,
         const uint32_t key = (uint32_t)L.cand[i];
         if ((key & himask) == (thr & himask))
           atomicAdd((unsigned long long*)&L.hist[(key >> shift) & (nb - 1u)],
-                    (unsigned long long)L.mass[i]);
+                    (unsigned long long)fmass(key_float(key), bins.mx));
       }
       __syncthreads();
       const uint64_t own = L.hist[kSplitThreads - 1 - t];  // (from the largest digit down)
@@ -1052,7 +1060,7 @@ __device__ __forceinline__ void topp_finish(const T* p, int vocab, int s, int b,
     const uint64_t c = L.cand[i];
     if ((uint32_t)c >= thr)
       atomicAdd((unsigned long long*)&s_tile[(uint32_t)(c >> 32) / kSplitTile],
-                (unsigned long long)L.mass[i]);
+                (unsigned long long)fmass(key_float((uint32_t)c), bins.mx));
   }
   __syncthreads();
   pick_token(p, vocab, vec, bins.mx, thr, s_tile, ntiles, uniform[b], out + b, L.redu, &L.at);

@@ -391,9 +391,9 @@ int pkv_top_k_top_p_sampling(const void* logits, int64_t row_stride, int32_t row
 int64_t pkv_sampling_workspace_bytes(int32_t rows, int32_t vocab);
 
 /* pkv_top_k_top_p_sampling with a workspace (8-byte aligned, workspace_bytes >=
- * pkv_sampling_workspace_bytes): rows sampled from their whole distribution (top_k <= 0 or
- * >= vocab and top_p >= 1, the serving loop's default request) are then spread over many
- * workgroups per row instead of one.  Same tokens, bit for bit; the workspace needs no
+ * pkv_sampling_workspace_bytes): rows without a filter (the serving loop's default request), with a
+ * top-p filter alone or with a top-k filter of k <= 256 are then read by many workgroups each instead
+ * of one.  Same tokens, bit for bit; the workspace needs no
  * initialisation (its counters are reset by the call itself). */
 int pkv_top_k_top_p_sampling_ws(const void* logits, int64_t row_stride, int32_t rows, int32_t vocab,
                                 int32_t dtype, const int32_t* top_k, int32_t top_k_all, const float* top_p,
