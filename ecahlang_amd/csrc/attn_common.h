@@ -78,7 +78,8 @@ __device__ __forceinline__ Prm uniform_params(const Prm& arg, int* lds_words) {
 // so no line holds two slots.  The merger of a sequence reads its slots with plain loads; were a
 // line shared with another sequence's slot, that load could bring the other slot's line into
 // this XCD's L2 before its writer (on another XCD) stored it, and the other sequence's merger
-// on this XCD would then read the stale copy.
+// on this XCD would then read the stale copy.  (A merge per KV head, decode_f32.hip, has several
+// mergers on one line: they load it with ld_dev2.)
 constexpr int kLineBytes = 128;
 __host__ __device__ __forceinline__ int ml_slot_stride(int hq) {
   constexpr int per = kLineBytes / 8;  // float2 entries per line
@@ -126,9 +127,16 @@ __device__ __forceinline__ int seq_len_of(const DecodeParams& P, int b) {
 //  * the last arriver then reads them with plain loads: no L2 on its XCD has held those
 //    lines since the kernel began (each partial slot is read once, by that merger only,
 //    and caches start the kernel invalidated), so the loads fetch the written values, and
-//    being plain they can all be in flight at once.
+//    being plain they can all be in flight at once.  Where a line has several mergers, the
+//    first one's load may leave a copy behind that lacks what others store later, so there
+//    every merger loads at device scope (ld_dev2), past that copy.
 __device__ __forceinline__ void st_dev(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// A (max, sum) pair read at device scope: never served from a copy in this CU's or this XCD's caches.
+__device__ __forceinline__ float2 ld_dev2(const float2* p) {
+  const uint64_t u = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return make_float2(__uint_as_float((uint32_t)u), __uint_as_float((uint32_t)(u >> 32)));
 }
 // 16-byte device-scope (write-through, sc1) vector store: the same effect as four st_dev,
 // issued as a buffer store with the sc1 cache policy so the compiler still tracks its

@@ -282,8 +282,10 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 4 : 2) void decode_f32_kernel(Dec
   if (!arrive_last(P, head_counters ? b * P.hkv + h : b, head_counters ? nparts : nparts * P.hkv, &s_last)) return;
 
   // ---- merge of the sequence's parts, for this KV head or (one counter a sequence) for all: four dims
-  // of one head a lane, the parts shared by NW waves, the rows of kMergeParts parts requested at once
-  // and folded under a running max (a part without mass holds zeros; repeats weigh nothing)
+  // of one head a lane, the parts shared by nw waves, the rows of kMergeParts parts requested at once
+  // and folded under a running max (a part without mass holds zeros; repeats weigh nothing).  With head
+  // counters a line of (max, sum) pairs has a reader per KV head, so the pairs are loaded past the
+  // caches (ld_dev2); a head's partial rows are whole lines of its own.
   const int x0 = head_counters ? h * g * (D / 4) : 0, nx = (head_counters ? g : P.hq) * (D / 4);
   const int groups = (nx + 63) / 64, nw = groups >= W ? 1 : W / groups;  // waves a group of 64 items
   const int share = (nparts + nw - 1) / nw;
@@ -306,7 +308,7 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 4 : 2) void decode_f32_kernel(Dec
 #pragma unroll
       for (int q = 0; q < kMergeParts; ++q) {
         const int64_t sl = min(q0 + q, q1 - 1);
-        y[q] = ml[sl * P.ml_stride];
+        y[q] = ld_dev2(ml + sl * P.ml_stride);
         row[q] = *reinterpret_cast<const f4*>(po + sl * P.hq * D);
       }
       float Mn = M2;

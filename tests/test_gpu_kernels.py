@@ -344,6 +344,31 @@ def test_decode_fp32_on_the_matrix_cores(name):
     np.testing.assert_allclose(o.cpu().numpy(), ref, **TOL[torch.float32])
 
 
+@pytest.mark.parametrize("hq,hkv,d", [(12, 6, 64), (16, 16, 64), (12, 12, 64), (32, 16, 128), (40, 40, 64)])
+def test_decode_fp32_split_merge_reads_this_calls_partials(hq, hkv, d):
+    """Every KV head merges its own heads' parts, from (max, sum) lines that several KV heads write: with
+    these head counts, heads whose workgroups share an XCD or a CU.  Other queries and another cache on the
+    same workspace from run to run, whose partial areas start out as NaN, so that a pair of an earlier call
+    (or none) in a merge shows."""
+    lens = [700 + 97 * i for i in range(14)] + [1, 40]
+    batches = [workloads.build_batch(lens, [1] * 16, hq, hkv, d, torch.float32, seed) for seed in (91, 92)]
+    ws = torch.empty(64 << 20, dtype=torch.uint8, device=DEV)
+    w = BatchDecodeWithPagedKVCacheWrapper(ws, "NHD")
+    ws[4 * 8192:].fill_(0xFF)  # (past the counters, which the constructor zeroes)
+    dvs, refs = [], []
+    for scale, wb in zip((1.0, 4.0), batches):
+        wb.q = wb.q * scale  # (other maxima, too)
+        dv = wb.to(DEV)
+        _append_dev(dv)
+        _, vals = _oracle_appended(wb)
+        refs.append(kv_ref.decode(wb.q.numpy(), vals, wb.indptr.numpy(), wb.indices.numpy(), wb.last.numpy(), wb.ps))
+        dvs.append(dv)
+    for turn in range(6):
+        dv, ref = dvs[turn % 2], refs[turn % 2]
+        w.plan(dv.indptr, dv.indices, dv.last, hq, hkv, d, dv.ps, q_data_type=torch.float32)
+        np.testing.assert_allclose(w.run(dv.q, dv.cache).cpu().numpy(), ref, **TOL[torch.float32], err_msg=str(turn))
+
+
 @pytest.mark.parametrize("force_valu", [False, True])
 def test_decode_pages_before_first_sequence(force_valu):
     # kv_indptr[0] > 0: the leading page-list entries belong to no sequence
