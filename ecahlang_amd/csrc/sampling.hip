@@ -1611,6 +1611,9 @@ extern "C" int pkv_scale_logits(const void* logits, int64_t row_stride, int32_t 
   return (int)hipGetLastError();
 }
 
+// Whether sample_kernel takes rows of `vocab` logits of es bytes (a word of LDS per tile).
+static bool row_fits(int32_t vocab, int es) { return (int64_t)vocab <= (int64_t)kMaxTiles * kThreads * (16 / es); }
+
 static int sample_entry(const void* logits, int64_t row_stride, int32_t rows, int32_t vocab, int32_t dtype,
                         const int32_t* top_k, int32_t top_k_all, const float* top_p, float top_p_all,
                         const float* uniform, int32_t* out, void* workspace, int64_t workspace_bytes,
@@ -1618,7 +1621,7 @@ static int sample_entry(const void* logits, int64_t row_stride, int32_t rows, in
   if (rows < 0 || vocab <= 0 || row_stride < vocab || !uniform || !out) return kBadArg;
   if (rows == 0) return kOk;
   const int es = dtype == kF32 ? 4 : 2;
-  if ((int64_t)vocab > (int64_t)kMaxTiles * kThreads * (16 / es)) return kBadArg;
+  if (!row_fits(vocab, es)) return kBadArg;
   hipStream_t s = (hipStream_t)stream;
   if (dtype == kF16)
     return scan_and_sample((const _Float16*)logits, row_stride, rows, vocab, top_k, top_k_all, top_p, top_p_all,
@@ -1667,6 +1670,7 @@ extern "C" int pkv_scaled_top_k_top_p_sampling(const void* logits, int64_t row_s
   if (scaled_stride < vocab || !scaled) return kBadArg;
   if (penalty && (!penalty_rows || penalty_stride < vocab || penalty_slots <= 0)) return kBadArg;
   if (dtype != kF16 && dtype != kBF16 && dtype != kF32) return kBadDType;
+  if (!row_fits(vocab, 4)) return kBadArg;  // (the scaled rows are fp32, whatever the logits)
   const SamplePlan plan(rows, vocab, top_k, top_k_all, top_p, top_p_all, workspace, workspace_bytes);
   if (!plan.split || ((uintptr_t)scaled | (uintptr_t)(scaled_stride * 4)) % 16) {
     const int rc = pkv_scale_logits(logits, row_stride, rows, vocab, dtype, penalty, penalty_stride, penalty_slots,

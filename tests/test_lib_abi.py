@@ -125,3 +125,19 @@ def test_noalloc_decode_refuses_geometry_beyond_its_array():
     rc = L.pkv_batch_decode_noalloc(None, 0, 0, None, None, 0, 0, None, None, 10_000_000, None, 64, 16, 2, 128,
                                     16, 0.1, 256, None, 0, 0, 0, None)
     assert rc == -6
+
+
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+def test_scaled_sampling_refuses_rows_beyond_the_fp32_limit(dtype):
+    # The scaled rows are fp32, whatever the logits' dtype, and the one-workgroup sampler takes 512 tiles
+    # of 4096 of them: a longer vocabulary is refused before anything is enqueued, with a workspace and
+    # without (no device call is made, so this runs on the CPU with pointers that are never read).
+    from ecahlang_amd import _lib
+
+    L = _lib.lib()
+    for vocab in (512 * 4096 + 1, 4 * 1024 * 1024):
+        need = L.pkv_sampling_workspace_bytes(1, vocab)
+        for ws, n in ((4096, need), (None, 0)):
+            rc = L.pkv_scaled_top_k_top_p_sampling(4096, vocab, 1, vocab, dtype, None, 0, 0, None, 4096, 4096,
+                                                   (vocab + 3) // 4 * 4, None, 300, None, 1.0, 4096, 4096, ws, n, None)
+            assert rc == -5, (vocab, ws, rc)
