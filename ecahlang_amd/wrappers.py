@@ -355,12 +355,13 @@ class BatchPrefillWithPagedKVCacheWrapper:
         g = self._hq // self._hkv
         # Shapes that can also run without a work list, on the vector kernel, which reads the table
         # at run time, needs no workspace and can be planned and captured: they do where the work
-        # list cannot be built or kept (plan() while capturing, a workspace too small for it) and
-        # in run() for a captured call or a q of another length than the plan's.
+        # list cannot be built (plan() while capturing, a workspace smaller than it) and in run()
+        # for a captured call or a q of another length than the plan's.  They leave the workspace
+        # untouched: the list is the wrapper's own and a call's partials are that call's, so
+        # wrappers may share a buffer, and plan and runs any streams, as on the vector kernel.
         self._valu_ok = g not in (1, 2, 4, 8, 16) or self._q_dtype == torch.float32
         if self._mfma and self._valu_ok:
-            self._mfma = self._batch > 0 and self._sm_scale > 0 and self._workspace_usable(qo_indptr.device) and \
-                not torch.cuda.is_current_stream_capturing()
+            self._mfma = self._batch > 0 and self._sm_scale > 0 and not torch.cuda.is_current_stream_capturing()
         if self._mfma:
             self._schedule(qo_indptr.device)
         self._planned = True
@@ -368,19 +369,17 @@ class BatchPrefillWithPagedKVCacheWrapper:
     # rows per matrix-core work item (8 waves x 32 rows, fp32 8 x 16): rows / g query tokens of one KV head
     _ROWS, _ROWS_F32 = 256, 128
 
-    def _workspace_usable(self, dev: torch.device) -> bool:
-        ws = self._workspace
-        return isinstance(ws, torch.Tensor) and ws.device == dev and ws.is_contiguous() and ws.data_ptr() % 256 == 0
-
     def _schedule(self, dev: torch.device) -> None:
         """The matrix-core kernel's work list (``prefill_work_list``) copied into the
-        workspace.  Like FlashInfer's plan, this reads the (small) indptr arrays back to the
-        host once per batch."""
+        workspace, or (shapes that ran on the vector kernel before) into a tensor of the
+        wrapper's own, no larger than the workspace.  Like FlashInfer's plan, this reads the
+        (small) indptr arrays back to the host once per batch."""
         qo = self._qo_indptr.cpu().tolist()
         kp = self._indptr.cpu().tolist()
         last = self._last.cpu().tolist()
         self._nnz_q = qo[-1]
-        ws_bytes = self._workspace.numel() * self._workspace.element_size()
+        ws = self._workspace
+        ws_bytes = ws.numel() * ws.element_size() if isinstance(ws, torch.Tensor) else 0
         g = self._hq // self._hkv
         # (the kernel keeps the split partials of an fp16 cache's power-of-two groups in fp16)
         half = self._q_dtype == torch.float16 and not self._valu_ok
@@ -395,17 +394,39 @@ class BatchPrefillWithPagedKVCacheWrapper:
             return
         items, merges = wl["items_np"], wl["groups_np"]
         off_g, off_ml, off_o = wl["off_groups"], wl["off_ml"], wl["off_o"]
+        self._n_items, self._n_groups = len(items), len(merges)
+        base = 0 if self._valu_ok else self._workspace.data_ptr()
         if len(items):
             flat = np.zeros(off_g // 4 + merges.size, dtype=np.int32)
             flat[: items.size] = items.reshape(-1)
             flat[off_g // 4:] = merges.reshape(-1)
             host = torch.from_numpy(flat).pin_memory()
-            self._workspace.view(torch.uint8)[: 4 * flat.size].view(torch.int32).copy_(host, non_blocking=True)
-        base = self._workspace.data_ptr()
-        self._n_items, self._n_groups = len(items), len(merges)
+            if self._valu_ok:
+                self._list = torch.empty(flat.size, dtype=torch.int32, device=dev)
+                base = self._list.data_ptr()
+            else:
+                self._list = self._workspace.view(torch.uint8)[: 4 * flat.size].view(torch.int32)
+            self._list.copy_(host, non_blocking=True)
+            if self._valu_ok:
+                stream = torch.cuda.current_stream(dev)
+                self._list_stream, self._list_ready = stream.cuda_stream, torch.cuda.Event()
+                self._list_ready.record(stream)
         self._items_ptr, self._groups_ptr = base, base + off_g
         self._ml_ptr, self._o_ptr = base + off_ml, base + off_o
+        self._part_bytes, self._part_o = wl["bytes"] - off_ml, off_o - off_ml
         self._chunk = wl["chunk"]
+
+    def _own_list(self, dev: torch.device, stream: int):
+        """A call's use of the wrapper's own list on `stream`: it waits for plan's copy if that was
+        enqueued on another one, and gets a scratch of its own for the split groups' partials."""
+        if self._n_items and stream != self._list_stream:
+            cur = torch.cuda.current_stream(dev)
+            cur.wait_event(self._list_ready)
+            self._list.record_stream(cur)
+        if not self._n_groups:
+            return None, 0, 0
+        part = torch.empty(self._part_bytes, dtype=torch.uint8, device=dev)
+        return part, part.data_ptr(), part.data_ptr() + self._part_o
 
     def run(self, q: torch.Tensor, paged_kv_cache, *args, q_scale=None, k_scale=None,
             v_scale=None, out: torch.Tensor | None = None, lse=None, return_lse: bool = False,
@@ -435,12 +456,16 @@ class BatchPrefillWithPagedKVCacheWrapper:
         if mfma:
             if nnz < self._nnz_q:
                 raise ValueError(f"q has {nnz} rows, qo_indptr needs {self._nnz_q}")
+            stream = stream_ptr(q.device)
+            ml_ptr, o_ptr = self._ml_ptr, self._o_ptr
+            if self._valu_ok:
+                _part, ml_ptr, o_ptr = self._own_list(q.device, stream)
             check(lib().pkv_batch_prefill_mfma(
                 q.data_ptr(), q.stride(0), q.stride(1), cv.k_ptr, cv.v_ptr, cv.page_stride, cv.num_pages,
                 self._indices.data_ptr(), self._indices.numel(), self._hq, self._hkv, self._d, self._ps,
                 int(self._causal), self._sm_scale, self._items_ptr, self._n_items, self._groups_ptr,
-                self._n_groups, self._ml_ptr, self._o_ptr, out.data_ptr(), out.stride(0), out.stride(1),
-                dtype_code(q.dtype), stream_ptr(q.device)), "BatchPrefillWithPagedKVCacheWrapper.run")
+                self._n_groups, ml_ptr, o_ptr, out.data_ptr(), out.stride(0), out.stride(1),
+                dtype_code(q.dtype), stream), "BatchPrefillWithPagedKVCacheWrapper.run")
             return out
         check(lib().pkv_batch_prefill_valu(
             q.data_ptr(), q.stride(0), q.stride(1), self._qo_indptr.data_ptr(), nnz, cv.k_ptr,

@@ -633,6 +633,66 @@ def test_prefill_fp32_and_odd_groups_on_the_matrix_cores(name, causal):
     assert torch.equal(small.run(dv.q, dv.cache), ov) and torch.equal(out, ov)
 
 
+def _prefill_wrapper(ws, dv):
+    w = BatchPrefillWithPagedKVCacheWrapper(ws, "NHD")
+    w.plan(dv.append_indptr, dv.indptr, dv.indices, dv.last, dv.hq, dv.hkv, dv.d, dv.ps, causal=True, q_data_type=dv.dtype)
+    assert w._mfma
+    return w
+
+
+@pytest.mark.parametrize("a,b", [("g4_fp32_d64", "g8_fp32_d128"), ("g5_fp16_d128", "g7_bf16_d128")])
+def test_prefill_plans_leave_a_shared_workspace_alone(a, b):
+    """Shapes that once ran on the vector kernel, which uses no workspace: two planned wrappers and a decode
+    wrapper on one buffer, planned first and run afterwards, give what each gives on a buffer of its own, and
+    the buffer holds what it held."""
+    dvs = [ODD_GROUPS[n]().to(DEV) for n in (a, b)]
+    for dv in dvs:
+        _append_dev(dv)
+    alone = [_prefill_wrapper(torch.empty(64 << 20, dtype=torch.uint8, device=DEV), dv).run(dv.q, dv.cache) for dv in dvs]
+    dec = workloads.build_batch([2000, 33, 1500], [1] * 3, 32, 8, 64, torch.float32, 93).to(DEV)
+    _append_dev(dec)
+    dec_alone = _decode_dev(dec, dec.q)
+    ws = torch.empty(128 << 20, dtype=torch.uint8, device=DEV)
+    w = BatchDecodeWithPagedKVCacheWrapper(ws, "NHD")
+    w.plan(dec.indptr, dec.indices, dec.last, dec.hq, dec.hkv, dec.d, dec.ps, q_data_type=dec.dtype)
+    before = ws.clone()
+    shared = [_prefill_wrapper(ws, dv) for dv in dvs]
+    for _ in range(2):
+        assert torch.equal(w.run(dec.q, dec.cache), dec_alone)
+        ws.copy_(before)  # (the decode's own partials)
+        for sw, dv, ref in zip(shared, dvs, alone):
+            assert torch.equal(sw.run(dv.q, dv.cache), ref)
+        assert torch.equal(ws, before)
+
+
+@pytest.mark.parametrize("name", ["g4_fp32_d64", "g5_fp16_d128"])
+def test_prefill_runs_of_one_plan_on_several_streams(name):
+    """One plan, runs with other queries on two streams at a time, neither of them plan's, and a new plan
+    while they may still be running: every result is that of a run by itself."""
+    dv = ODD_GROUPS[name]().to(DEV)
+    _append_dev(dv)
+    qs = [dv.q * x for x in (1.0, 0.5, -1.0, 2.0)]
+    ws = torch.empty(64 << 20, dtype=torch.uint8, device=DEV)
+    w = _prefill_wrapper(ws, dv)
+    assert w._n_groups  # (split key ranges: partials)
+    alone = [w.run(q, dv.cache) for q in qs]
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(streams[2]):
+        w = _prefill_wrapper(ws, dv)
+    outs = []
+    for i, q in enumerate(qs):
+        with torch.cuda.stream(streams[i % 2]):
+            outs.append(w.run(q, dv.cache))
+    with torch.cuda.stream(streams[2]):
+        w.plan(dv.append_indptr, dv.indptr, dv.indices, dv.last, dv.hq, dv.hkv, dv.d, dv.ps, causal=True,
+               q_data_type=dv.dtype)
+        torch.zeros(1 << 22, dtype=torch.int32, device=DEV)
+    torch.cuda.synchronize()
+    for i, (o, ref) in enumerate(zip(outs, alone)):
+        assert torch.equal(o, ref), i
+
+
 @pytest.mark.parametrize("name", ["g7_bf16_d128", "g4_fp32_d64", "g8_fp32_d128"])
 def test_prefill_infinite_and_nan_values_stay_with_the_rows_that_see_them(name):
     """A value row holding an infinity or a NaN reaches the query rows whose keys include it and no
