@@ -14,8 +14,8 @@
 // doubled while the partials would not fit in the workspace.
 #include <algorithm>
 #include <array>
+#include <cmath>
 #include <functional>
-#include <queue>
 #include <vector>
 #include "../../include/pagedkv.h"
 
@@ -29,8 +29,9 @@ constexpr int kChunkMin = 256, kChunkMax = 8192;
 // its products' issue time on the compute unit (128 x 64 keys x head_dim / 64 at 0.61 TFLOP/s).
 constexpr double kStepUs = 1.9, kItemUs = 11.0, kSplitUs = 6.0, kStepF32Us = 3.4;
 constexpr int kRowsF32 = 128;
-// Candidate chunks, as multiples of total keys / CUs (in 1/16).
-constexpr int kCandidates[] = {8, 10, 12, 14, 16, 17, 18, 20, 24};
+// Candidate chunks, as multiples of total keys / CUs (in 1/16); the longest first, since a simulation
+// ends where it passes the best so far, and shorter chunks have more items to place.
+constexpr int kCandidates[] = {24, 20, 18, 17, 16, 14, 12, 10, 8};
 
 struct Group {
   int h, t0, tq, kv_end, kv_len, qo_len, qo_start, kp0, b;
@@ -59,28 +60,56 @@ Layout layout_for(const std::vector<Group>& groups, int chunk, int rows, int hea
   return L;
 }
 
+// The upper half of a sort key that puts longer key ranges first.
+uint64_t longest_first(int len) { return (uint64_t)(0x7fffffffu - (uint32_t)len) << 32; }
+
 // Simulated kernel time of the work list cut at `chunk`: items longest first, each to the
-// least loaded of ncu compute units.
-double makespan(const std::vector<Group>& groups, int chunk, int ncu, double step_us) {
-  struct It {
-    int len;
-    bool split;
-  };
-  std::vector<It> its;
-  for (const Group& gr : groups) {
-    const int nch = std::max(1, (gr.kv_end + chunk - 1) / chunk);
-    for (int c = 0; c < nch; ++c) its.push_back({std::min(gr.kv_end, (c + 1) * chunk) - c * chunk, nch > 1});
+// least loaded of ncu compute units.  (Some time over `limit` where the work list takes longer.)
+double makespan(const std::vector<Group>& groups, int hkv, int chunk, int ncu, double step_us, double limit) {
+  // (a tile's KV heads and whole chunks are alike and neighbours in the order, so a tile is one or two
+  // entries with a count; from the longest, equal lengths in their order: one key each)
+  std::vector<uint64_t> its;
+  std::vector<int> count;
+  its.reserve(2 * groups.size() / hkv);
+  count.reserve(2 * groups.size() / hkv);
+  double sum = 0.0;  // (a unit's share is at least the mean)
+  for (size_t i = 0; i < groups.size(); i += hkv) {
+    const int end = groups[i].kv_end, nch = std::max(1, (end + chunk - 1) / chunk);
+    auto add = [&](int len, int n) {
+      its.push_back(longest_first(len) | (uint64_t)its.size() << 1 | (nch > 1));
+      count.push_back(n);
+      sum += n * (kItemUs + (nch > 1 ? kSplitUs : 0.0) + step_us * ((len + kStepKeys - 1) / kStepKeys));
+    };
+    if (nch > 1) add(chunk, (nch - 1) * hkv);
+    add(end - (nch - 1) * chunk, hkv);
   }
-  std::stable_sort(its.begin(), its.end(), [](const It& a, const It& b) { return a.len > b.len; });
-  std::priority_queue<double, std::vector<double>, std::greater<double>> load;
-  for (int i = 0; i < ncu; ++i) load.push(0.0);
+  if (sum / ncu > limit * (1.0 + 1e-9)) return sum / ncu;
+  std::sort(its.begin(), its.end());
+  // units in use (a heap once all are: the least loaded one's entry then grows in place)
+  std::vector<double> load;
+  load.reserve(ncu);
   double worst = 0.0;
-  for (const It& it : its) {
-    const double t = load.top() + kItemUs + (it.split ? kSplitUs : 0.0) +
-                     step_us * ((it.len + kStepKeys - 1) / kStepKeys);
-    load.pop();
-    load.push(t);
-    worst = std::max(worst, t);
+  for (const uint64_t it : its) {
+    const int len = (int)(0x7fffffffu - (uint32_t)(it >> 32));
+    const double split = it & 1 ? kSplitUs : 0.0, steps = step_us * ((len + kStepKeys - 1) / kStepKeys);
+    for (int n = count[(uint32_t)it >> 1]; n > 0; --n) {
+      if ((int)load.size() < ncu) {
+        load.push_back(0.0 + kItemUs + split + steps);
+        worst = std::max(worst, load.back());
+        if ((int)load.size() == ncu) std::make_heap(load.begin(), load.end(), std::greater<double>());
+        continue;
+      }
+      const double t = load[0] + kItemUs + split + steps;
+      worst = std::max(worst, t);
+      if (worst > limit) return worst;
+      size_t at = 0;
+      for (size_t kid; (kid = 2 * at + 1) < load.size(); at = kid) {
+        kid += kid + 1 < load.size() && load[kid + 1] < load[kid];
+        if (load[kid] >= t) break;
+        load[at] = load[kid];
+      }
+      load[at] = t;
+    }
   }
   return worst;
 }
@@ -130,13 +159,19 @@ extern "C" int pkv_prefill_work_list(const int32_t* qo_indptr, const int32_t* kv
   if (chunk != 0) {
     best = chunk;
   } else {
-    double best_t = 0.0;
+    int longest = 0;
+    for (const Group& gr : grs) longest = std::max(longest, gr.kv_end);
+    double best_t = 0.0, whole_t = -1.0;  // (whole_t: no range is cut, whichever such chunk)
     int widest = kChunkMin;
     for (int f : kCandidates) {
       const int c = round_chunk(per_cu * f / 16);
       widest = std::max(widest, c);
       if (layout_for(grs, c, rows, head_dim, partial_bytes).bytes > workspace_bytes) continue;
-      const double t = makespan(grs, c, num_cus, step_us);
+      if (c == best) continue;  // (clamped to the same chunk)
+      const bool whole = c >= longest;
+      const double limit = best == 0 ? HUGE_VAL : best_t;
+      const double t = whole && whole_t >= 0.0 ? whole_t : makespan(grs, num_kv_heads, c, num_cus, step_us, limit);
+      if (whole) whole_t = t;
       if (best == 0 || t < best_t || (t == best_t && c > best)) {
         best = c;
         best_t = t;
@@ -179,10 +214,13 @@ extern "C" int pkv_prefill_work_list(const int32_t* qo_indptr, const int32_t* kv
     ++ng;
     nslots += nch;
   }
-  std::stable_sort(its.begin(), its.end(), [](const std::array<int32_t, kItemWords>& a,
-                                              const std::array<int32_t, kItemWords>& b) {
-    return a[5] - a[4] > b[5] - b[4];
-  });
-  for (size_t i = 0; i < its.size(); ++i) std::copy(its[i].begin(), its[i].end(), items + i * kItemWords);
+  std::vector<uint64_t> order;
+  order.reserve(its.size());
+  for (const auto& it : its) order.push_back(longest_first(it[5] - it[4]) | order.size());
+  std::sort(order.begin(), order.end());
+  for (size_t i = 0; i < its.size(); ++i) {
+    const auto& it = its[(uint32_t)order[i]];
+    std::copy(it.begin(), it.end(), items + i * kItemWords);
+  }
   return 0;
 }

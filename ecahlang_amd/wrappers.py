@@ -271,6 +271,14 @@ def prefill_work_list(qo_indptr, kv_indptr, last_page_len, g: int, hkv: int, pag
     for fp16 caches (the kernel keeps their partials in fp16), 4 otherwise.  Items are issued
     longest first.  ``items`` / ``groups`` are lists of records; ``items_np`` / ``groups_np``
     the same as int32 arrays."""
+    wl = _work_list(qo_indptr, kv_indptr, last_page_len, g, hkv, page_size, causal, head_dim, num_cus, ws_bytes, rows,
+                    partial_bytes, chunk)
+    return {"items": wl["items_np"].tolist(), "groups": wl["groups_np"].tolist(), **wl}
+
+
+def _work_list(qo_indptr, kv_indptr, last_page_len, g, hkv, page_size, causal, head_dim, num_cus, ws_bytes, rows,
+               partial_bytes, chunk=None) -> dict:
+    """``prefill_work_list`` without the records as lists."""
     qo = np.ascontiguousarray(np.asarray(qo_indptr, dtype=np.int64), dtype=np.int32)
     kv = np.ascontiguousarray(np.asarray(kv_indptr, dtype=np.int64), dtype=np.int32)
     last = np.ascontiguousarray(np.asarray(last_page_len, dtype=np.int64), dtype=np.int32)
@@ -298,9 +306,8 @@ def prefill_work_list(qo_indptr, kv_indptr, last_page_len, g: int, hkv: int, pag
     check(int(rc), "prefill plan")
     ni, ng = int(info[0]), int(info[1])
     items, groups = items[:ni], groups[:ng]
-    return {"items": items.tolist(), "groups": groups.tolist(), "items_np": items, "groups_np": groups,
-            "chunk": int(info[2]), "slots": int(info[3]), "off_groups": int(info[4]), "off_ml": int(info[5]),
-            "off_o": int(info[6]), "bytes": int(info[7])}
+    return {"items_np": items, "groups_np": groups, "chunk": int(info[2]), "slots": int(info[3]),
+            "off_groups": int(info[4]), "off_ml": int(info[5]), "off_o": int(info[6]), "bytes": int(info[7])}
 
 
 class BatchPrefillWithPagedKVCacheWrapper:
@@ -373,11 +380,11 @@ class BatchPrefillWithPagedKVCacheWrapper:
         """The matrix-core kernel's work list (``prefill_work_list``) copied into the
         workspace, or (shapes that ran on the vector kernel before) into a tensor of the
         wrapper's own, no larger than the workspace.  Like FlashInfer's plan, this reads the
-        (small) indptr arrays back to the host once per batch."""
-        qo = self._qo_indptr.cpu().tolist()
-        kp = self._indptr.cpu().tolist()
-        last = self._last.cpu().tolist()
-        self._nnz_q = qo[-1]
+        (small) indptr arrays back to the host once per batch, in one copy."""
+        n = self._batch + 1
+        table = torch.cat((self._qo_indptr, self._indptr, self._last)).cpu().numpy()
+        qo, kp, last = table[:n], table[n:2 * n], table[2 * n:]
+        self._nnz_q = int(qo[-1])
         ws = self._workspace
         ws_bytes = ws.numel() * ws.element_size() if isinstance(ws, torch.Tensor) else 0
         g = self._hq // self._hkv
@@ -385,8 +392,8 @@ class BatchPrefillWithPagedKVCacheWrapper:
         half = self._q_dtype == torch.float16 and not self._valu_ok
         try:
             rows = self._ROWS_F32 if self._q_dtype == torch.float32 else self._ROWS
-            wl = prefill_work_list(qo, kp, last, g, self._hkv, self._ps, self._causal, self._d, _num_cus(dev),
-                                   ws_bytes, rows // g * g, partial_bytes=2 if half else 4)
+            wl = _work_list(qo, kp, last, g, self._hkv, self._ps, self._causal, self._d, _num_cus(dev), ws_bytes,
+                            rows // g * g, 2 if half else 4)
         except RuntimeError:
             if not self._valu_ok:
                 raise

@@ -666,6 +666,17 @@ def test_prefill_plans_leave_a_shared_workspace_alone(a, b):
 
 
 @pytest.mark.parametrize("name", ["g4_fp32_d64", "g5_fp16_d128"])
+def test_prefill_plan_reads_the_table_in_one_copy(name, monkeypatch):
+    """plan() waits for the device once, however many index arrays it reads."""
+    dv = ODD_GROUPS[name]().to(DEV)
+    reads = []
+    cpu = torch.Tensor.cpu
+    monkeypatch.setattr(torch.Tensor, "cpu", lambda t, *a, **k: (reads.append(t.numel()), cpu(t, *a, **k))[1])
+    w = _prefill_wrapper(torch.empty(64 << 20, dtype=torch.uint8, device=DEV), dv)
+    assert reads == [2 * (w._batch + 1) + w._batch]
+
+
+@pytest.mark.parametrize("name", ["g4_fp32_d64", "g5_fp16_d128"])
 def test_prefill_runs_of_one_plan_on_several_streams(name):
     """One plan, runs with other queries on two streams at a time, neither of them plan's, and a new plan
     while they may still be running: every result is that of a run by itself."""

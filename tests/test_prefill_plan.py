@@ -2,6 +2,7 @@
 BatchPrefillWithPagedKVCacheWrapper.plan) on the CPU: every (request, KV head, query tile) sees
 exactly the keys causal (bottom-right aligned) or full attention gives it, cut into chunks that
 tile that range without gaps or overlaps, and every split group's record matches its chunks."""
+import heapq
 import random
 
 import pytest
@@ -147,3 +148,39 @@ def test_given_chunk_and_chosen_chunk_match_the_restatement(seed):
     wl = prefill_work_list(qo, kv, last, g, hkv, 16, causal, 128, ncu, 1 << 40)
     assert wl["chunk"] == want, (wl["chunk"], times)
     assert (wl["items"], wl["groups"]) == _list_for(groups, want)
+
+
+def _simulated(tiles, hkv, chunk, ncu, step_us):
+    """Kernel time of the list cut at `chunk`, item by item: the longest first (equal lengths in list
+    order), each to the least loaded unit."""
+    its = []
+    for end in tiles:
+        n = max(1, -(-end // chunk))
+        its += [(min(end, (c + 1) * chunk) - c * chunk, n > 1) for _ in range(hkv) for c in range(n)]
+    its.sort(key=lambda it: -it[0])
+    load = [0.0] * ncu
+    for length, split in its:
+        heapq.heapreplace(load, load[0] + 11.0 + (6.0 if split else 0.0) + step_us * (-(-length // 64)))
+    return max(load)
+
+
+@pytest.mark.parametrize("seed", range(8))
+def test_chunk_is_the_candidate_with_the_lowest_simulated_time(seed):
+    """The library ends a simulation that has passed the best and places alike items together; the choice
+    is that of simulating every candidate item by item (ties to the longer chunk)."""
+    rng = random.Random(100 + seed)
+    for _ in range(12):
+        g, hkv, d, base = rng.choice([(8, 2, 128, 256), (7, 4, 128, 256), (4, 8, 64, 128), (1, 8, 128, 128)])
+        rows = base // g * g
+        qo, kv, last = _batch(rng, rng.randint(1, 9))
+        ncu = rng.choice([8, 64, 256])
+        wl = prefill_work_list(qo, kv, last, g, hkv, 16, True, d, ncu, 1 << 40, rows)
+        tq, tiles = rows // g, []
+        for b in range(len(qo) - 1):
+            n, pages = qo[b + 1] - qo[b], kv[b + 1] - kv[b]
+            L = (pages - 1) * 16 + last[b] if pages else 0
+            tiles += [min(L, max(0, min(t0 + tq, n) + L - n)) for t0 in range(0, n, tq)]
+        per = -(-sum(tiles) * hkv // ncu)
+        cand = {min(8192, max(256, (per * f // 16 + 32) // 64 * 64)) for f in (8, 10, 12, 14, 16, 17, 18, 20, 24)}
+        step = 1.9 if rows > 128 else 3.4 * d / 64
+        assert wl["chunk"] == min(cand, key=lambda c: (_simulated(tiles, hkv, c, ncu, step), -c))
