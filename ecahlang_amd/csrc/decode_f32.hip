@@ -2,8 +2,8 @@
 // to 16).  Same contract as the vector kernel (BatchDecodeWithPagedKVCacheWrapper.run,
 // ecahlang/main.py:68); everything stays in fp32: v_mfma_f32_16x16x4_f32 takes fp32 operands.
 //
-// A workgroup (8 waves) takes one KV head of one part of one sequence's pages; wave r takes the part's
-// pages r, r + 8, ...  With lane l = (lr = l % 16, lg = l / 16), a page:
+// A workgroup (W = 4 waves) takes one KV head of one part of one sequence's pages; wave r takes the part's
+// pages r, r + W, ...  With lane l = (lr = l % 16, lg = l / 16), a page:
 //   S[token][head]      = K . Q^T   A: lane holds K[token lr][dim 16 s + 4 lg + e], B: Q[head lr][the same
 //                                   dims]: one 16-byte load feeds the four products e = 0 .. 3
 //   online softmax                  lane: head lr, tokens 4 lg + i
@@ -12,8 +12,9 @@
 //                                   64 c + 4 lr + e], one 16-byte load for the four output tiles e
 // so K and V go from memory straight into the operand registers (no LDS, no lane exchange), each
 // refilled with the next page's rows as soon as its products are issued, and the group's heads share
-// every row read.  The 8 states meet in LDS at the end; a sequence of several parts is merged by the
-// workgroup that arrives last, over all heads.
+// every row read.  The waves' states meet in LDS at the end.  A sequence of several parts is merged by the
+// workgroup that arrives last: of a KV head's parts, for that head, or (without head counters) of all of
+// the sequence's, for all heads.
 //
 // What bounds it: the bytes of K and V at large batches (5.3 TB/s at 197 MB); a small batch is a chain
 // of latencies (page list, page ids, rows: 5.2 us for one sequence of 100 tokens; partials, arrival,
@@ -23,6 +24,12 @@
 // eight: more of them start while others wait (11.1 and 13.1 us).  On the vector kernel the same call
 // took 280 us: every lane read a whole K row, V one token at a time, and a sequence of 2048 tokens was
 // cut into 128 parts.  Error against 64 bits: 1.7e-7, 2.4e-7 there.
+//
+// A large batch of short sequences is bound by the workgroups there are, one per KV head and sequence
+// (about 3.5 ns each): 1024 / 4096 / 8192 sequences of 16 tokens at 8 KV heads 30 / 110 / 235 us (65 / 266 /
+// 571 on the vector kernel; 70 / 595 / 2071 when every workgroup looked through the whole batch for its
+// part).  Below about four tokens a sequence the vector kernel's few workgroups are still ahead there (16 KV
+// heads, 1024 sequences of 1 / 4 / 16 tokens: 48 us for its 28 / 43 / 103); the host does not know the lengths.
 #include <algorithm>
 #include "attn_common.h"
 #include "mfma_common.h"
@@ -58,48 +65,66 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 4 : 2) void decode_f32_kernel(Dec
   const int B = P.batch, g = P.hq / P.hkv;
   const int h = blockIdx.x % P.hkv, w = blockIdx.x / P.hkv;
 
-  // ---- part w of the batch: sequence b's parts follow those of b - 1; 64 sequences a round
+  // ---- workgroup w: the first part of sequence w, or (w >= B) the (w - B)-th of the further parts, which
+  // follow each other in sequence order.  Only those and cut sequences look for their place among the
+  // batch, 64 sequences a round (each workgroup over all of it, the time of a large batch of short
+  // sequences went with its square).
   const int cut = (int)min((int64_t)INT_MAX, P.num_indices);  // the page list ends there
-  int ip0 = P.indptr[min(lane, B)], ip1 = P.indptr[min(lane + 1, B)];
-  int lastv = P.last[min(lane, B - 1)];
+  const int own = min(w, B - 1);
+  int ip0 = P.indptr[min(lane, B)], ip1 = P.indptr[min(lane + 1, B)], lastv = P.last[min(lane, B - 1)];
+  int b = own, s0 = P.indptr[own], e0 = P.indptr[own + 1], lastp = P.last[own];
   const int total = max(min(P.indptr[B], cut), 1);
   const int aim = max(kMinPages, (total + nr - 1) / nr);
-  int base = 0, b = -1, s0 = 0, np = 0, avail = 0, nparts = 0, slot0 = 0, lastp = 0;
-  for (int b0 = 0; b0 < B; b0 += 64) {
-    if (b0 > 0) {
-      ip0 = P.indptr[min(b0 + lane, B)], ip1 = P.indptr[min(b0 + lane + 1, B)];
-      lastv = P.last[min(b0 + lane, B - 1)];
-    }
-    const int av = max(min(ip1, cut) - max(ip0, 0), 0);  // listed pages
-    const int n = b0 + lane < B ? parts_of(av, aim, max_parts) : 0;
-    int incl = n;
+  auto listed = [&](int i0, int i1) { return max(min(i1, cut) - max(i0, 0), 0); };  // pages of the list
+  int avail = listed(s0, e0), nparts = parts_of(avail, aim, max_parts), part = 0, more0 = 0;
+  if (w >= B || nparts > 1) {
+    bool found = false;
+    int base = 0;
+#pragma unroll 1
+    for (int b0 = 0; b0 < B; b0 += 64) {
+      const int n0 = P.indptr[min(b0 + 64 + lane, B)], n1 = P.indptr[min(b0 + 65 + lane, B)];  // (the next round's)
+      const int nl = P.last[min(b0 + 64 + lane, B - 1)];
+      const int av = listed(ip0, ip1);
+      const int n = b0 + lane < B ? parts_of(av, aim, max_parts) - 1 : 0;
+      int incl = n;
 #pragma unroll
-    for (int x = 1; x < 64; x <<= 1) {
-      const int v = __shfl_up(incl, x, 64);
-      incl += lane >= x ? v : 0;
+      for (int x = 1; x < 64; x <<= 1) {
+        const int v = __shfl_up(incl, x, 64);
+        incl += lane >= x ? v : 0;
+      }
+      const int all = __builtin_amdgcn_readlane(incl, 63);
+      if (w < B ? w < b0 + 64 : w - B < base + all) {
+        const int l = w < B ? w - b0 : __popcll(__ballot(base + incl <= w - B));
+        more0 = base + __builtin_amdgcn_readlane(incl, l) - __builtin_amdgcn_readlane(n, l);
+        if (w >= B) {
+          b = b0 + l;
+          s0 = __builtin_amdgcn_readlane(ip0, l);
+          e0 = __builtin_amdgcn_readlane(ip1, l);
+          lastp = __builtin_amdgcn_readlane(lastv, l);
+          avail = __builtin_amdgcn_readlane(av, l);
+          nparts = parts_of(avail, aim, max_parts);
+          part = 1 + w - B - more0;
+        }
+        found = true;
+        break;
+      }
+      base += all;
+      ip0 = n0, ip1 = n1, lastv = nl;
     }
-    const int all = __builtin_amdgcn_readlane(incl, 63);
-    if (w < base + all) {
-      const int l = __popcll(__ballot(base + incl <= w));
-      b = b0 + l;
-      s0 = __builtin_amdgcn_readlane(ip0, l);
-      np = __builtin_amdgcn_readlane(ip1, l) - s0;
-      avail = __builtin_amdgcn_readlane(av, l);
-      nparts = __builtin_amdgcn_readlane(n, l);
-      slot0 = base + __builtin_amdgcn_readlane(incl, l) - nparts;
-      lastp = __builtin_amdgcn_readlane(lastv, l);
-      break;
-    }
-    base += all;
+    if (!found) return;  // (the grid is sized for the most parts there can be)
+    nparts = 1 + min(nparts - 1, max(nr - more0, 0));  // (a kv_indptr that runs backwards)
   }
-  if (b < 0) return;  // (the grid is sized for the most parts there can be)
+  const int np = e0 - s0;
   // the part's pages [p0, end) of the page list, a wave's p0 + wave, + W, ... (the ids of 64 of them a
   // lane each)
-  const int part = w - slot0;
   const int per = avail / nparts, more = avail - per * nparts;  // (the first `more` parts hold a page more)
   const int p0 = max(s0, 0) + part * per + min(part, more), end = p0 + per + (part < more ? 1 : 0);
   const int len = np > 0 ? (np - 1) * 16 + lastp : 0;
   const int n = end - p0 > wave ? (end - p0 - 1 - wave) / W + 1 : 0;
+  // a sequence of one page at most is wave 0's, which writes its own state; the others leave their
+  // places to further workgroups
+  const bool one = nparts == 1 && end - p0 <= 1;
+  if (one && wave > 0) return;
   int pidv = n > 0 ? P.indices[min(p0 + wave + W * lane, end - 1)] : -1;
 
   const int64_t rowstride = (int64_t)P.hkv * D, hoff = (int64_t)h * D;
@@ -238,7 +263,7 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 4 : 2) void decode_f32_kernel(Dec
   lds_barrier();
   float2 v[W];
 #pragma unroll
-  for (int x = 0; x < W; ++x) v[x] = s_ml[x][lr];
+  for (int x = 0; x < W; ++x) v[x] = x == 0 || !one ? s_ml[x][lr] : make_float2(-INFINITY, 0.f);
   float M = -INFINITY, L = 0.f;
 #pragma unroll
   for (int x = 0; x < W; ++x) M = fmaxf(M, v[x].x);
@@ -264,13 +289,14 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 4 : 2) void decode_f32_kernel(Dec
   if (lr < g) {
     const float inv = L > 0.f ? 1.f / L : 0.f;
     const int64_t hq = h * g + lr;
-#pragma unroll
-    for (int y = 0; y < (NP + W - 1) / W; ++y) {  // piece 4 c + i by wave (4 c + i) % W
-      const int pc = y * W + wave;
-      if (NP % W && pc >= NP) break;
+#pragma unroll 1
+    for (int pc = wave; pc < NP; pc += one ? 1 : W) {  // piece 4 c + i by wave (4 c + i) % W
       f4 acc = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int x = 0; x < W; ++x) acc += s_o[x][pc][lane];
+      for (int x = 0; x < W; ++x) {
+        const f4 y = s_o[x][pc][lane];
+        acc += x == 0 || !one ? y : f4{0.f, 0.f, 0.f, 0.f};
+      }
       acc *= inv;
       const int d = 64 * (pc / 4) + 16 * lg + 4 * (pc % 4);
       if (nparts == 1) store_row(hq, d, acc);
@@ -292,8 +318,8 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 4 : 2) void decode_f32_kernel(Dec
   for (int gr = wave / nw; gr < (groups + W / nw - 1) / (W / nw) * (W / nw); gr += W / nw) {  // (the same rounds for every wave)
     const int x = x0 + min(gr * 64 + lane, nx - 1);
     const int hq = x / (D / 4), d = (x - hq * (D / 4)) * 4;
-    const float2* ml = P.part_ml + (int64_t)slot0 * P.ml_stride + hq;
-    const float* po = P.part_o + ((int64_t)slot0 * P.hq + hq) * D + d;
+    const float2* ml = P.part_ml + hq;
+    const float* po = P.part_o + (int64_t)hq * D + d;
     const int q1 = min(share * (wave % nw + 1), nparts);
     float M2 = -INFINITY, den = 0.f;
     f4 acc = f4{0.f, 0.f, 0.f, 0.f};
@@ -307,7 +333,8 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 4 : 2) void decode_f32_kernel(Dec
       f4 row[kMergeParts];
 #pragma unroll
       for (int q = 0; q < kMergeParts; ++q) {
-        const int64_t sl = min(q0 + q, q1 - 1);
+        const int pq = min(q0 + q, q1 - 1);
+        const int64_t sl = pq == 0 ? b : B + more0 + pq - 1;
         y[q] = ld_dev2(ml + sl * P.ml_stride);
         row[q] = *reinterpret_cast<const f4*>(po + sl * P.hq * D);
       }

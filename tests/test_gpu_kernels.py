@@ -309,6 +309,11 @@ F32_DECODE = {
     "b70_d64": (lambda: workloads.build_batch([(7 * i) % 190 + 1 for i in range(70)], [1] * 70, 4, 2, 64, torch.float32, 85), None),
     "b300_hkv8_d64": (lambda: workloads.build_batch([(5 * i) % 150 + 1 for i in range(300)], [1] * 300, 8, 8, 64,
                                                     torch.float32, 86), None),
+    # cut sequences at the edges of the rounds of 64 in which a further part looks for its sequence
+    "b200_cut_d64": (lambda: workloads.build_batch([700 + b if b in (0, 63, 64, 65, 127, 128, 199) else b % 17 + 1 for b in range(200)],
+                                                   [1] * 200, 6, 6, 64, torch.float32, 89), None),
+    "b129_cut_d128": (lambda: workloads.build_batch([b % 40 + 1 if b < 127 else 900 for b in range(129)], [1] * 129, 8, 2, 128,
+                                                    torch.float32, 90), 64),
     "b1_long_d64": (lambda: workloads.build_batch([9000], [1], 8, 2, 64, torch.float32, 87), None),
     "b1_one_part_d128": (lambda: workloads.build_batch([4200, 40], [1] * 2, 8, 2, 128, torch.float32, 88), 1),
 }
