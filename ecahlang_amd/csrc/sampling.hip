@@ -15,6 +15,7 @@
 // so the result depends on nothing but the row and u (no floating-point summation order).
 // Every pass reads the row with 16-byte loads (8 fp16/bf16 or 4 fp32 logits per thread, 8 tiles
 // in flight); after the first pass the row is served from L2.
+#include <type_traits>
 #include "common.h"
 #include "../../include/pagedkv.h"
 
@@ -491,6 +492,12 @@ struct TileSums {
     m = wave_sum_u64(m);
     if ((threadIdx.x & 63) == 0) red[jj][threadIdx.x >> 6] = m;
   }
+  // (a row of one slice: for the workgroup itself)
+  __device__ __forceinline__ void keep(uint64_t* s_tile, int n) const {
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t < n) s_tile[t] = red[t][0] + red[t][1] + red[t][2] + red[t][3];
+  }
   // (written through to device scope)
   __device__ __forceinline__ void store(uint64_t* tm, int n) const {
     __syncthreads();
@@ -499,6 +506,14 @@ struct TileSums {
       __hip_atomic_store(tm + t, red[t][0] + red[t][1] + red[t][2] + red[t][3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 };
+// Largest of mx over the workgroup; red: 4 floats.
+__device__ __forceinline__ float block_max256(float mx, float* red) {
+  mx = wave_max_f32(mx);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+}
 // Largest of mx (x) and smallest of mn (y) over the workgroup; red: 8 floats.
 __device__ __forceinline__ float2 block_range256(float mx, float mn, float* red) {
   mx = wave_max_f32(mx);
@@ -538,7 +553,11 @@ struct ScaleArgs {
   int64_t out_stride;
 };
 
-template <typename T, bool SCALE>
+// WHOLE, here and in the pass: the host knows that every row is a whole row, and the kernels hold nothing
+// else (one row of 1000 logits 10.5 -> 9.0 us, 128 of 32,000 16.8 -> 15.2, of 151,936 33.7 -> 30.4, in a graph,
+// with rows of one slice done without an arrival and the token's tile found without a barrier; 9.2, 15.1 and
+// 32.0 when the kinds had launches of their own).
+template <typename T, bool SCALE, bool WHOLE>
 __global__ __launch_bounds__(kSplitThreads) void split_scan_kernel(const T* logits, int64_t row_stride, int vocab,
                                                                    const int32_t* top_k, int32_t top_k_all,
                                                                    const float* top_p, float top_p_all,
@@ -549,7 +568,7 @@ __global__ __launch_bounds__(kSplitThreads) void split_scan_kernel(const T* logi
     ws.counter[b * kCountStride] = 0;
     ws.fallback[b] = 0;
   }
-  const int kind = row_kind(b, vocab, top_k, top_k_all, top_p, top_p_all);
+  const int kind = WHOLE ? (int)kWholeRow : row_kind(b, vocab, top_k, top_k_all, top_p, top_p_all);
   if (!SCALE && kind == kOtherRow) return;
   const T* p = logits + (int64_t)b * row_stride;
   const bool vec = ((uintptr_t)p % 16) == 0;
@@ -561,7 +580,7 @@ __global__ __launch_bounds__(kSplitThreads) void split_scan_kernel(const T* logi
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       gx = ok[k] ? fmaxf(gx, x[k]) : gx;
-      mn = ok[k] ? fminf(mn, x[k]) : mn;
+      if constexpr (!WHOLE) mn = ok[k] ? fminf(mn, x[k]) : mn;
     }
   };
   auto group_end = [&](int jj) __attribute__((always_inline)) {
@@ -643,7 +662,10 @@ __global__ __launch_bounds__(kSplitThreads) void split_scan_kernel(const T* logi
       group_end(jj);
     }
   }
-  if (kind == kWholeRow || kind == kTopPRow) {
+  if constexpr (WHOLE) {
+    const float r = block_max256(gx, red);
+    if (threadIdx.x == 0) ws.smax[(int64_t)b * S + s] = r;
+  } else if (kind == kWholeRow || kind == kTopPRow) {
     const float2 r = block_range256(fmaxf(mx, gx), mn, red);
     if (threadIdx.x == 0) {
       ws.smax[(int64_t)b * S + s] = r.x;
@@ -709,21 +731,25 @@ __device__ __forceinline__ void wave_to_lds_sum(uint64_t* p, uint64_t v) {
   v = wave_sum_u64(v);
   if ((threadIdx.x & 63) == 0) atomicAdd((unsigned long long*)p, (unsigned long long)v);
 }
-struct TokenAt {
-  uint64_t before;  // the kept mass of the tiles before the token's
-  int tile;
-};
 // The token of a whole or top-p row from its tiles' kept masses (in s_tile, for every thread): the
 // tile holding the target, then each thread's kept mass in it, an exclusive scan in thread (=
-// vocabulary) order, and the owner walks its 8 logits.  Kept: key >= thr.
+// vocabulary) order, and the owner walks its 8 logits.  Kept: key >= thr.  redu: written here, read by
+// nobody since the last barrier.
 template <typename T>
 __device__ __forceinline__ void pick_token(const T* p, int vocab, bool vec, float mx, uint32_t thr, const uint64_t* s_tile,
-                                           int ntiles, float u, int32_t* out, uint64_t* redu, TokenAt* at) {
-  // thread t: the tiles [per t, per (t + 1))
-  const int per = (ntiles + kSplitThreads - 1) / kSplitThreads, q0 = per * (int)threadIdx.x;
-  uint64_t own = 0, ms;
+                                           int ntiles, float u, int32_t* out, uint64_t* redu) {
+  // lane l: the tiles [per l, per (l + 1)); every wave for itself, without a barrier
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int per = (ntiles + kWave - 1) / kWave, q0 = per * lane;
+  uint64_t own = 0;
   for (int j = q0; j < min(q0 + per, ntiles); ++j) own += s_tile[j];
-  const uint64_t upto = block_scan256(own, redu, ms);
+  uint64_t upto = own;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint64_t v = __shfl_up(upto, o, kWave);
+    if (lane >= o) upto += v;
+  }
+  const uint64_t ms = __shfl(upto, 63, kWave);
   if (ms == 0) {  // (uniform)
     if (threadIdx.x == 0) *out = -1;  // (no token carries mass: an all-NaN row)
     return;
@@ -731,16 +757,10 @@ __device__ __forceinline__ void pick_token(const T* p, int vocab, bool vec, floa
   const double uu = fminf(fmaxf(u, 0.f), 1.f);
   uint64_t target = (uint64_t)(uu * (double)ms);
   if (target >= ms) target = ms - 1;
-  if (upto > target && upto - own <= target) {
-    uint64_t before = upto - own;
-    int tt = q0;
-    while (before + s_tile[tt] <= target) before += s_tile[tt++];
-    at->before = before;
-    at->tile = tt;
-  }
-  __syncthreads();
-  const int tt = at->tile;
-  const uint64_t before = at->before;
+  const int at = __builtin_ctzll(__ballot(upto > target));  // the lane whose tiles hold it
+  uint64_t before = __shfl(upto - own, at, kWave);
+  int tt = per * at;
+  while (before + s_tile[tt] <= target) before += s_tile[tt++];
   float x[8];
   bool ok[8];
   load8(p, vocab, vec, tt, x, ok);
@@ -751,13 +771,11 @@ __device__ __forceinline__ void pick_token(const T* p, int vocab, bool vec, floa
     if (ok[k]) mine += fmass(x[k], mx);
   }
   uint64_t inc = mine;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
     const uint64_t v = __shfl_up(inc, o, kWave);
     if (lane >= o) inc += v;
   }
-  __syncthreads();
   if (lane == 63) redu[wv] = inc;
   __syncthreads();
   uint64_t off = before;
@@ -806,10 +824,12 @@ __device__ __forceinline__ float2 row_range(const SplitWs& ws, int b, int S, flo
 template <typename T>
 __device__ __forceinline__ void whole_slice(const T* p, int vocab, bool vec, const SliceLoad<T>& sl, int s, int b, int S,
                                             const float* uniform, int32_t* out, const SplitWs& ws, uint64_t* s_tile,
-                                            float* redf, uint64_t (*redu)[4], int* s_last, TokenAt* at) {
+                                            float* redf, uint64_t (*redu)[4], int* s_last) {
   const TileSums sums{redu};
   const int ntiles = split_tiles(vocab), j0 = s * kSliceTiles, j1 = min(j0 + kSliceTiles, ntiles);
-  const float mx = row_range(ws, b, S, redf).x;
+  float mx = -INFINITY;
+  for (int i = threadIdx.x; i < S; i += kSplitThreads) mx = fmaxf(mx, ws.smax[(int64_t)b * S + i]);
+  mx = block_max256(mx, redf);
   // this slice's tile masses, written through to device scope
   uint64_t* tm = ws.tmass + (int64_t)b * ntiles;
 #pragma unroll
@@ -824,11 +844,15 @@ __device__ __forceinline__ void whole_slice(const T* p, int vocab, bool vec, con
       if (ok[k]) m += fmass(x[k], mx);
     sums.add(jj, m);
   }
-  sums.store(tm + j0, j1 - j0);
-  if (!slice_arrive(&ws.counter[b * kCountStride], S, s_last)) return;
-  for (int j = threadIdx.x; j < ntiles; j += kSplitThreads) s_tile[j] = ld_dev(tm + j);
+  if (S == 1) {  // (uniform)
+    sums.keep(s_tile, ntiles);
+  } else {
+    sums.store(tm + j0, j1 - j0);
+    if (!slice_arrive(&ws.counter[b * kCountStride], S, s_last)) return;
+    for (int j = threadIdx.x; j < ntiles; j += kSplitThreads) s_tile[j] = ld_dev(tm + j);
+  }
   __syncthreads();
-  pick_token(p, vocab, vec, mx, 0u, s_tile, ntiles, uniform[b], out + b, redu[0], at);
+  pick_token(p, vocab, vec, mx, 0u, s_tile, ntiles, uniform[b], out + b, redu[0]);
 }
 
 // ---- Top-p rows.  The row's masses are binned by distance from its largest logit (kPBins bins over
@@ -906,7 +930,6 @@ struct ToppLds {
   uint64_t hist[kSplitThreads];
   uint64_t redu[4], tsum[kSliceTiles][4];
   uint64_t above;
-  TokenAt at;
   int off[kMaxSplitTiles / kSliceTiles + 1];
   uint32_t diff, thr;
   int bin, n, last;
@@ -1063,7 +1086,7 @@ __device__ __forceinline__ void topp_finish(const T* p, int vocab, int s, int b,
                 (unsigned long long)fmass(key_float((uint32_t)c), bins.mx));
   }
   __syncthreads();
-  pick_token(p, vocab, vec, bins.mx, thr, s_tile, ntiles, uniform[b], out + b, L.redu, &L.at);
+  pick_token(p, vocab, vec, bins.mx, thr, s_tile, ntiles, uniform[b], out + b, L.redu);
 }
 
 // ---- Top-k rows (0 < k <= kTopKMax, any top-p), one workgroup a row.  The k-th largest of the row's
@@ -1430,35 +1453,42 @@ __device__ __forceinline__ void topk_row(const T* p, int vocab, bool vec, int b,
   topk_merge(b, n, k, pp, uniform, out, ws, L);
 }
 
-template <typename T>
+template <typename T, bool WHOLE>
 __global__ __launch_bounds__(kSplitThreads) __attribute__((amdgpu_waves_per_eu(5))) void split_pass_kernel(
     const T* logits, int64_t row_stride, int vocab, const int32_t* top_k, int32_t top_k_all, const float* top_p,
     float top_p_all, const float* uniform, int32_t* out, SplitWs ws) {
-  union Lds {
+  union AnyLds {
     uint64_t tile[kMaxSplitTiles];
     uint64_t hist[kPBins];
     TopkLds k;
   };
-  __shared__ __align__(16) Lds L;
+  struct WholeLds {
+    uint64_t tile[kMaxSplitTiles];
+  };
+  __shared__ __align__(16) std::conditional_t<WHOLE, WholeLds, AnyLds> L;
   __shared__ float redf[8];
   __shared__ uint64_t redu[kSliceTiles][4];
   __shared__ int s_last;
-  __shared__ TokenAt s_at;
   const int s = blockIdx.x, b = blockIdx.y, S = gridDim.x;
-  const int kind = row_kind(b, vocab, top_k, top_k_all, top_p, top_p_all);
+  const int kind = WHOLE ? (int)kWholeRow : row_kind(b, vocab, top_k, top_k_all, top_p, top_p_all);
   if (kind == kOtherRow) return;
   const T* p = logits + (int64_t)b * row_stride;
   const bool vec = ((uintptr_t)p % 16) == 0;
   const int j0 = s * kSliceTiles, j1 = min(j0 + kSliceTiles, split_tiles(vocab));
-  const float pp = top_p ? top_p[b] : top_p_all;
-  if (kind == kTopKRow) {
-    if (s == 0) topk_row(p, vocab, vec, b, top_k ? top_k[b] : top_k_all, pp, uniform, out, ws, L.k);
-    return;
-  }
   SliceLoad<T> sl;
-  sl.issue(p, vocab, vec, j0, j1);
-  if (kind == kWholeRow) whole_slice(p, vocab, vec, sl, s, b, S, uniform, out, ws, L.tile, redf, redu, &s_last, &s_at);
-  else topp_hist(p, vocab, vec, sl, s, b, S, pp, out, ws, L.hist, redf, redu[0], &s_last);
+  if constexpr (WHOLE) {
+    sl.issue(p, vocab, vec, j0, j1);
+    whole_slice(p, vocab, vec, sl, s, b, S, uniform, out, ws, L.tile, redf, redu, &s_last);
+  } else {
+    const float pp = top_p ? top_p[b] : top_p_all;
+    if (kind == kTopKRow) {
+      if (s == 0) topk_row(p, vocab, vec, b, top_k ? top_k[b] : top_k_all, pp, uniform, out, ws, L.k);
+      return;
+    }
+    sl.issue(p, vocab, vec, j0, j1);
+    if (kind == kWholeRow) whole_slice(p, vocab, vec, sl, s, b, S, uniform, out, ws, L.tile, redf, redu, &s_last);
+    else topp_hist(p, vocab, vec, sl, s, b, S, pp, out, ws, L.hist, redf, redu[0], &s_last);
+  }
 }
 
 template <typename T>
@@ -1476,7 +1506,7 @@ __global__ __launch_bounds__(kSplitThreads) void split_finish_kernel(const T* lo
 // Which kinds of rows a call can hold (scalars settle it on the host, per-row tensors need all), and
 // whether the workspace takes them over many workgroups.
 struct SamplePlan {
-  bool topk = true, topp = true, whole = true, other = true, split = false;
+  bool topk = true, topp = true, whole = true, other = true, whole_only = false, split = false;
   SamplePlan(int rows, int vocab, const int32_t* top_k, int32_t top_k_all, const float* top_p, float top_p_all,
              const void* ws, int64_t ws_bytes) {
     if (!top_k && !top_p) {
@@ -1486,6 +1516,7 @@ struct SamplePlan {
       topp = kind == kTopPRow;
       other = kind == kOtherRow;
     }
+    whole_only = whole && !topk && !topp && !other;
     split = ws && (whole || topk || topp) && rows <= 65535 && split_tiles(vocab) <= kMaxSplitTiles &&
             ws_bytes >= split_ws_bytes(rows, vocab);
   }
@@ -1499,9 +1530,9 @@ int launch_sample(const T* logits, int64_t row_stride, int rows, int vocab, cons
   const dim3 grid((unsigned)split_slices(vocab), (unsigned)rows);
   if (plan.split) {
     // (top-k rows take one workgroup)
-    hipLaunchKernelGGL(split_pass_kernel<T>, plan.whole || plan.topp ? grid : dim3(1, (unsigned)rows),
-                       dim3(kSplitThreads), 0, s, logits, row_stride, vocab, top_k, top_k_all, top_p, top_p_all, uniform,
-                       out, w);
+    hipLaunchKernelGGL((plan.whole_only ? split_pass_kernel<T, true> : split_pass_kernel<T, false>),
+                       plan.whole || plan.topp ? grid : dim3(1, (unsigned)rows), dim3(kSplitThreads), 0, s, logits, row_stride,
+                       vocab, top_k, top_k_all, top_p, top_p_all, uniform, out, w);
     if (plan.topp)
       hipLaunchKernelGGL(split_finish_kernel<T>, grid, dim3(kSplitThreads), split_tiles(vocab) * sizeof(uint64_t), s, logits, row_stride, vocab, top_k,
                          top_k_all, top_p, top_p_all, uniform, out, w);
@@ -1520,7 +1551,7 @@ int scan_and_sample(const T* logits, int64_t row_stride, int rows, int vocab, co
   SplitWs w{};
   if (plan.split) {
     w = split_ws(ws, rows, vocab);
-    hipLaunchKernelGGL((split_scan_kernel<T, false>), dim3((unsigned)split_slices(vocab), (unsigned)rows),
+    hipLaunchKernelGGL((plan.whole_only ? split_scan_kernel<T, false, true> : split_scan_kernel<T, false, false>), dim3((unsigned)split_slices(vocab), (unsigned)rows),
                        dim3(kSplitThreads), 0, s, logits, row_stride, vocab, top_k, top_k_all, top_p, top_p_all,
                        ScaleArgs<T>{}, w);
   }
@@ -1682,7 +1713,7 @@ extern "C" int pkv_scaled_top_k_top_p_sampling(const void* logits, int64_t row_s
   const SplitWs w = split_ws(workspace, rows, vocab);
   const dim3 grid((unsigned)split_slices(vocab), (unsigned)rows);
 #define PKV_SCALE_SCAN(T)                                                                                          \
-  hipLaunchKernelGGL((split_scan_kernel<T, true>), grid, dim3(kSplitThreads), 0, s, (const T*)logits, row_stride,  \
+  hipLaunchKernelGGL((plan.whole_only ? split_scan_kernel<T, true, true> : split_scan_kernel<T, true, false>), grid, dim3(kSplitThreads), 0, s, (const T*)logits, row_stride,  \
                      vocab, top_k, top_k_all, top_p, top_p_all,                                                    \
                      (ScaleArgs<T>{(const T*)penalty, penalty_stride, penalty_slots, penalty_rows, temperature, scaled, \
                                    scaled_stride}),                                                                \

@@ -385,3 +385,25 @@ def test_top_p_split_path_equals_single_workgroup(dtype, vocab):
     torch.cuda.synchronize()
     assert torch.equal(got, want) and torch.equal(got2, want2)
     assert got2[3].item() == -1
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("vocab", [2048, 16384, 16385, 131072, 131073, 300001])
+def test_whole_rows_at_slice_and_tile_edges(dtype, vocab):
+    """Calls of whole rows alone have kernels of their own: one slice and just over (no arrival), as many
+    tiles as a wave has lanes and one more, with the scaling and without; uniforms at both ends."""
+    from ecahlang_amd.sampling import scale_logits
+
+    rows = 6
+    g = torch.Generator().manual_seed(vocab)
+    x = (torch.randn(rows, vocab, generator=g) * 2).to(dtype)
+    x[3] = float("nan")
+    x[4, : vocab - 1] = float("-inf")
+    x = x.to(DEV)
+    u = torch.tensor([0.0, 0.9999999, 0.5, 0.3, 0.7, 0.25], device=DEV)
+    temp = torch.tensor([1.0, 0.7, 1.3, 1.0, 2.0, 0.9], device=DEV)
+    got, want = sample(x, 0, 1.0, uniform=u), _single_wg(x, 0, 1.0, u)
+    got2, want2 = sample(x, 0, 1.0, uniform=u, temperature=temp), _single_wg(scale_logits(x, temperature=temp), 0, 1.0, u)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and torch.equal(got2, want2)
+    assert got[3].item() == -1 and got[4].item() == vocab - 1
