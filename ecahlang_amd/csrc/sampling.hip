@@ -110,6 +110,16 @@ __device__ __forceinline__ float block_max(float v, float* red) {
   for (int i = 0; i < kThreads / 64; ++i) r = fmaxf(r, red[i]);
   return r;
 }
+__device__ __forceinline__ uint32_t block_max_u32(uint32_t v, uint32_t* red) {
+  v = wave_max_u32(v);
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  __syncthreads();
+  if (l == 0) red[w] = v;
+  __syncthreads();
+  uint32_t r = 0;
+  for (int i = 0; i < kThreads / 64; ++i) r = max(r, red[i]);
+  return r;
+}
 __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) { return wave_sum_u64_dpp(v); }
 __device__ __forceinline__ uint64_t block_sum_u64(uint64_t v, uint64_t* red) {
   v = wave_sum_u64(v);
@@ -121,6 +131,17 @@ __device__ __forceinline__ uint64_t block_sum_u64(uint64_t v, uint64_t* red) {
   for (int i = 0; i < kThreads / 64; ++i) r += red[i];
   return r;
 }
+
+// What the launches over many workgroups leave of a row they hand back (fallback[row]): nothing but the
+// row, or the range of keys that holds the k-th largest (known.above .. known.need).
+enum Back : int { kNotBack = 0, kBackRow = 1, kBackKeys = 2 };
+// Where a top-p row's threshold lies: its bin (-1: no mass), the mass of the bins above it, the mass to
+// reach.
+struct ToppBin {
+  uint64_t above, need;
+  float mx, scale;  // (PBins)
+  int64_t bin;
+};
 
 struct SampleLds {
   uint64_t hist[kBins];     // counts (top-k) or masses (top-p) per digit
@@ -134,18 +155,38 @@ struct SampleLds {
 template <typename T, typename RowT>
 __device__ __forceinline__ void sample_row(const RowT& row, SampleLds& L, int b, int vocab, const int32_t* top_k,
                                            int32_t top_k_all, const float* top_p, float top_p_all,
-                                           const float* uniform, int32_t* out) {
+                                           const float* uniform, int32_t* out, int how, const ToppBin* known) {
   uint64_t* s_hist = L.hist;
   uint64_t* s_tile = L.tile;
   uint64_t* s_red = L.red;
   float* s_redf = L.redf;
   uint64_t* s_scan = L.scan;
   uint32_t* s_sel = L.sel;
+  uint32_t* s_sel32 = reinterpret_cast<uint32_t*>(L.red);
   const int ntiles = row.tiles();
 
-  // ---- max logit
+  // ---- max logit; in a range of keys that holds the k-th largest, whether all are alike
   float mx = -INFINITY;
-  row.each([&](int, float x) { mx = fmaxf(mx, x); });
+  uint32_t thr = 0;
+  bool have_k = false;
+  if (how == kBackKeys) {
+    const uint32_t lo = (uint32_t)known->above, hi = (uint32_t)known->need;
+    uint32_t kmax = 0, knot = 0;  // largest key and (complemented) smallest
+    row.each([&](int, float x) {
+      mx = fmaxf(mx, x);
+      const uint32_t key = fkey(x);
+      if (key >= lo && key <= hi) {
+        kmax = max(kmax, key);
+        knot = max(knot, ~key);
+      }
+    });
+    kmax = block_max_u32(kmax, s_sel32);
+    knot = block_max_u32(knot, s_sel32);
+    have_k = kmax == ~knot;
+    thr = have_k ? kmax : 0u;
+  } else {
+    row.each([&](int, float x) { mx = fmaxf(mx, x); });
+  }
   mx = block_max(mx, s_redf);
 
   // ---- radix selection, most significant digit first.  `above` is what lies above the
@@ -208,21 +249,31 @@ __device__ __forceinline__ void sample_row(const RowT& row, SampleLds& L, int b,
 
   // ---- top-k threshold (key of the k-th largest logit; ties kept)
   const int k = top_k ? top_k[b] : top_k_all;
-  uint32_t thr = 0;
   uint64_t dummy;
-  if (k > 0 && k < vocab) thr = select(false, 0u, (uint64_t)k, dummy);
+  if (!have_k && k > 0 && k < vocab) thr = select(false, 0u, (uint64_t)k, dummy);
 
   // ---- top-p threshold over the top-k set
   const float pp = top_p ? top_p[b] : top_p_all;
   if (pp < 1.f) {
-    // mass of the top-k set first (the first level's histogram total), then the selection
-    uint64_t mk = 0;
-    row.each([&](int, float x) { if (fkey(x) >= thr) mk += fmass(x, mx); });
+    // mass of the top-k set first (the first level's histogram total), then the selection; a row handed
+    // back for its ties: their number too, since the threshold stands where the mass above it does not
+    // reach the target (5 % of a top-k row's time, so only there)
+    uint64_t mk = 0, ties = 0;
+    if (have_k) {
+      row.each([&](int, float x) {
+        const uint32_t key = fkey(x);
+        if (key >= thr) mk += fmass(x, mx);
+        ties += key == thr;
+      });
+      ties = block_sum_u64(ties, s_red) * fmass(key_float(thr), mx);
+    } else {
+      row.each([&](int, float x) { if (fkey(x) >= thr) mk += fmass(x, mx); });
+    }
     mk = block_sum_u64(mk, s_red);
     double needd = ceil((double)fmaxf(pp, 0.f) * (double)mk);
     uint64_t need = needd < 1.0 ? 1 : (uint64_t)needd;
     if (need > mk) need = mk;
-    if (mk > 0) {
+    if (mk > 0 && need + ties <= mk) {
       uint64_t tot;
       const uint32_t tp = select(true, thr, need, tot);
       thr = tp > thr ? tp : thr;
@@ -308,15 +359,16 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const T* logits, int64
                                                           const int32_t* top_k, int32_t top_k_all,
                                                           const float* top_p, float top_p_all,
                                                           const float* uniform, int32_t* out, int split,
-                                                          const int32_t* fallback) {
+                                                          const int32_t* fallback, const ToppBin* known) {
   __shared__ SampleLds L;
   const int b = blockIdx.x;
   // with the split kernels in use, all kinds but kOtherRow are theirs, except the rows they handed
   // back (fallback[b])
-  if (split && row_kind(b, vocab, top_k, top_k_all, top_p, top_p_all) != kOtherRow && !fallback[b]) return;
+  const int how = split ? fallback[b] : (int)kNotBack;
+  if (split && row_kind(b, vocab, top_k, top_k_all, top_p, top_p_all) != kOtherRow && how == kNotBack) return;
   const T* p = logits + (int64_t)b * row_stride;
   const Row<T> row{p, vocab, ((uintptr_t)p % 16) == 0};
-  sample_row<T>(row, L, b, vocab, top_k, top_k_all, top_p, top_p_all, uniform, out);
+  sample_row<T>(row, L, b, vocab, top_k, top_k_all, top_p, top_p_all, uniform, out, how, known + b);
 }
 
 // ---- Rows over many workgroups.  One workgroup per row leaves half the chip idle and is bound by the
@@ -351,13 +403,6 @@ constexpr int kPCandMax = 2048;  // candidates of a top-p row (at 512 bins and 1
 
 __host__ __device__ inline int split_tiles(int vocab) { return (vocab + kSplitTile - 1) / kSplitTile; }
 __host__ __device__ inline int split_slices(int vocab) { return (split_tiles(vocab) + kSliceTiles - 1) / kSliceTiles; }
-// Where a top-p row's threshold lies: its bin (-1: no mass), the mass of the bins above it, the mass to
-// reach.
-struct ToppBin {
-  uint64_t above, need;
-  float mx, scale;  // (PBins)
-  int64_t bin;
-};
 // The groups whose maxima a row keeps, at most kGroups of them and as small as that allows: a thread's
 // logits of 2^tg tiles of a slice, over 2^gl neighbouring threads.
 struct GroupShape {
@@ -380,13 +425,13 @@ struct SplitWs {
   uint64_t* tmass;    // [rows][ntiles] tile masses (whole and top-p rows)
   uint64_t* hist;     // [rows][slices][kPBins] masses by bin (top-p rows)
   uint64_t* cand;     // [rows][slices][kCandCap] candidates, index << 32 | key (top-p rows)
-  ToppBin* bin;       // [rows] where the threshold lies (top-p rows)
+  ToppBin* bin;       // [rows] where the threshold lies (top-p rows; top-k rows that are handed back)
   uint16_t* gmax;     // [rows][kGroups] group maxima: the keys' upper halves
   float* smax;        // [rows][slices] slice maxima
   float* smin;        // [rows][slices] slice minima
   int32_t* ncand;     // [rows][slices] candidates per slice, -1: more than kCandCap
   int32_t* counter;   // [rows][kCountStride] slices finished: a cache line each
-  int32_t* fallback;  // [rows] 1: handed back to the one-workgroup kernel
+  int32_t* fallback;  // [rows] whether handed back to the one-workgroup kernel (Back)
   GroupShape g;
 };
 __host__ __device__ inline int64_t split_ws_bytes(int rows, int vocab) {
@@ -1010,7 +1055,7 @@ __device__ __forceinline__ void topp_finish(const T* p, int vocab, int s, int b,
   const uint64_t upto = block_scan256((uint64_t)nc | ((uint64_t)(nc > kCandCap ? 1 : 0) << 40), L.redu, n64);
   const int n = (int)(uint32_t)n64;
   if ((n64 >> 40) || n > kPCandMax) {  // (uniform)
-    if (t == 0) ws.fallback[b] = 1;
+    if (t == 0) ws.fallback[b] = kBackRow;
     return;
   }
   if (t < S) L.off[t] = (int)(uint32_t)upto - nc;
@@ -1096,11 +1141,20 @@ __device__ __forceinline__ void topp_finish(const T* p, int vocab, int s, int b,
 // candidates: over them, the largest T with #{key >= T} >= k is T* itself.  sample_row's rule on the
 // candidates alone (T*, the top-p threshold, the inverse CDF in vocabulary order, with the same integer
 // masses) gives the same token.  Where more than kTopkCands logits lie above T0 (large logits close
-// together in the vocabulary), the bound is raised first.  Rows that cannot be finished this way (ties
-// beyond kTopkCands, fewer than k numbers) are handed back to sample_kernel through `fallback`.
+// together in the vocabulary), the bound is raised first.  Rows with more ties than this takes are handed
+// back to sample_kernel, with the range of keys that holds T*.
 constexpr int kRadixBins = 2048;  // the largest digit (11 bits) of the radix selection
 
 constexpr int kTopkCands = 1024;  // candidates of a top-k row at most
+constexpr int kPairsMax = 512;    // of which kept by the filter (all ties but 255): comparing each with all takes
+                                  // 28 us a stage at 512 and 110 at 1000; a call on 1000 equal logits 160 us that way,
+                                  // 32 with the one-workgroup kernel going on from the known threshold
+// A top-k row whose k-th largest key lies in [lo, hi], to the one-workgroup kernel.
+__device__ __forceinline__ void hand_back(const SplitWs& ws, int b, uint32_t lo, uint32_t hi) {
+  ws.bin[b].above = lo;
+  ws.bin[b].need = hi;
+  ws.fallback[b] = kBackKeys;
+}
 struct TopkLds {
   union {
     int h[kRadixBins];  // (16-byte vector accesses)
@@ -1161,9 +1215,9 @@ __device__ __forceinline__ void clear_hist(TopkLds& L) {
 }
 
 // A bound that k of the row's n group maxima reach, and no more than the upper half of the k-th largest
-// of them (0: fewer than k groups), by bisection on its bits; every wave for itself, the maxima in its
+// of them (0: fewer than k groups), and the largest of all (top), by bisection on its bits; every wave for itself, the maxima in its
 // registers.
-__device__ __forceinline__ uint32_t group_bound(const uint16_t* gm, int n, int k) {
+__device__ __forceinline__ uint32_t group_bound(const uint16_t* gm, int n, int k, uint32_t& top) {
   constexpr int R = kGroups / kWave / 4;
   const int lane = threadIdx.x & (kWave - 1);
   uint32_t v[kGroups / kWave];
@@ -1186,6 +1240,7 @@ __device__ __forceinline__ uint32_t group_bound(const uint16_t* gm, int n, int k
   }
   hi = wave_max_u32(hi);
   lo = ~wave_max_u32(~lo);
+  top = hi;
   if (n < k) return 0;
   const uint32_t diff = hi ^ min(lo, hi);
   uint32_t bit = diff ? 0x80000000u >> __builtin_clz(diff) : 0u;
@@ -1284,6 +1339,10 @@ __device__ __forceinline__ void topk_merge(int b, int n, int k, float pp, const 
       if (t == 0) L.top = 0u;
       __syncthreads();
       m = L.na;
+      if (m > kPairsMax) {  // (uniform)
+        if (t == 0) hand_back(ws, b, thr, thr);
+        return;
+      }
       const uint64_t kmass = L.sum;
       const double needd = ceil((double)fmaxf(pp, 0.f) * (double)kmass);
       need = needd < 1.0 ? 1 : (uint64_t)needd;
@@ -1393,7 +1452,13 @@ __device__ __forceinline__ void topk_row(const T* p, int vocab, bool vec, int b,
   const GroupShape& g = ws.g;
   const uint16_t* gm = ws.gmax + (int64_t)b * kGroups;
   if (t == 0) L.n = L.na = 0;
-  uint32_t ts = max(group_bound(gm, g.n, k), 1u);  // (0 is no number)
+  uint32_t top, ts = group_bound(gm, g.n, k, top);
+  // A logit 23 or more below the largest has no mass, so it is never the token and never moves the top-p
+  // threshold: the bound need not go below that (rows masked with -inf, fewer than k numbers), and fewer
+  // than k candidates are then all that is kept.  (24: top is a little below the largest, and differences
+  // are rounded.)
+  const float least = half_key_float(top) - 24.f;
+  ts = max(ts, fkey(least) >> 16);
   __syncthreads();
   for (int i = t; i < g.n; i += kSplitThreads)
     if (gm[i] >= ts) L.active[atomicAdd(&L.na, 1)] = (uint16_t)i;
@@ -1402,7 +1467,7 @@ __device__ __forceinline__ void topk_row(const T* p, int vocab, bool vec, int b,
   const int total = L.na << (g.tg + g.gl);
 #pragma unroll 1
   for (bool raised = false;; raised = true) {
-    const float lim = half_key_float(ts);
+    const float lim = fmaxf(half_key_float(ts), least);
     each_active<2>(p, vocab, vec, av, total, [&](int i0, const float (&x)[2][8], const bool (&ok)[2][8]) __attribute__((always_inline)) {
       uint32_t in = 0;
 #pragma unroll
@@ -1444,10 +1509,17 @@ __device__ __forceinline__ void topk_row(const T* p, int vocab, bool vec, int b,
       ts = max(prefix, floor_key);
       if (L.cnt <= kTopkCands) break;  // (uniform)
     }
+    if (L.cnt > kTopkCands) {  // (uniform) more than fit share the upper half of the k-th largest key
+      if (t == 0) hand_back(ws, b, ts << 16, ts << 16 | 0xFFFFu);
+      return;
+    }
   }
   const int n = L.n;
-  if (n > kTopkCands || n < k) {  // (uniform; fewer than k: the row has fewer numbers)
-    if (t == 0) ws.fallback[b] = 1;
+  if (n == 0 || n > kTopkCands) {  // (uniform) no number in the row; zeros of both signs at the bound
+    if (t == 0) {
+      if (n == 0) out[b] = -1;
+      else ws.fallback[b] = kBackRow;
+    }
     return;
   }
   topk_merge(b, n, k, pp, uniform, out, ws, L);
@@ -1539,7 +1611,7 @@ int launch_sample(const T* logits, int64_t row_stride, int rows, int vocab, cons
   }
   if (!plan.split || plan.other || plan.topk || plan.topp)  // (rows may be handed back)
     hipLaunchKernelGGL(sample_kernel<T>, dim3(rows), dim3(kThreads), 0, s, logits, row_stride, vocab, top_k,
-                       top_k_all, top_p, top_p_all, uniform, out, plan.split ? 1 : 0, w.fallback);
+                       top_k_all, top_p, top_p_all, uniform, out, plan.split ? 1 : 0, w.fallback, w.bin);
   return (int)hipGetLastError();
 }
 

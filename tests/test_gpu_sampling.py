@@ -407,3 +407,46 @@ def test_whole_rows_at_slice_and_tile_edges(dtype, vocab):
     torch.cuda.synchronize()
     assert torch.equal(got, want) and torch.equal(got2, want2)
     assert got[3].item() == -1 and got[4].item() == vocab - 1
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vocab", [1000, 20000, 151936])
+def test_top_k_rows_with_many_ties_or_few_numbers(dtype, vocab):
+    """Top-k rows whose threshold hundreds or all of the logits share (kept by the split kernels up to 512,
+    finished from the known threshold above), whose upper key halves agree while the keys differ, and rows
+    with fewer than k logits that carry mass: the token is the one-workgroup kernel's, bit for bit."""
+    rows = 14
+    g = torch.Generator().manual_seed(vocab + 5)
+    x = torch.randn(rows, vocab, generator=g)
+    x[0] = 0.25                                              # flat
+    x[1] = 0.25
+    x[1, ::3] = -2.0                                         # two values
+    x[2] = -1.0
+    x[2, 7::vocab // 9] = 3.0                                # a few above the ties
+    x[3, :] = float("-inf")
+    x[3, 5::vocab // 11] = 1.0                               # masked: about 11 left
+    x[4, :] = float("nan")
+    x[4, 3::vocab // 30] = torch.randn(x[4, 3::vocab // 30].shape, generator=g)
+    x[5] = torch.round(x[5] * 2) / 2                         # coarse steps
+    x[6] = 5.0 + 1e-6 * torch.arange(vocab)                  # (fp32) distinct keys, few upper halves
+    x[7] = -0.0
+    x[7, ::2] = 0.0
+    x[8, 3] = 60.0                                           # one logit far above the rest: all others without mass
+    x[9, 3] = float("inf")
+    x[10] = float("-inf")
+    x[11] = torch.round(x[11]) * 1e4                         # far apart, tied
+    n = min(600, vocab - 1)
+    x[12] = -30.0
+    x[12, :n] = 2.0                                          # 600 ties, the rest without mass
+    x[13] = -30.0
+    x[13, vocab - 400:] = 2.0                                # 400 ties
+    x = x.to(dtype).to(DEV)
+    for trial in range(3):
+        u = torch.rand(rows, generator=g).to(DEV)
+        if trial == 0:
+            u[:] = 0.9999999
+        for k in (1, 8, 50, 256):
+            for p in (1.0, 0.9, 0.3, 1e-6):
+                got, want = sample(x, k, p, uniform=u), _single_wg(x, k, p, u)
+                torch.cuda.synchronize()
+                assert torch.equal(got, want), (k, p, trial, (got != want).nonzero().flatten().tolist())
