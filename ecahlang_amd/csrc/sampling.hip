@@ -133,14 +133,23 @@ __device__ __forceinline__ uint64_t block_sum_u64(uint64_t v, uint64_t* red) {
 }
 
 // What the launches over many workgroups leave of a row they hand back (fallback[row]): nothing but the
-// row, or the range of keys that holds the k-th largest (known.above .. known.need).
-enum Back : int { kNotBack = 0, kBackRow = 1, kBackKeys = 2 };
+// row, the range of keys that holds the k-th largest (known.above .. known.need), or the bin that holds the
+// top-p threshold.
+enum Back : int { kNotBack = 0, kBackRow = 1, kBackKeys = 2, kBackBin = 3 };
+constexpr int kPBins = 1024;  // bins of a top-p row's mass
 // Where a top-p row's threshold lies: its bin (-1: no mass), the mass of the bins above it, the mass to
 // reach.
 struct ToppBin {
   uint64_t above, need;
   float mx, scale;  // (PBins)
   int64_t bin;
+};
+struct PBins {
+  float mx, scale;
+  __device__ __forceinline__ PBins(float mx_, float scale_) : mx(mx_), scale(scale_) {}
+  __device__ __forceinline__ PBins(float2 range)
+      : mx(range.x), scale((float)kPBins / fmaxf(fminf(range.x - range.y, 23.f), 1e-20f)) {}
+  __device__ __forceinline__ int of(float x) const { return min((int)((mx - x) * scale), kPBins - 1); }
 };
 
 struct SampleLds {
@@ -151,6 +160,88 @@ struct SampleLds {
   uint64_t scan[kThreads / 64];
   uint32_t sel[4];
 };
+
+// A top-p row's threshold where its bin is known but holds more logits than split_finish_kernel takes: the
+// bin's mass in finer bins, unless all its keys are alike (ties are why there are so many), then the keys of
+// the one that the target falls in, with a bisection on their bits.  False if there are too many different
+// ones.  One or two passes over the row in place of five (128 rows of 151,936 logits in steps of 1/4: 119 us a call,
+// 223 when such rows started over, 151 when all top-p rows ran on one workgroup).
+template <typename RowT>
+__device__ __forceinline__ bool bin_threshold(const RowT& row, SampleLds& L, const ToppBin& tb, uint32_t& thr) {
+  const PBins bins(tb.mx, tb.scale);
+  const int t = threadIdx.x, cb = (int)tb.bin;
+  // the finer bin of a logit, -1 outside the bin or without mass; f: its mass
+  auto finer = [&](float x, uint64_t& f) __attribute__((always_inline)) -> int {
+    if (bins.of(x) != cb) return -1;
+    f = fmass(x, tb.mx);
+    return f ? min((int)(__builtin_fmaf(tb.mx - x, tb.scale, -(float)cb) * (float)kBins), kBins - 1) : -1;
+  };
+  static_assert(kBins == 2 * kThreads, "two finer bins a thread");
+  L.hist[2 * t] = L.hist[2 * t + 1] = 0;
+  if (t == 0) L.sel[3] = 0;
+  __syncthreads();
+  uint32_t kmax = 0, knot = 0;  // largest key and (complemented) smallest
+  row.each([&](int, float x) {
+    uint64_t f;
+    const int i = finer(x, f);
+    if (i >= 0) {
+      atomicAdd((unsigned long long*)&L.hist[i], (unsigned long long)f);
+      kmax = max(kmax, fkey(x));
+      knot = max(knot, ~fkey(x));
+    }
+  });
+  kmax = block_max_u32(kmax, reinterpret_cast<uint32_t*>(L.red));
+  knot = block_max_u32(knot, reinterpret_cast<uint32_t*>(L.red));
+  thr = kmax;
+  if (kmax == ~knot) return true;  // (uniform)
+  const uint64_t h0 = L.hist[2 * t], own = h0 + L.hist[2 * t + 1];
+  uint64_t upto = own;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint64_t v = __shfl_up(upto, o, kWave);
+    if ((t & 63) >= o) upto += v;
+  }
+  if ((t & 63) == 63) L.scan[t >> 6] = upto;
+  __syncthreads();
+  upto += tb.above;
+  for (int i = 0; i < t >> 6; ++i) upto += L.scan[i];
+  if (upto >= tb.need && upto - own < tb.need) {
+    const bool second = upto - own + h0 < tb.need;
+    const uint64_t before = upto - own + (second ? h0 : 0);
+    L.sel[0] = 2 * t + (second ? 1 : 0);
+    L.sel[1] = (uint32_t)before;
+    L.sel[2] = (uint32_t)(before >> 32);
+  }
+  __syncthreads();  // (and every thread has read the finer bins)
+  const int fb = (int)L.sel[0];
+  const uint64_t above = (uint64_t)L.sel[1] | (uint64_t)L.sel[2] << 32;
+  uint32_t* keys = reinterpret_cast<uint32_t*>(L.hist);
+  constexpr int kKeys = 2 * kBins;
+  kmax = knot = 0;
+  row.each([&](int, float x) {
+    uint64_t f;
+    if (finer(x, f) == fb) {
+      const uint32_t key = fkey(x), pos = atomicAdd(&L.sel[3], 1u);
+      if (pos < kKeys) keys[pos] = key;
+      kmax = max(kmax, key);
+      knot = max(knot, ~key);
+    }
+  });
+  kmax = block_max_u32(kmax, reinterpret_cast<uint32_t*>(L.red));  // (and the keys are written)
+  knot = block_max_u32(knot, reinterpret_cast<uint32_t*>(L.red));
+  const int n = (int)L.sel[3];
+  thr = kmax;
+  if (kmax == ~knot) return true;
+  if (n > kKeys) return false;
+  // the largest value that keys with enough mass reach: of the bits in which they differ, from the highest
+  uint32_t bit = 0x80000000u >> __builtin_clz(kmax ^ ~knot);
+  for (thr = kmax & ~(2 * bit - 1); bit; bit >>= 1) {
+    uint64_t m = 0;
+    for (int i = t; i < n; i += kThreads) m += keys[i] >= (thr | bit) ? fmass(key_float(keys[i]), tb.mx) : 0;
+    if (above + block_sum_u64(m, L.red) >= tb.need) thr |= bit;
+  }
+  return true;
+}
 
 template <typename T, typename RowT>
 __device__ __forceinline__ void sample_row(const RowT& row, SampleLds& L, int b, int vocab, const int32_t* top_k,
@@ -184,10 +275,12 @@ __device__ __forceinline__ void sample_row(const RowT& row, SampleLds& L, int b,
     knot = block_max_u32(knot, s_sel32);
     have_k = kmax == ~knot;
     thr = have_k ? kmax : 0u;
-  } else {
+  } else if (how != kBackBin) {
     row.each([&](int, float x) { mx = fmaxf(mx, x); });
   }
-  mx = block_max(mx, s_redf);
+  mx = how == kBackBin ? known->mx : block_max(mx, s_redf);
+  const bool have_p = how == kBackBin && bin_threshold(row, L, *known, thr);
+  if (!have_k && !have_p) thr = 0;
 
   // ---- radix selection, most significant digit first.  `above` is what lies above the
   // current prefix (a count for top-k, a mass for top-p); the digit where the running total
@@ -254,7 +347,7 @@ __device__ __forceinline__ void sample_row(const RowT& row, SampleLds& L, int b,
 
   // ---- top-p threshold over the top-k set
   const float pp = top_p ? top_p[b] : top_p_all;
-  if (pp < 1.f) {
+  if (pp < 1.f && !have_p) {
     // mass of the top-k set first (the first level's histogram total), then the selection; a row handed
     // back for its ties: their number too, since the threshold stands where the mass above it does not
     // reach the target (5 % of a top-k row's time, so only there)
@@ -397,7 +490,6 @@ constexpr int kMaxSplitTiles = 2048;           // vocabularies up to 4 M
 constexpr int kCandCap = 512;    // candidates a slice hands over for a top-p row
 
 constexpr int kGroups = 1024;    // group maxima per row at most
-constexpr int kPBins = 1024;     // bins of a top-p row's mass
 constexpr int kPCandMax = 2048;  // candidates of a top-p row (at 512 bins and 1024 of them, a wide body at a high
                                  // temperature went over, and the one row handed back took 45 us)
 
@@ -906,14 +998,6 @@ __device__ __forceinline__ void whole_slice(const T* p, int vocab, bool vec, con
 // that finishes the row's last slice finds it.  In the next launch logits in the bins above are kept,
 // those in it are candidates (a few hundred of 151,936), and the last slice's workgroup selects the
 // exact threshold among them.  That launch reads only the groups whose largest logit reaches the bin.
-struct PBins {
-  float mx, scale;
-  __device__ __forceinline__ PBins(float mx_, float scale_) : mx(mx_), scale(scale_) {}
-  __device__ __forceinline__ PBins(float2 range)
-      : mx(range.x), scale((float)kPBins / fmaxf(fminf(range.x - range.y, 23.f), 1e-20f)) {}
-  __device__ __forceinline__ int of(float x) const { return min((int)((mx - x) * scale), kPBins - 1); }
-};
-
 template <typename T>
 __device__ __forceinline__ void topp_hist(const T* p, int vocab, bool vec, const SliceLoad<T>& sl, int s, int b, int S,
                                           float pp, int32_t* out, const SplitWs& ws, uint64_t* s_hist, float* redf,
@@ -966,6 +1050,13 @@ __device__ __forceinline__ void topp_hist(const T* p, int vocab, bool vec, const
       e += on ? 1 : 0;
     }
     ws.bin[b] = ToppBin{above, need, bins.mx, bins.scale, 4 * t + e};
+    // at least this many logits carry the bin's mass; too many for the next launch, which then leaves the
+    // row alone (ties, mostly)
+    uint64_t mine = 0;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) mine = e == x ? hb[x] : mine;
+    const float most = __expf(-(float)(4 * t + e) / bins.scale) * 4294967296.0f;  // (of one of them)
+    if ((float)mine > (float)min(kPCandMax, S * kCandCap) * (1.01f * most + 1.f)) ws.fallback[b] = kBackBin;
   }
 }
 
@@ -991,7 +1082,7 @@ __device__ __forceinline__ void topp_finish(const T* p, int vocab, int s, int b,
   const ToppBin tb = ws.bin[b];
   const int cb = (int)tb.bin;
   const uint64_t above = tb.above, need = tb.need;
-  if (cb < 0) return;  // (uniform; the token is written)
+  if (cb < 0 || ws.fallback[b] != kNotBack) return;  // (uniform; the token is written, or the row handed back)
   if (t == 0) L.n = 0, L.diff = 0;
   const PBins bins(tb.mx, tb.scale);
   __syncthreads();
@@ -1055,7 +1146,7 @@ __device__ __forceinline__ void topp_finish(const T* p, int vocab, int s, int b,
   const uint64_t upto = block_scan256((uint64_t)nc | ((uint64_t)(nc > kCandCap ? 1 : 0) << 40), L.redu, n64);
   const int n = (int)(uint32_t)n64;
   if ((n64 >> 40) || n > kPCandMax) {  // (uniform)
-    if (t == 0) ws.fallback[b] = kBackRow;
+    if (t == 0) ws.fallback[b] = kBackBin;
     return;
   }
   if (t < S) L.off[t] = (int)(uint32_t)upto - nc;

@@ -450,3 +450,37 @@ def test_top_k_rows_with_many_ties_or_few_numbers(dtype, vocab):
                 got, want = sample(x, k, p, uniform=u), _single_wg(x, k, p, u)
                 torch.cuda.synchronize()
                 assert torch.equal(got, want), (k, p, trial, (got != want).nonzero().flatten().tolist())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vocab", [3000, 20000, 151936])
+def test_top_p_rows_whose_bin_overflows(dtype, vocab):
+    """Top-p rows with more logits in the threshold's bin than the finish takes: ties, a narrow body under a
+    far peak, a cluster of different keys around zero, one value more than the key buffer holds.  The
+    one-workgroup kernel goes on from the bin; the token is the one it finds by itself, bit for bit."""
+    rows = 10
+    g = torch.Generator().manual_seed(vocab + 6)
+    x = torch.randn(rows, vocab, generator=g)
+    x[0] = 0.25
+    x[1] = torch.round(x[1] * 4) / 4
+    x[2] = torch.round(x[2])
+    x[3] = x[3] * 0.01
+    x[3, 9] = 12.0                                            # the body carries about as much as the peak
+    x[4] = x[4] * 1e-4
+    x[4, 9] = 11.0
+    x[5] = x[5] * 1e-30                                       # different keys over many exponents, one bin
+    x[5, 11] = 9.0
+    x[6] = -30.0
+    x[6, : vocab // 2] = 1.0
+    x[6, vocab // 2: vocab // 2 + 900] = 1.5
+    x[7] = torch.where(torch.arange(vocab) % 2 == 0, 2.0, 2.0 + 1e-6)
+    x[8, ::2] = float("nan")
+    x[8, 1::2] = -0.5
+    x[9] = torch.round(x[9] * 64) / 64 * 0.05
+    x = x.to(dtype).to(DEV)
+    for trial in range(2):
+        u = torch.rand(rows, generator=g).to(DEV)
+        for p in (0.05, 0.3, 0.5, 0.9, 0.97, 0.999):
+            got, want = sample(x, 0, p, uniform=u), _single_wg(x, 0, p, u)
+            torch.cuda.synchronize()
+            assert torch.equal(got, want), (p, trial, (got != want).nonzero().flatten().tolist())
