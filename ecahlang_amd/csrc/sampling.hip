@@ -150,51 +150,28 @@ struct PBins {
   __device__ __forceinline__ PBins(float2 range)
       : mx(range.x), scale((float)kPBins / fmaxf(fminf(range.x - range.y, 23.f), 1e-20f)) {}
   __device__ __forceinline__ int of(float x) const { return min((int)((mx - x) * scale), kPBins - 1); }
+  // The finer bin of a logit of bin b.
+  __device__ __forceinline__ int finer(float x, int b) const {
+    return min((int)(__builtin_fmaf(mx - x, scale, -(float)b) * (float)kPBins), kPBins - 1);
+  }
 };
 
 struct SampleLds {
   uint64_t hist[kBins];     // counts (top-k) or masses (top-p) per digit
   uint64_t tile[kMaxTiles];  // kept mass per tile
+  uint64_t tile2[kMaxTiles];  // (row_from_bin: mass in the finer bin; the candidates' masses)
   uint64_t red[kThreads / 64];
   float redf[kThreads / 64];
   uint64_t scan[kThreads / 64];
   uint32_t sel[4];
 };
 
-// A top-p row's threshold where its bin is known but holds more logits than split_finish_kernel takes: the
-// bin's mass in finer bins, unless all its keys are alike (ties are why there are so many), then the keys of
-// the one that the target falls in, with a bisection on their bits.  False if there are too many different
-// ones.  One or two passes over the row in place of five (128 rows of 151,936 logits in steps of 1/4: 119 us a call,
-// 223 when such rows started over, 151 when all top-p rows ran on one workgroup).
-template <typename RowT>
-__device__ __forceinline__ bool bin_threshold(const RowT& row, SampleLds& L, const ToppBin& tb, uint32_t& thr) {
-  const PBins bins(tb.mx, tb.scale);
-  const int t = threadIdx.x, cb = (int)tb.bin;
-  // the finer bin of a logit, -1 outside the bin or without mass; f: its mass
-  auto finer = [&](float x, uint64_t& f) __attribute__((always_inline)) -> int {
-    if (bins.of(x) != cb) return -1;
-    f = fmass(x, tb.mx);
-    return f ? min((int)(__builtin_fmaf(tb.mx - x, tb.scale, -(float)cb) * (float)kBins), kBins - 1) : -1;
-  };
-  static_assert(kBins == 2 * kThreads, "two finer bins a thread");
-  L.hist[2 * t] = L.hist[2 * t + 1] = 0;
-  if (t == 0) L.sel[3] = 0;
-  __syncthreads();
-  uint32_t kmax = 0, knot = 0;  // largest key and (complemented) smallest
-  row.each([&](int, float x) {
-    uint64_t f;
-    const int i = finer(x, f);
-    if (i >= 0) {
-      atomicAdd((unsigned long long*)&L.hist[i], (unsigned long long)f);
-      kmax = max(kmax, fkey(x));
-      knot = max(knot, ~fkey(x));
-    }
-  });
-  kmax = block_max_u32(kmax, reinterpret_cast<uint32_t*>(L.red));
-  knot = block_max_u32(knot, reinterpret_cast<uint32_t*>(L.red));
-  thr = kmax;
-  if (kmax == ~knot) return true;  // (uniform)
-  const uint64_t h0 = L.hist[2 * t], own = h0 + L.hist[2 * t + 1];
+// The bins of a row whose masses are in L.hist[0 .. kPBins): the one at which the mass from the first one on,
+// `above` included, reaches need; above becomes the mass before it.
+__device__ __forceinline__ int mass_bin(SampleLds& L, uint64_t& above, uint64_t need) {
+  static_assert(kPBins == kThreads, "a bin a thread");
+  const int t = threadIdx.x;
+  const uint64_t own = L.hist[t];
   uint64_t upto = own;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -203,43 +180,118 @@ __device__ __forceinline__ bool bin_threshold(const RowT& row, SampleLds& L, con
   }
   if ((t & 63) == 63) L.scan[t >> 6] = upto;
   __syncthreads();
-  upto += tb.above;
+  upto += above;
   for (int i = 0; i < t >> 6; ++i) upto += L.scan[i];
-  if (upto >= tb.need && upto - own < tb.need) {
-    const bool second = upto - own + h0 < tb.need;
-    const uint64_t before = upto - own + (second ? h0 : 0);
-    L.sel[0] = 2 * t + (second ? 1 : 0);
-    L.sel[1] = (uint32_t)before;
-    L.sel[2] = (uint32_t)(before >> 32);
+  if (upto >= need && upto - own < need) {
+    L.sel[0] = t;
+    L.sel[1] = (uint32_t)(upto - own);
+    L.sel[2] = (uint32_t)((upto - own) >> 32);
   }
-  __syncthreads();  // (and every thread has read the finer bins)
-  const int fb = (int)L.sel[0];
-  const uint64_t above = (uint64_t)L.sel[1] | (uint64_t)L.sel[2] << 32;
-  uint32_t* keys = reinterpret_cast<uint32_t*>(L.hist);
-  constexpr int kKeys = 2 * kBins;
-  kmax = knot = 0;
+  __syncthreads();
+  above = (uint64_t)L.sel[1] | (uint64_t)L.sel[2] << 32;
+  return (int)L.sel[0];
+}
+
+// A top-p row whose bin is known but holds more logits than split_finish_kernel takes.  One pass over the row
+// for the bin's mass in finer bins and its range of keys: mostly they are alike (ties are why there are so
+// many), and that is the threshold.  Else a second takes the tiles' mass before the finer bin that the target
+// falls in, and that bin's logits, among which the threshold is found (tiles: the tiles' kept masses are in
+// L.tile).  False if there are too many of them.  (128 rows of 151,936 logits in steps of 1/4: 113 us a call,
+// 223 when such rows started over, 151 when all top-p rows ran on one workgroup.)
+template <typename RowT>
+__device__ __forceinline__ bool row_from_bin(const RowT& row, SampleLds& L, const ToppBin& tb, uint32_t& thr, bool& tiles) {
+  constexpr int kPairs = 256;  // keys compared each with all
+  const PBins bins(tb.mx, tb.scale);
+  const int t = threadIdx.x, cb = (int)tb.bin;
+  tiles = false;
+  L.hist[t] = 0;
+  __syncthreads();
+  uint32_t kmax = 0, knot = 0;  // largest key and (complemented) smallest
   row.each([&](int, float x) {
-    uint64_t f;
-    if (finer(x, f) == fb) {
+    if (bins.of(x) != cb) return;
+    const uint64_t f = fmass(x, tb.mx);
+    if (f) {
+      atomicAdd((unsigned long long*)&L.hist[bins.finer(x, cb)], (unsigned long long)f);
+      kmax = max(kmax, fkey(x));
+      knot = max(knot, ~fkey(x));
+    }
+  });
+  kmax = block_max_u32(kmax, reinterpret_cast<uint32_t*>(L.red));  // (and the finer bins are complete)
+  knot = block_max_u32(knot, reinterpret_cast<uint32_t*>(L.red));
+  thr = kmax;
+  if (kmax == ~knot) return true;  // (uniform)
+  tiles = true;
+  uint64_t above = tb.above;
+  const int fb = mass_bin(L, above, tb.need);
+  const int ntiles = row.tiles();
+  for (int i = t; i < ntiles; i += kThreads) L.tile[i] = L.tile2[i] = 0;
+  if (t == 0) L.sel[3] = 0;
+  __syncthreads();  // (and every thread has read the finer bins)
+  kmax = knot = 0;
+  uint64_t m = 0, m2 = 0;
+  int cur = 0;
+  auto flush = [&]() __attribute__((always_inline)) {
+    if (m) atomicAdd((unsigned long long*)&L.tile[cur], (unsigned long long)m);
+    if (m2) atomicAdd((unsigned long long*)&L.tile2[cur], (unsigned long long)m2);
+    m = m2 = 0;
+  };
+  row.each([&](int i, float x) {
+    const int tile = i / (kThreads * RowT::E);
+    if (tile != cur) {  // (tiles come in increasing order)
+      flush();
+      cur = tile;
+    }
+    const int bin = bins.of(x);
+    if (bin > cb) return;
+    const uint64_t f = fmass(x, tb.mx);
+    const int fi = bin < cb ? -1 : bins.finer(x, cb);
+    m += fi < fb ? f : 0;
+    if (fi == fb && f) {
+      m2 += f;
       const uint32_t key = fkey(x), pos = atomicAdd(&L.sel[3], 1u);
-      if (pos < kKeys) keys[pos] = key;
+      if (pos < kBins) L.hist[pos] = (uint64_t)(uint32_t)i << 32 | key;
       kmax = max(kmax, key);
       knot = max(knot, ~key);
     }
   });
-  kmax = block_max_u32(kmax, reinterpret_cast<uint32_t*>(L.red));  // (and the keys are written)
+  flush();
+  kmax = block_max_u32(kmax, reinterpret_cast<uint32_t*>(L.red));  // (and the candidates are written)
   knot = block_max_u32(knot, reinterpret_cast<uint32_t*>(L.red));
   const int n = (int)L.sel[3];
   thr = kmax;
-  if (kmax == ~knot) return true;
-  if (n > kKeys) return false;
-  // the largest value that keys with enough mass reach: of the bits in which they differ, from the highest
-  uint32_t bit = 0x80000000u >> __builtin_clz(kmax ^ ~knot);
-  for (thr = kmax & ~(2 * bit - 1); bit; bit >>= 1) {
-    uint64_t m = 0;
-    for (int i = t; i < n; i += kThreads) m += keys[i] >= (thr | bit) ? fmass(key_float(keys[i]), tb.mx) : 0;
-    if (above + block_sum_u64(m, L.red) >= tb.need) thr |= bit;
+  if (kmax == ~knot) {
+    for (int i = t; i < ntiles; i += kThreads) L.tile[i] += L.tile2[i];
+    __syncthreads();
+    return true;
   }
+  if (n > kBins) return false;
+  if (n <= kPairs) {
+    // the largest key that enough mass reaches: each against all
+    if (t < n) L.tile2[t] = fmass(key_float((uint32_t)L.hist[t]), tb.mx);
+    __syncthreads();
+    const uint32_t key = (uint32_t)L.hist[min(t, n - 1)];
+    uint64_t sum = above;
+    for (int i = 0; i < n; ++i) sum += (uint32_t)L.hist[i] >= key ? L.tile2[i] : 0;
+    thr = block_max_u32(sum >= tb.need ? key : 0u, reinterpret_cast<uint32_t*>(L.red));
+  } else {
+    // the largest value that it reaches: of the bits in which the keys differ, from the highest
+    uint32_t bit = 0x80000000u >> __builtin_clz(kmax ^ ~knot);
+    for (thr = kmax & ~(2 * bit - 1); bit; bit >>= 1) {
+      uint64_t sum = 0;
+      for (int i = t; i < n; i += kThreads) {
+        const uint32_t key = (uint32_t)L.hist[i];
+        sum += key >= (thr | bit) ? fmass(key_float(key), tb.mx) : 0;
+      }
+      if (above + block_sum_u64(sum, L.red) >= tb.need) thr |= bit;
+    }
+  }
+  for (int i = t; i < n; i += kThreads) {
+    const uint32_t key = (uint32_t)L.hist[i];
+    if (key >= thr)
+      atomicAdd((unsigned long long*)&L.tile[(uint32_t)(L.hist[i] >> 32) / (kThreads * RowT::E)],
+                (unsigned long long)fmass(key_float(key), tb.mx));
+  }
+  __syncthreads();
   return true;
 }
 
@@ -279,7 +331,9 @@ __device__ __forceinline__ void sample_row(const RowT& row, SampleLds& L, int b,
     row.each([&](int, float x) { mx = fmaxf(mx, x); });
   }
   mx = how == kBackBin ? known->mx : block_max(mx, s_redf);
-  const bool have_p = how == kBackBin && bin_threshold(row, L, *known, thr);
+  bool have_tiles = false;
+  const bool have_p = how == kBackBin && row_from_bin(row, L, *known, thr, have_tiles);
+  have_tiles = have_tiles && have_p;
   if (!have_k && !have_p) thr = 0;
 
   // ---- radix selection, most significant digit first.  `above` is what lies above the
@@ -374,9 +428,9 @@ __device__ __forceinline__ void sample_row(const RowT& row, SampleLds& L, int b,
   }
 
   // ---- sample: kept mass per tile, the tile holding the target, then the thread and token
-  for (int t = threadIdx.x; t < ntiles; t += kThreads) s_tile[t] = 0;
-  __syncthreads();
-  {
+  if (!have_tiles) {
+    for (int t = threadIdx.x; t < ntiles; t += kThreads) s_tile[t] = 0;
+    __syncthreads();
     constexpr int E = RowT::E;
     uint64_t m = 0;
     int cur = 0;
@@ -1056,7 +1110,9 @@ __device__ __forceinline__ void topp_hist(const T* p, int vocab, bool vec, const
 #pragma unroll
     for (int x = 0; x < 4; ++x) mine = e == x ? hb[x] : mine;
     const float most = __expf(-(float)(4 * t + e) / bins.scale) * 4294967296.0f;  // (of one of them)
-    if ((float)mine > (float)min(kPCandMax, S * kCandCap) * (1.01f * most + 1.f)) ws.fallback[b] = kBackBin;
+    // (several slices do not share them evenly)
+    const int room = min(kPCandMax, S == 1 ? kCandCap : S * (kCandCap - kCandCap / 8));
+    if ((float)mine > (float)room * (1.01f * most + 1.f)) ws.fallback[b] = kBackBin;
   }
 }
 
