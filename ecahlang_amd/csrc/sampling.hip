@@ -1922,7 +1922,12 @@ extern "C" int pkv_scaled_top_k_top_p_sampling(const void* logits, int64_t row_s
   if (dtype != kF16 && dtype != kBF16 && dtype != kF32) return kBadDType;
   if (!row_fits(vocab, 4)) return kBadArg;  // (the scaled rows are fp32, whatever the logits)
   const SamplePlan plan(rows, vocab, top_k, top_k_all, top_p, top_p_all, workspace, workspace_bytes);
-  if (!plan.split || ((uintptr_t)scaled | (uintptr_t)(scaled_stride * 4)) % 16) {
+  // Few slices of over three tiles: the scan's workgroups would scale a slice each, a tile after the other,
+  // while most of the chip is idle; scale_logits spreads the tiles (one row of 32,000 / 151,936 logits, no filter:
+  // 20.8 / 21.0 us in one launch, 16.7 / 17.1 in two; 8 of 151,936, 80 slices: 22.7, 19.8; 160 slices: 23.3, 23.2;
+  // 320: 30.0, 28.4; 640: 38.6, 40.1; one row of 4000, two tiles: 10.3, 11.6).
+  const bool few = split_tiles(vocab) > 3 && (int64_t)rows * split_slices(vocab) <= 128;
+  if (!plan.split || few || ((uintptr_t)scaled | (uintptr_t)(scaled_stride * 4)) % 16) {
     const int rc = pkv_scale_logits(logits, row_stride, rows, vocab, dtype, penalty, penalty_stride, penalty_slots,
                                     penalty_rows, temperature, scaled, scaled_stride, stream);
     return rc ? rc : sample_entry(scaled, scaled_stride, rows, vocab, kF32, top_k, top_k_all, top_p, top_p_all, uniform,

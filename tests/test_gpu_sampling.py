@@ -394,14 +394,14 @@ def test_whole_rows_at_slice_and_tile_edges(dtype, vocab):
     tiles as a wave has lanes and one more, with the scaling and without; uniforms at both ends."""
     from ecahlang_amd.sampling import scale_logits
 
-    rows = 6
+    rows = 24  # (the scaling rides in the first launch up to three tiles a row, and at over 128 slices)
     g = torch.Generator().manual_seed(vocab)
     x = (torch.randn(rows, vocab, generator=g) * 2).to(dtype)
     x[3] = float("nan")
     x[4, : vocab - 1] = float("-inf")
     x = x.to(DEV)
-    u = torch.tensor([0.0, 0.9999999, 0.5, 0.3, 0.7, 0.25], device=DEV)
-    temp = torch.tensor([1.0, 0.7, 1.3, 1.0, 2.0, 0.9], device=DEV)
+    u = torch.tensor([0.0, 0.9999999, 0.5, 0.3, 0.7, 0.25] * 4, device=DEV)
+    temp = torch.tensor([1.0, 0.7, 1.3, 1.0, 2.0, 0.9] * 4, device=DEV)
     got, want = sample(x, 0, 1.0, uniform=u), _single_wg(x, 0, 1.0, u)
     got2, want2 = sample(x, 0, 1.0, uniform=u, temperature=temp), _single_wg(scale_logits(x, temperature=temp), 0, 1.0, u)
     torch.cuda.synchronize()
