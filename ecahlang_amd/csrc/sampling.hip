@@ -567,10 +567,11 @@ inline GroupShape group_shape(int vocab) {
 }
 
 constexpr int kCountStride = 32;
+static_assert(kCandCap <= kPBins, "candidates in the bins' place");
 struct SplitWs {
   uint64_t* tmass;    // [rows][ntiles] tile masses (whole and top-p rows)
-  uint64_t* hist;     // [rows][slices][kPBins] masses by bin (top-p rows)
-  uint64_t* cand;     // [rows][slices][kCandCap] candidates, index << 32 | key (top-p rows)
+  uint64_t* hist;     // [rows][slices][kPBins] masses by bin (top-p rows, split_pass_kernel)
+  uint64_t* cand;     // the same area: kCandCap candidates a slice, index << 32 | key (split_finish_kernel)
   ToppBin* bin;       // [rows] where the threshold lies (top-p rows; top-k rows that are handed back)
   uint16_t* gmax;     // [rows][kGroups] group maxima: the keys' upper halves
   float* smax;        // [rows][slices] slice maxima
@@ -582,7 +583,7 @@ struct SplitWs {
 };
 __host__ __device__ inline int64_t split_ws_bytes(int rows, int vocab) {
   const int64_t S = split_slices(vocab);
-  return (int64_t)rows * (split_tiles(vocab) * 8 + S * (kPBins + kCandCap) * 8 + (int64_t)sizeof(ToppBin) + kGroups * 2 + S * 12 + kCountStride * 4 + 4);
+  return (int64_t)rows * (split_tiles(vocab) * 8 + S * kPBins * 8 + (int64_t)sizeof(ToppBin) + kGroups * 2 + S * 12 + kCountStride * 4 + 4);
 }
 inline SplitWs split_ws(void* ws, int rows, int vocab) {
   const int64_t S = split_slices(vocab);
@@ -595,7 +596,7 @@ inline SplitWs split_ws(void* ws, int rows, int vocab) {
   SplitWs w;
   w.tmass = reinterpret_cast<uint64_t*>(take(split_tiles(vocab) * 8));
   w.hist = reinterpret_cast<uint64_t*>(take(S * kPBins * 8));
-  w.cand = reinterpret_cast<uint64_t*>(take(S * kCandCap * 8));
+  w.cand = w.hist;
   w.bin = reinterpret_cast<ToppBin*>(take(sizeof(ToppBin)));
   w.gmax = reinterpret_cast<uint16_t*>(take(kGroups * 2));
   w.smax = reinterpret_cast<float*>(take(S * 4));
@@ -1145,7 +1146,7 @@ __device__ __forceinline__ void topp_finish(const T* p, int vocab, int s, int b,
   // ---- this slice: its tiles' mass above the bin, and its candidates, written through to device scope
   const TileSums sums{L.tsum};
   uint64_t* tm = ws.tmass + (int64_t)b * ntiles;
-  uint64_t* pc = ws.cand + ((int64_t)b * S + s) * kCandCap;
+  uint64_t* pc = ws.cand + ((int64_t)b * S + s) * kPBins;
   // a group's largest logit is at most the float of its key's upper half and all lower bits set; threads
   // of groups that do not reach the bin load the row's first vector instead
   constexpr int R = 8 * sizeof(T) / 16;
@@ -1216,7 +1217,7 @@ __device__ __forceinline__ void topp_finish(const T* p, int vocab, int s, int b,
       const int mid = (lo + hi) >> 1;
       if (L.off[mid] <= i) lo = mid; else hi = mid;
     }
-    const uint64_t c = ld_dev(ws.cand + ((int64_t)b * S + lo) * kCandCap + (i - L.off[lo]));
+    const uint64_t c = ld_dev(ws.cand + ((int64_t)b * S + lo) * kPBins + (i - L.off[lo]));
     L.cand[i] = c;
     if (n <= kSplitThreads) L.mass[i] = fmass(key_float((uint32_t)c), bins.mx);
   }

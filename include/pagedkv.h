@@ -414,8 +414,9 @@ int pkv_scale_logits(const void* logits, int64_t row_stride, int32_t rows, int32
                      void* stream);
 
 /* pkv_scale_logits into scaled (float32, rows of scaled_stride floats: a scratch area), then
- * pkv_top_k_top_p_sampling_ws on it, with the scaling done in the sampler's first pass (where the
- * workspace suffices and scaled's rows are 16-byte aligned; else as two calls).  Tokens as by the two. */
+ * pkv_top_k_top_p_sampling_ws on it, with the scaling done in the sampler's first pass where that
+ * is faster (and the workspace suffices and scaled's rows are 16-byte aligned; else as two calls).  Tokens as by
+ * the two.  Like the sampler on fp32 logits it takes vocabularies of up to 2,097,152 (PKV_E_ARG above). */
 int pkv_scaled_top_k_top_p_sampling(const void* logits, int64_t row_stride, int32_t rows, int32_t vocab, int32_t dtype,
                                     const void* penalty, int64_t penalty_stride, int32_t penalty_slots,
                                     const int32_t* penalty_rows, const float* temperature, float* scaled,
