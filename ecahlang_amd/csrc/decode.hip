@@ -8,7 +8,8 @@
 //   (ecahlang/main.py:203-204 construct, :341-347 / :444-455 plan, :68 run)
 //
 // Workspace (caller-owned bytes, 256-byte aligned regions; R = decode_ranges_cap ranges):
-//   [counters: int32 x batch]
+//   [counters: int32 x batch, or x PKV_MAX_HEAD_COUNTERS where that is more and the workspace has
+//    room, so that a schedule never lies on the counters of an fp32 decode on the same workspace]
 //   [schedule: global header + empty list (kGlobHdr + batch int32), R heads of kHeadWords
 //    int32, R range records of kRecStride int32, R prefix item records of kPrecStride int32,
 //    first-sequence[R], range starts[R + 1], non-empty ranges before[R + 1], plan scratch
@@ -43,12 +44,13 @@ struct WsLayout {
   size_t cnt, ghdr, heads, recs, precs, bf, starts, nzb, scratch, ml, o, total;
   int64_t rcap, slots;
 };
-// Layout for a workspace of ws_bytes (< 0: the smallest one, without shared-prefix slots).
-inline WsLayout ws_layout(int batch, int hq, int d, int ctas, int64_t num_indices, int64_t ws_bytes = -1) {
+// Layout for a workspace of ws_bytes (< 0: the smallest one, without shared-prefix slots) with
+// `counters` words before the schedule.
+inline WsLayout ws_layout_of(int batch, int hq, int d, int ctas, int64_t num_indices, int64_t ws_bytes, int counters) {
   WsLayout L;
   L.rcap = decode_ranges_cap(ctas, num_indices);
   L.cnt = 0;
-  L.ghdr = align256(sizeof(int32_t) * (size_t)batch);
+  L.ghdr = align256(sizeof(int32_t) * (size_t)counters);
   L.heads = L.ghdr + align256(sizeof(int32_t) * ((size_t)kGlobHdr + batch));
   L.recs = L.heads + align256(sizeof(int32_t) * (size_t)L.rcap * kHeadWords);
   L.precs = L.recs + align256(sizeof(int32_t) * (size_t)L.rcap * kRecStride);
@@ -71,6 +73,13 @@ inline WsLayout ws_layout(int batch, int hq, int d, int ctas, int64_t num_indice
   L.o = L.ml + align256(ml_slot * (size_t)L.slots);
   L.total = L.o + align256(o_slot * (size_t)L.slots);
   return L;
+}
+inline WsLayout ws_layout(int batch, int hq, int d, int ctas, int64_t num_indices, int64_t ws_bytes = -1) {
+  if (ws_bytes > 0 && batch < PKV_MAX_HEAD_COUNTERS) {
+    const WsLayout L = ws_layout_of(batch, hq, d, ctas, num_indices, ws_bytes, PKV_MAX_HEAD_COUNTERS);
+    if ((int64_t)L.total <= ws_bytes) return L;
+  }
+  return ws_layout_of(batch, hq, d, ctas, num_indices, ws_bytes, batch);
 }
 
 // Which workspaces hold a cascade schedule (the decode launches the kernel variant that reads

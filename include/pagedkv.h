@@ -175,8 +175,8 @@ int pkv_decode_uses_mfma(int32_t dtype, int32_t head_dim, int32_t num_qo_heads,
  * vector-ALU kernel (cross-checks); PKV_DECODE_DYNAMIC lets that kernel's waves take pages on
  * demand (the summation order, and so the last bits of the result, then vary from call to
  * call).  PKV_DECODE_HEAD_COUNTERS (fp32 caches) says that the first batch * num_kv_heads words of
- * the workspace are zeroed counters (pkv_decode_workspace_init of that many; a plan of the matrix-core
- * schedule overwrites those past batch), so that the merge of a split sequence is shared by its KV
+ * the workspace are zeroed counters (pkv_decode_workspace_init of that many; in a workspace with less than
+ * 8 KB to spare a plan of the matrix-core schedule overwrites those past its batch), so that the merge of a split sequence is shared by its KV
  * heads' workgroups; it is ignored above PKV_MAX_HEAD_COUNTERS of them.  Without PKV_DECODE_DYNAMIC
  * the result is bitwise reproducible for a given num_ctas and flags.  Page ids outside [0, num_pages)
  * and page-list entries past num_indices are never read (their tokens are

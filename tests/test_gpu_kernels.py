@@ -374,6 +374,23 @@ def test_decode_fp32_split_merge_reads_this_calls_partials(hq, hkv, d):
         np.testing.assert_allclose(w.run(dv.q, dv.cache).cpu().numpy(), ref, **TOL[torch.float32], err_msg=str(turn))
 
 
+def test_decode_wrappers_of_two_dtypes_share_a_workspace():
+    """A 16-bit plan's schedule and an fp32 decode's counters on one buffer: both planned, then both run,
+    as often as they like."""
+    lens = [900 + 61 * i for i in range(16)]
+    dvs = [workloads.build_batch(lens, [1] * 16, 32, 8, 64, dt, 94).to(DEV) for dt in (torch.bfloat16, torch.float32)]
+    for dv in dvs:
+        _append_dev(dv)
+    alone = [_decode_dev(dv, dv.q) for dv in dvs]
+    ws = torch.empty(128 << 20, dtype=torch.uint8, device=DEV)
+    wrappers = [BatchDecodeWithPagedKVCacheWrapper(ws, "NHD") for _ in dvs]
+    for _ in range(3):
+        for w, dv in zip(wrappers, dvs):
+            w.plan(dv.indptr, dv.indices, dv.last, dv.hq, dv.hkv, dv.d, dv.ps, q_data_type=dv.dtype)
+        for w, dv, ref in zip(wrappers, dvs, alone):
+            assert torch.equal(w.run(dv.q, dv.cache), ref), dv.dtype
+
+
 @pytest.mark.parametrize("force_valu", [False, True])
 def test_decode_pages_before_first_sequence(force_valu):
     # kv_indptr[0] > 0: the leading page-list entries belong to no sequence

@@ -141,3 +141,18 @@ def test_scaled_sampling_refuses_rows_beyond_the_fp32_limit(dtype):
             rc = L.pkv_scaled_top_k_top_p_sampling(4096, vocab, 1, vocab, dtype, None, 0, 0, None, 4096, 4096,
                                                    (vocab + 3) // 4 * 4, None, 300, None, 1.0, 4096, 4096, ws, n, None)
             assert rc == -5, (vocab, ws, rc)
+
+
+def test_decode_schedule_lies_past_the_head_counters():
+    # An fp32 decode counts arrivals per KV head, in up to 2048 words at the workspace's head, where a
+    # 16-bit decode has one per sequence: its schedule starts past all of them, unless the workspace
+    # has no room for that (which it takes as before).
+    from ecahlang_amd import _lib
+
+    L, out = _lib.lib(), (ctypes.c_int64 * 8)()
+    need = L.pkv_decode_workspace_bytes(16, 16, 128, 256, 2000)
+    for ws, first in ((128 << 20, 4 * 2048), (need, 256), (need + 4 * 2048, 4 * 2048)):
+        assert L.pkv_decode_schedule_layout(16, 16, 128, 256, 2000, ws, out) == 0
+        assert out[0] == first, (ws, out[0])
+    assert L.pkv_decode_schedule_layout(16, 16, 128, 256, 2000, need - 1, out) == -6
+    assert L.pkv_decode_schedule_layout(3000, 16, 128, 256, 9000, 1 << 30, out) == 0 and out[0] == 12032
