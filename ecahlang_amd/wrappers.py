@@ -279,28 +279,23 @@ def prefill_work_list(qo_indptr, kv_indptr, last_page_len, g: int, hkv: int, pag
 def _work_list(qo_indptr, kv_indptr, last_page_len, g, hkv, page_size, causal, head_dim, num_cus, ws_bytes, rows,
                partial_bytes, chunk=None) -> dict:
     """``prefill_work_list`` without the records as lists."""
-    qo = np.ascontiguousarray(np.asarray(qo_indptr, dtype=np.int64), dtype=np.int32)
-    kv = np.ascontiguousarray(np.asarray(kv_indptr, dtype=np.int64), dtype=np.int32)
-    last = np.ascontiguousarray(np.asarray(last_page_len, dtype=np.int64), dtype=np.int32)
+    qo, kv, last = (a if isinstance(a, np.ndarray) and a.dtype == np.int32 and a.flags.c_contiguous else
+                    np.ascontiguousarray(np.asarray(a, dtype=np.int64), dtype=np.int32)
+                    for a in (qo_indptr, kv_indptr, last_page_len))
     B = len(qo) - 1
     if len(kv) != B + 1 or len(last) < B:
         raise ValueError("indptr / last_page_len lengths do not match")
-    # capacity: every (request, query tile, KV head) holds at most max(1, kv_len / 256) chunks
-    tq_max = max(1, rows // max(1, g))
-    qn = np.diff(qo.astype(np.int64))
-    npg = np.diff(kv.astype(np.int64))
-    kvl = np.where(npg > 0, (npg - 1) * page_size + last[:B], 0)
-    tiles = -(-np.maximum(qn, 0) // tq_max)
-    n_groups_cap = int((tiles * hkv).sum())
-    n_items_cap = int((tiles * hkv * np.maximum(1, -(-np.maximum(kvl, 0) // 256))).sum())
-    items = np.zeros((max(1, n_items_cap), 12), dtype=np.int32)
-    groups = np.zeros((max(1, n_groups_cap), 8), dtype=np.int32)
     info = np.zeros(8, dtype=np.int64)
-    L = lib()
-    rc = L.pkv_prefill_work_list(qo.ctypes.data, kv.ctypes.data, last.ctypes.data, B, int(g), int(hkv),
-                                 int(page_size), 1 if causal else 0, int(head_dim), int(num_cus), int(ws_bytes),
-                                 int(rows), int(partial_bytes), int(chunk or 0), items.ctypes.data,
-                                 items.shape[0], groups.ctypes.data, groups.shape[0], info.ctypes.data)
+    cap_i, cap_g = 4096, 1024
+    while True:  # (again if the list is longer than that: info says how long)
+        items, groups = np.empty((cap_i, 12), dtype=np.int32), np.empty((cap_g, 8), dtype=np.int32)
+        rc = lib().pkv_prefill_work_list(qo.ctypes.data, kv.ctypes.data, last.ctypes.data, B, int(g), int(hkv),
+                                         int(page_size), 1 if causal else 0, int(head_dim), int(num_cus), int(ws_bytes),
+                                         int(rows), int(partial_bytes), int(chunk or 0), items.ctypes.data,
+                                         cap_i, groups.ctypes.data, cap_g, info.ctypes.data)
+        if rc != -5 or (info[0] <= cap_i and info[1] <= cap_g):
+            break
+        cap_i, cap_g = max(cap_i, int(info[0])), max(cap_g, int(info[1]))
     if rc == -6:
         raise RuntimeError(f"prefill workspace too small: need {int(info[7])} bytes")
     check(int(rc), "prefill plan")
@@ -323,6 +318,7 @@ class BatchPrefillWithPagedKVCacheWrapper:
         self._kv_layout = "NHD"
         self._use_cuda_graph = use_cuda_graph
         self._planned = False
+        self._list_ready = None
 
     @property
     def is_cuda_graph_enabled(self) -> bool:
@@ -416,7 +412,9 @@ class BatchPrefillWithPagedKVCacheWrapper:
             self._list.copy_(host, non_blocking=True)
             if self._valu_ok:
                 stream = torch.cuda.current_stream(dev)
-                self._list_stream, self._list_ready = stream.cuda_stream, torch.cuda.Event()
+                if self._list_ready is None:
+                    self._list_ready = torch.cuda.Event()
+                self._list_stream = stream.cuda_stream
                 self._list_ready.record(stream)
         self._items_ptr, self._groups_ptr = base, base + off_g
         self._ml_ptr, self._o_ptr = base + off_ml, base + off_o
