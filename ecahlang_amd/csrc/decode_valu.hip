@@ -1,6 +1,7 @@
 // Generic paged attention on the vector ALUs: any of fp32 / fp16 / bf16, head_dim 64/128/256,
-// GQA group up to 16.  It serves fp32 caches (where no 16-bit matrix instruction applies)
-// and shapes the matrix-core kernels do not cover, for both decode and prefill.
+// GQA group up to 16.  It serves the shapes and calls that the matrix-core kernels do not cover
+// (16-bit caches and, with decode_f32.hip and prefill_f32.hip, fp32), for both decode and prefill,
+// and is their cross-check.
 //
 // Decode semantics (FlashInfer BatchDecodeWithPagedKVCacheWrapper.run, called at
 // ecahlang/main.py:68): o[b,h] = softmax(q[b,h] . K_b[:, h/g]^T * sm_scale) V_b[:, h/g] over the

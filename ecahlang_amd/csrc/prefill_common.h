@@ -58,7 +58,8 @@ struct PrefillMfmaParams {
 
 // Split groups' partial outputs are kept in fp16 when the cache is fp16 (averages of fp16 V
 // rows, so they fit; half the bytes written by the items and read by the merge), else fp32.
-// (the run-time groups, G = 0, keep fp32 partials, as they keep fp32-exact weights).
+// (the run-time groups, G = 0, keep fp32 partials: on the vector kernel, which ran them before, nothing
+// between the scores and the output was rounded to 16 bits).
 template <typename T, int G>
 constexpr bool kHalfPartials = std::is_same<T, _Float16>::value && G != 0;
 

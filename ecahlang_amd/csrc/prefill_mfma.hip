@@ -30,9 +30,10 @@
 // Groups that do not divide 256 (3, 5, 6, 7, 9 .. 15) take the same kernel with the group as a run
 // time value (G = 0): an item holds (256 / g) * g rows, and the few left over are masked like the
 // rows of a short tile.  These groups ran on the vector kernel before, which keeps the softmax
-// weights in fp32; here each weight is the sum of two 16-bit values, P = hi + lo, and P.V takes
-// both (half as many products again as the power-of-two groups), so that the result stays as
-// close to the 64-bit one as it was: the output's own rounding is what is left of the error.
+// weights in fp32; here each weight is the sum of two 16-bit values, P = hi + lo (16 significant
+// bits in bf16, 22 in fp16), and P.V takes both (half as many products again as the power-of-two
+// groups), so that the result stays as close to the 64-bit one as it was: the output's own
+// rounding (8 and 11 bits) is what is left of the error.
 // Measured at 28 / 4 heads of 128 dims, bf16, 11 prompts of 20 to 1500 tokens (26 GFLOP of valid
 // pairs): 1418 us on the vector kernel, 63.4 us here (413 TFLOP/s), both 1.6e-3 off 64 bits.
 #include <type_traits>

@@ -25,8 +25,11 @@ constexpr int kItemWords = 12;
 constexpr int kGroupWords = 8;
 constexpr int kStepKeys = 64;
 constexpr int kChunkMin = 256, kChunkMax = 8192;
-// Makespan model, in microseconds.  Items of at most 128 rows are the fp32 kernel's, whose step is
-// its products' issue time on the compute unit (128 x 64 keys x head_dim / 64 at 0.61 TFLOP/s).
+// Makespan model, in microseconds, measured for the 16-bit kernel at power-of-two groups (and used as it is
+// for the run-time groups, whose steps hold half as many products again).  Items of at most 128 rows are
+// the fp32 kernel's, whose step is its products' issue time on the compute unit (128 x 64 keys x head_dim
+// / 64 at 0.61 TFLOP/s); its item and split costs, and that two of its items reside on a unit, are not
+// modelled, and no chunk is under 256 keys (4 or 8 of its steps).  Neither was fitted to those kernels.
 constexpr double kStepUs = 1.9, kItemUs = 11.0, kSplitUs = 6.0, kStepF32Us = 3.4;
 constexpr int kRowsF32 = 128;
 // Candidate chunks, as multiples of total keys / CUs (in 1/16); the longest first, since a simulation

@@ -1,5 +1,5 @@
-// Top-k / top-p sampling from logits, one row per workgroup: the sampler the serving loop calls
-// after the last layer (flashinfer.sampling.top_k_top_p_sampling_from_logits at
+// Top-k / top-p sampling from logits, the sampler the serving loop calls after the last layer
+// (flashinfer.sampling.top_k_top_p_sampling_from_logits at
 // ecahlang/main.py:377-379, 400-402, 489-491, 582-584; top-k filter first, then top-p on the
 // renormalised top-k distribution, deterministic=True).
 //
@@ -9,12 +9,15 @@
 //   S   = { i in K : x_i >= t }, t the largest logit with mass({j in K : x_j >= t}) >= top_p * mass(K)
 //                                                             (S = K when top_p >= 1)
 //   token = first i in S, in vocabulary order, whose cumulative mass over S exceeds u * mass(S)
-// Ties at a threshold are kept.  No sort: both thresholds are found by radix selection over an
-// order-preserving 32-bit key of the logit (three digit passes of 11, 11 and 10 bits, histograms
-// in LDS), and every mass is an integer: exp(x_i - max) in 32-bit fixed point, summed in 64 bits,
-// so the result depends on nothing but the row and u (no floating-point summation order).
-// Every pass reads the row with 16-byte loads (8 fp16/bf16 or 4 fp32 logits per thread, 8 tiles
-// in flight); after the first pass the row is served from L2.
+// Ties at a threshold are kept.  No sort, and every mass is an integer: exp(x_i - max) in 32-bit fixed
+// point, summed in 64 bits, so the result depends on nothing but the row and u (no floating-point
+// summation order), nor on which of two ways a row goes:
+//   one workgroup (sample_kernel: top-k filters over kTopKMax with any top-p, rows that the other kernels
+//   hand back, calls without a workspace): both thresholds by radix selection over an order-preserving
+//   32-bit key of the logit (three digit passes of 11, 11 and 10 bits, histograms in LDS).  Every pass reads
+//   the row with 16-byte loads (8 fp16/bf16 or 4 fp32 logits per thread, 8 tiles in flight); after the first
+//   one the row is served from L2.
+//   many workgroups (the split kernels): all other rows, cut into slices.
 #include <type_traits>
 #include "common.h"
 #include "../../include/pagedkv.h"
@@ -528,7 +531,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const T* logits, int64
 //                        slice finds the tile and the token; top-k rows: the token; top-p rows: the
 //                        mass by distance from the row's largest logit
 //   split_finish_kernel  top-p rows: the threshold and the token
-//   sample_kernel        other rows, and rows handed back
+//   sample_kernel        other rows, and rows handed back, with what is known of them (Back)
 // All masses and targets are the integers sample_row computes, so the token is identical.
 // What bounds them: the scan moves the logits, the penalties and the scaled logits (156 MB in 33 us at
 // 128 x 151,936 fp16); the later launches are chains of latencies (arrivals, LDS rounds) beside 3 to 4

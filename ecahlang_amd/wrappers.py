@@ -6,9 +6,10 @@ calls ``plan`` once per scheduler step with the step's page table (main.py:341-3
 hook (main.py:68), also inside captured CUDA graphs (main.py:146-148).  The classes below
 keep that call shape:
 
-* ``plan`` reads no device data on the host: the decode schedule is built on the device (two
-  small kernels, plus a fill kernel that zeroes the split counters when the batch grows), so
-  it stays cheap, never synchronises and can be captured.
+* The decode wrapper's ``plan`` reads no device data on the host: the decode schedule is built on
+  the device (two small kernels, plus a fill kernel that zeroes the split counters when the batch
+  grows), so it stays cheap, never synchronises and can be captured.  The prefill wrapper's reads
+  the index arrays back once, as FlashInfer's does, and builds its work list on the host.
 * ``run`` only enqueues kernels on the current stream and is safe to capture in a hipGraph;
   its geometry (workgroup count, kernel choice) is fixed by ``plan``'s arguments alone.
 """
@@ -61,7 +62,12 @@ _MAX_HEAD_COUNTERS = 2048  # PKV_MAX_HEAD_COUNTERS
 _INIT_COUNTERS = 8192  # decode split counters zeroed when a workspace is given
 
 class BatchDecodeWithPagedKVCacheWrapper:
-    """Paged decode attention: one query token per sequence (FlashInfer contract)."""
+    """Paged decode attention: one query token per sequence (FlashInfer contract).
+
+    The workspace holds the split counters (zeroed here, left at zero by every run), the plan's
+    schedule and a run's partials, so between a ``plan`` and its last ``run`` it belongs to this
+    wrapper, on one stream or streams ordered after each other; a buffer that a 16-bit prefill
+    wrapper plans into must be another one."""
 
     def __init__(self, float_workspace_buffer: torch.Tensor, kv_layout: str = "NHD",
                  use_cuda_graph: bool = False, use_tensor_cores: bool = False,
@@ -306,7 +312,11 @@ def _work_list(qo_indptr, kv_indptr, last_page_len, g, hkv, page_size, causal, h
 
 
 class BatchPrefillWithPagedKVCacheWrapper:
-    """Paged (chunked) prefill attention over ragged query rows (FlashInfer contract)."""
+    """Paged (chunked) prefill attention over ragged query rows (FlashInfer contract).
+
+    With a 16-bit cache and a power-of-two group, ``plan`` keeps its work list in the workspace and
+    a run its partials: the buffer belongs to one such wrapper, and its runs follow its plan on one
+    stream or streams ordered after each other.  All other shapes leave the workspace alone."""
 
     def __init__(self, float_workspace_buffer: torch.Tensor, kv_layout: str = "NHD",
                  use_cuda_graph: bool = False, qo_indptr_buf=None, paged_kv_indptr_buf=None,

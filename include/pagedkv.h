@@ -387,7 +387,8 @@ int pkv_top_k_top_p_sampling(const void* logits, int64_t row_stride, int32_t row
                              const float* top_p, float top_p_all, const float* uniform,
                              int32_t* out, void* stream);
 
-/* Workspace bytes pkv_top_k_top_p_sampling_ws can use for rows x vocab. */
+/* Workspace bytes pkv_top_k_top_p_sampling_ws can use for rows x vocab (whatever the filters; at a
+ * vocabulary of 151,936 85 KB a row, most of it the bins of top-p rows). */
 int64_t pkv_sampling_workspace_bytes(int32_t rows, int32_t vocab);
 
 /* pkv_top_k_top_p_sampling with a workspace (8-byte aligned, workspace_bytes >=
